@@ -432,6 +432,17 @@ __global__ void __launch_bounds__(64 * kWaves) scan_generic(const ScanArgs<L> A)
 
 // ---- host-side launcher -------------------------------------------------------------
 
+// The scan of few pairs (fms_few.hpp): false when the call is not its.
+template <class Op, class L>
+bool launch_few(const ScanArgs<L>& A, bool vec, bool two, hipStream_t stream, hipError_t* err);
+// The layouts it serves (document order holds many pairs: fp32 only).
+template <class Op, class L>
+struct few_layout { static constexpr bool value = true; };
+template <class Op>
+struct few_layout<Op, LayCandSorted> { static constexpr bool value = Op::kEsz == 4; };
+template <class Op>
+struct few_layout<Op, LayInBatch> { static constexpr bool value = false; };
+
 // Fast-kernel instantiation for a given nkb (k-blocks per token); 0 = none,
 // use the generic kernel.  16-bit features: dim 64 / 128 / 256; int8: dim
 // 64 / 128 / 256; fp32 always uses the generic kernel.
@@ -466,6 +477,12 @@ hipError_t launch_scan(const L& lay, int dim, int rows, int64_t npairs, int32_t*
   const dim3 block(64 * kWaves);
   const bool fast_ok = vec && (dim % Op::kKb == 0) && dim > 0;
   const int nkb_fast = fast_ok ? fast_nkb<Op>(A.nkb) : 0;
+  constexpr int kbat = split_kbat<Op>();
+  const bool split = nkb_fast == 0 && vec && dim > 0 && dim % (kbat * Op::kKb) == 0;
+  if constexpr (few_layout<Op, L>::value) {
+    hipError_t e = hipSuccess;
+    if (launch_few<Op, L>(A, vec, split, stream, &e)) return e;
+  }
   if constexpr (Op::kEsz != 4) {
     constexpr int b = (Op::kKb == 16) ? 4 : 2;
     if (nkb_fast == b) {
@@ -482,8 +499,7 @@ hipError_t launch_scan(const L& lay, int dim, int rows, int64_t npairs, int32_t*
     }
   }
   // Split-d: any dim that is a whole number of KBAT-k-block batches.
-  constexpr int kbat = split_kbat<Op>();
-  if (vec && dim > 0 && dim % (kbat * Op::kKb) == 0) return launch_split<Op, L>(A, grid, block, stream);
+  if (split) return launch_split<Op, L>(A, grid, block, stream);
   if (vec) {
     hipLaunchKernelGGL((scan_generic<Op, L, true>), grid, block, 0, stream, A);
   } else {

@@ -1,5 +1,5 @@
 // Explicit instantiation of the F16 scan launchers for every float layout.
-#include "fms_scan.hpp"
+#include "fms_few.hpp"
 
 namespace fms {
 #define FMS_INST(L)                                                                    \

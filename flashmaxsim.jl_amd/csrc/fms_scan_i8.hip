@@ -1,6 +1,6 @@
 // Explicit instantiation of the INT8 scan launchers (pair/paired and the
 // candidate layout; the reference has no INT8 in-batch / packed methods).
-#include "fms_scan.hpp"
+#include "fms_few.hpp"
 
 namespace fms {
 #define FMS_INST(L)                                                                    \
