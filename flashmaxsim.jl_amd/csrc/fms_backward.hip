@@ -6,7 +6,6 @@
 // cover one row (Lr = the power of two >= chunks per row, at most 64, with
 // two chunks per lane past 64), so one wave instruction moves 64 / Lr rows.
 // Per call:
-//   delta     delta_p = Delta[p] * inv_n[query of p], fp32.
 //   dQ        bwd_dq_vec: a wave owns a block of tokens of one query group and
 //             a share of the group's pairs; per pair it reads the tape block
 //             once (one dword per lane), hands each lane its tokens' entries
@@ -16,12 +15,15 @@
 //             index mod nsplit, so split s runs on XCD s mod 8 and keeps its
 //             share of the documents in that XCD's L2) fp32 partials are
 //             summed in split order by bwd_dq_reduce.  Deterministic.
-//   dD        bwd_doc_csr: a workgroup per document sorts the document's
-//             sources (pair, token) by destination row in LDS (count, scan,
-//             fill) and writes the row lists; bwd_dd_vec then sums each row's
-//             source query rows in registers.  Rows of no document (and
-//             documents of no pair) are written 0.  The order within a row
-//             is the LDS fill order (not fixed).
+//   dD        bwd_doc_dd: a workgroup per (document, share of its rows) sorts
+//             the share's sources (pair, token) by destination row in LDS
+//             (count, scan, fill) and sums each row's source query rows in
+//             registers.  Rows of no document (and documents of no pair) are
+//             written 0.  Documents of more than kDocList sources instead take
+//             bwd_doc_csr (a 1024-thread sort into global row lists) and
+//             bwd_dd_vec (row sums over all rows).  The order within a row is
+//             the LDS fill order (not fixed).
+// All compute delta_p = Delta[p] * inv_n[query of p] in fp32 where they use it.
 // Other row sizes take the generic path: one wave per output row, features
 // strided over the lanes, and a destination CSR built with global atomics.
 #include <hip/hip_runtime.h>
@@ -40,11 +42,16 @@ namespace {
 
 constexpr int kBwdThreads = 256;  // 4 waves
 constexpr int kBwdUnroll = 8;     // source rows in flight per wave (generic kernels)
-constexpr int kDocTile = 4096;    // destination rows per LDS tile of bwd_doc_csr
-constexpr int kDocThreads = 1024; // threads of bwd_doc_csr (16 waves)
-constexpr int kDocUnroll = 4;     // sources in flight per thread (bwd_doc_csr)
-constexpr int kDocKeep = 16;      // sources a thread keeps in registers (bwd_doc_csr, one tape read)
-constexpr int kDdUnroll = 8;      // sources in flight per row group (bwd_dd_vec)
+constexpr int kDocTile = 1024;    // destination rows per LDS tile of bwd_doc_dd
+constexpr int kDocThreads = 256;  // threads of bwd_doc_dd
+constexpr int kDocKeep = 8;       // sources a thread keeps in registers (bwd_doc_dd, one tape read)
+constexpr int kDocList = kDocKeep * kDocThreads;  // sources of a document whose list fits LDS
+constexpr int kCsrTile = 4096;    // destination rows per LDS tile of bwd_doc_csr
+constexpr int kCsrThreads = 1024; // threads of bwd_doc_csr (16 waves)
+constexpr int kCsrUnroll = 4;     // sources in flight per thread (bwd_doc_csr)
+constexpr int kCsrKeep = 16;      // sources a thread keeps in registers (bwd_doc_csr, one tape read)
+constexpr int kCsrDdUnroll = 8;   // sources in flight per row group (bwd_dd_vec)
+constexpr int kDdUnroll = 4;      // query rows in flight per row group (bwd_doc_dd)
 
 inline int64_t bcdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 inline size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -157,32 +164,37 @@ struct RowGeo {
   int tpw;    // dQ: tokens per wave (tpl * 64 / lanes per row, <= 64)
 };
 
-// ---- documents as the dD kernels see them -----------------------------------------
-// A document owns a run of dD rows (found from the view of its first pair) and
-// the pairs that score it; its sources are (pair k, query token t), numbered
-// p * rows + t, with list slots from slot0(d) on; qrow0(p) is the first dQ /
-// query row of p's query.  npairs / first / slot0 take a wave-uniform
-// document; pair / qok / qrow0 take per-lane arguments.
+// ---- documents as the dD kernel sees them ------------------------------------------
+// A document owns a run of dD rows and the pairs that score it; its sources
+// are (pair k, query token t), numbered p * rows + t, with list slots from
+// slot0(d) on; qrow0(p) is the first dQ / query row of p's query.  rows()
+// gives the rows the document's workgroups write: its own, and in the ragged
+// layouts those before the first and after the last document too (`off` rows
+// precede the document's first).  The documents' rows and these ends together
+// cover every row, whatever cu holds.  npairs / first / slot0 / rows take a
+// wave-uniform document; pair / qok / qrow0 take per-lane arguments.
 struct DocsInBatch {  // document j: pairs p = j + Bd * i, i < Bq
   int64_t ndocs;
   uint32_t Bd, Bq;
-  int rows, Tq;
+  int trows, Tq, Td;
   const uint8_t* qm;
+  __device__ void rows(int64_t d, int64_t& r0, int64_t& n, int64_t& off) const { r0 = d * Td; n = Td; off = 0; }
   __device__ int64_t npairs(int64_t) const { return Bq; }
   __device__ int64_t first(int64_t d) const { return d; }
   __device__ int64_t pair(int64_t d, uint32_t k) const { return d + (int64_t)Bd * k; }
-  __device__ int64_t slot0(int64_t d) const { return d * (int64_t)Bq * rows; }
+  __device__ int64_t slot0(int64_t d) const { return d * (int64_t)Bq * trows; }
   __device__ bool qok(uint32_t p, int t) const { return !qm || qm[(int64_t)(p / Bd) * Tq + t]; }
   __device__ int64_t qrow0(uint32_t p) const { return (int64_t)(p / Bd) * Tq; }
 };
 struct DocsPaired {  // document b: pair b
   int64_t ndocs;
-  int rows, Tq;
+  int trows, Tq, Td;
   const uint8_t* qm;
+  __device__ void rows(int64_t d, int64_t& r0, int64_t& n, int64_t& off) const { r0 = d * Td; n = Td; off = 0; }
   __device__ int64_t npairs(int64_t) const { return 1; }
   __device__ int64_t first(int64_t d) const { return d; }
   __device__ int64_t pair(int64_t d, uint32_t) const { return d; }
-  __device__ int64_t slot0(int64_t d) const { return d * rows; }
+  __device__ int64_t slot0(int64_t d) const { return d * trows; }
   __device__ bool qok(uint32_t p, int t) const { return !qm || qm[(int64_t)p * Tq + t]; }
   __device__ int64_t qrow0(uint32_t p) const { return (int64_t)p * Tq; }
 };
@@ -191,38 +203,64 @@ struct DocsCand {  // gallery document j: the pairs the document order lists for
   const uint32_t* end;
   const PairRef* order;
   uint32_t C;
-  int rows, Tq;
+  int trows, Tq, Td;
   const uint8_t* qm;
+  __device__ void rows(int64_t d, int64_t& r0, int64_t& n, int64_t& off) const { r0 = d * Td; n = Td; off = 0; }
   __device__ int64_t start(int64_t d) const { return d > 0 ? (int64_t)sload(end, d - 1) : 0; }
   __device__ int64_t npairs(int64_t d) const { return (int64_t)sload(end, d) - start(d); }
   __device__ int64_t first(int64_t d) const { return sload(&order[start(d)].p, 0); }
   __device__ int64_t pair(int64_t d, uint32_t k) const { return order[start(d) + k].p; }
-  __device__ int64_t slot0(int64_t d) const { return start(d) * rows; }
+  __device__ int64_t slot0(int64_t d) const { return start(d) * trows; }
   __device__ bool qok(uint32_t p, int t) const { return !qm || qm[(int64_t)(p / C) * Tq + t]; }
   __device__ int64_t qrow0(uint32_t p) const { return (int64_t)(p / C) * Tq; }
 };
+// Rows of segment d of a ragged store of n tokens, ends included (see above).
+__device__ __forceinline__ void ragged_rows(const int32_t* cu, int64_t nseg, int64_t n, int64_t d,
+                                            int64_t& r0, int64_t& cnt, int64_t& off) {
+  const int64_t a = clamp64((int64_t)sload(cu, d) - 1, 0, n);
+  const int64_t z = d + 1 == nseg ? n : clamp64((int64_t)sload(cu, d + 1) - 1, a, n);
+  r0 = d == 0 ? 0 : a;
+  off = a - r0;
+  cnt = z - r0;
+}
 struct DocsPacked {  // document b: pair b; one shared query
   int64_t ndocs;
-  int rows;
+  int trows;
   const uint8_t* qm;
+  const int32_t* cu;
+  int64_t ntok;
+  __device__ void rows(int64_t d, int64_t& r0, int64_t& n, int64_t& off) const { ragged_rows(cu, ndocs, ntok, d, r0, n, off); }
   __device__ int64_t npairs(int64_t) const { return 1; }
   __device__ int64_t first(int64_t d) const { return d; }
   __device__ int64_t pair(int64_t d, uint32_t) const { return d; }
-  __device__ int64_t slot0(int64_t d) const { return d * rows; }
+  __device__ int64_t slot0(int64_t d) const { return d * trows; }
   __device__ bool qok(uint32_t, int t) const { return !qm || qm[t]; }
   __device__ int64_t qrow0(uint32_t) const { return 0; }
 };
 struct DocsVarlen {  // document segment n: pair n
   int64_t ndocs;
-  int rows;
+  int trows;
   const int32_t* cu_q;
-  int64_t nq;
+  const int32_t* cu_d;
+  int64_t nq, nd;
+  __device__ void rows(int64_t d, int64_t& r0, int64_t& n, int64_t& off) const { ragged_rows(cu_d, ndocs, nd, d, r0, n, off); }
   __device__ int64_t npairs(int64_t) const { return 1; }
   __device__ int64_t first(int64_t d) const { return d; }
   __device__ int64_t pair(int64_t d, uint32_t) const { return d; }
-  __device__ int64_t slot0(int64_t d) const { return d * rows; }
+  __device__ int64_t slot0(int64_t d) const { return d * trows; }
   __device__ bool qok(uint32_t, int) const { return true; }
   __device__ int64_t qrow0(uint32_t p) const { return clamp64((int64_t)cu_q[p] - 1, 0, nq); }
+};
+
+// delta_p = Delta[p] * inv_n[p / G] in fp32 (no inv_n: Delta[p]).
+template <class E>
+struct DeltaOf {
+  const char* Delta;
+  const char* inv_n;
+  uint32_t G;
+  __device__ float at(uint32_t p) const { return E::ld(Delta + (int64_t)p * E::kSz) * inv(p / G); }
+  __device__ float inv(uint32_t g) const { return inv_n ? E::ld(inv_n + (int64_t)g * E::kSz) : 1.0f; }
+  __device__ float raw(int64_t p) const { return E::ld(Delta + p * E::kSz); }
 };
 
 template <class E>
@@ -252,12 +290,13 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_zero16_kernel(uint16_t* w, in
 // feature type; nsplit > 1 writes fp32 partials part[s][query row][dim].
 template <class L, class E, bool kWaveSplit>
 __global__ void __launch_bounds__(kBwdThreads) bwd_dq_vec_kernel(
-    const L lay, const float* delta, const int32_t* args, int64_t G, int rows, int ntb, int nsplit,
-    int64_t nitems, RowGeo geo, int64_t rb, int dim, const char* Qbase, char* dQ, float* part,
-    int64_t nq_rows) {
+    const L lay, const DeltaOf<E> delta, const int32_t* args, int64_t G, int rows, int ntb,
+    int nsplit, int64_t nitems, RowGeo geo, int64_t rb, int dim, const char* Qbase, char* dQ,
+    float* part, int64_t nq_rows, uint32_t* clear) {
   constexpr int kV = E::kV, kSL = 64 / kV;  // 16-byte slots per lane (64 fp32 accumulators)
   const int lane = threadIdx.x & 63;
   const int w = uniform((int)(threadIdx.x >> 6));
+  if (clear != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0u;  // bwd_doc_dd's count
   int64_t item;
   int split;
   if constexpr (kWaveSplit) {
@@ -280,6 +319,7 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dq_vec_kernel(
     pb = std::min(pb, pa + q);
   }
   const PairView v0 = uniform_view(lay.get(g * G));
+  const float inv_g = delta.inv((uint32_t)g);
   const int lg = geo.lg_lr, rpi = 64 >> lg;
   const int gid = lane >> lg, c0 = lane & ((1 << lg) - 1);
   const int t0 = tb * geo.tpw;
@@ -320,17 +360,17 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dq_vec_kernel(
   if (len > 0) {
     const int64_t p0 = pair_at(0);
     vnext = uniform_view(lay.get(p0));
-    dnext = sload(delta, p0);
+    dnext = delta.raw(p0);
     tnext = tlane ? args[p0 * rows + t0 + lane] : 0;
   }
   for (int64_t k = 0; k < len; ++k) {
     const PairView v = vnext;
-    const float dl = dnext;
+    const float dl = uniform_f(dnext * inv_g);
     const int tv = tnext;
     if (k + 1 < len) {
       const int64_t pn = pair_at(k + 1);
       vnext = uniform_view(lay.get(pn));
-      dnext = sload(delta, pn);
+      dnext = delta.raw(pn);
       if (tlane) tnext = args[pn * rows + t0 + lane];
     }
     if (!v.valid || dl == 0.0f) continue;
@@ -391,6 +431,21 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dq_vec_kernel(
             make_float4(acc[s][e], acc[s][e + 1], acc[s][e + 2], acc[s][e + 3]);
     }
   }
+  if constexpr (std::is_same<L, LayVarlen>::value) {
+    // Query rows of no pair: tokens past `rows` of this pair, and those before
+    // the first and after the last pair (rows past the segment's own tokens
+    // and before it; see ragged_rows).
+    if (tb == ntb - 1) {
+      int64_t r0, n, off;
+      ragged_rows(lay.cu_q, nitems / ntb, lay.nq, g, r0, n, off);
+      auto zero = [&](int64_t a, int64_t b) {
+        for (int64_t c = a * geo.nch + lane; c < b * geo.nch; c += 64)
+          *reinterpret_cast<uint4*>(dQ + c * 16) = make_uint4(0u, 0u, 0u, 0u);
+      };
+      zero(r0, r0 + off);
+      zero(r0 + off + v0.tq, r0 + n);
+    }
+  }
 }
 
 // In-batch dQ with the documents staged in LDS.  A workgroup of 16 waves owns
@@ -439,7 +494,7 @@ __device__ __forceinline__ void lds_read4(uint4 (&r)[4], const uint32_t (&a)[4])
 
 template <class E, int kCPL>
 __global__ void __launch_bounds__(kIbThreads) bwd_dq_ib_kernel(
-    const LayInBatch lay, const float* delta, const int32_t* args, int rows, int ntb, int nsplit,
+    const LayInBatch lay, const DeltaOf<E> delta, const int32_t* args, int rows, int ntb, int nsplit,
     int64_t nitems, RowGeo geo, int64_t rb, int dim, char* dQ, float* part, int64_t nq_rows) {
   constexpr int kV = E::kV, kSL = 64 / kV, kHalf = kSL / 2;
   constexpr int kOps = kIbStagePer + 2;  // loads a wave issues per document
@@ -502,15 +557,16 @@ __global__ void __launch_bounds__(kIbThreads) bwd_dq_ib_kernel(
                                                0, 0, 0);
     }
     const int64_t p = j + Bd * i;
-    dl = delta[p];
+    dl = delta.raw(p);
     tv = args[p * rows + tcol];
   };
+  const float inv_i = delta.inv((uint32_t)i);
   // The LDS reads go through lds_read4: the compiler cannot tell which buffer
   // a copy targets once the rotation wraps, and would otherwise wait for the
   // copies in flight (the next two documents) before each read.  The step
   // barrier already orders them: document j's copy completed before step j.
   auto gather = [&](const uint4* rowbase, float dlv, int tvv) {
-    const float dl = live ? uniform_f(dlv) : 0.0f;
+    const float dl = live ? uniform_f(dlv * inv_i) : 0.0f;
     const int tv = tlane ? tvv : 0;
     if (dl == 0.0f) return;
     const uint32_t lbase = lds_addr(rowbase);
@@ -608,10 +664,183 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dq_reduce_kernel(const float*
 
 // ---- vector path: dD ---------------------------------------------------------------------
 
-// Exclusive scan of cnt[0, n) (n <= kDocTile) into out[]; returns the total.
-// Every thread of the (kDocThreads) block calls it.
-__device__ uint32_t block_scan_tile(const uint32_t* cnt, uint32_t* out, int n) {
+// Exclusive scan of cnt[0, n) (n <= kDocTile) into out[].  Every thread of the
+// (kDocThreads) block calls it; barriers around it are the caller's, the last
+// one inside it excepted.
+__device__ void doc_scan_tile(const uint32_t* cnt, uint32_t* out, int n, uint32_t* wsum) {
   constexpr int kWaves = kDocThreads / 64, kPer = kDocTile / kDocThreads;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int i0 = tid * kPer;
+  uint32_t loc[kPer];
+  uint32_t sum = 0u;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    loc[j] = (i0 + j < n) ? cnt[i0 + j] : 0u;
+    sum += loc[j];
+  }
+  uint32_t x = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) wsum[w] = x;
+  __syncthreads();
+  uint32_t before = x - sum;
+#pragma unroll
+  for (int j = 0; j < kWaves; ++j)
+    if (j < w) before += wsum[j];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    if (i0 + j < n) out[i0 + j] = before;
+    before += loc[j];
+  }
+}
+
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v = std::max(v, (uint32_t)__shfl_xor((int)v, o));
+  return v;
+}
+
+// dD of (document, share of its rows): count the share's sources per row in LDS,
+// scan, fill the rows' lists with (query row, delta), then sum each row's
+// query rows, Lr lanes per row, and write it (0 without a source).  Serves
+// documents of at most kDocList sources, which stay in registers between count
+// and fill.  Candidates can hold others; the kernel lists those (heavy[0] of
+// them, cleared by bwd_dq_vec, from heavy[1] on) for bwd_doc_csr and bwd_dd_vec.
+//
+// One kernel in place of a clear of the row counts, a 1024-thread sort per
+// document into global row lists and a row-sum kernel over all rows: at 2048
+// pairs of 30 tokens on 1500 documents of 150 tokens (d = 128, bf16) those
+// took 2 + 45 + 25 us, the sort idle for want of sources (about 40 a
+// document).  Bound by the chain of dependent loads (pair, tape, delta, list,
+// query row) and by the write of dD.
+template <class L, class Docs, class E, int kCPL>
+__global__ void __launch_bounds__(kDocThreads) bwd_doc_dd_kernel(
+    const L lay, const Docs docs, const DeltaOf<E> delta, const int32_t* args, int rows, RowGeo geo,
+    int64_t rb, const char* Qbase, char* dD, int shares, uint32_t* heavy) {
+  constexpr int kV = E::kV;
+  __shared__ uint32_t cnt[kDocTile], cur[kDocTile];
+  __shared__ uint2 list[kDocList];
+  __shared__ uint32_t wsum[kDocThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
+  const int lg = geo.lg_lr, lr = 1 << lg, rpi = 64 >> lg;
+  const int gid = lane >> lg, c0 = lane & (lr - 1);
+  for (int64_t blk = blockIdx.x; blk < docs.ndocs * shares; blk += gridDim.x) {
+    const int64_t d = blk / shares;
+    const int share = (int)(blk - d * shares);
+    int64_t r0, nrow, off;
+    docs.rows(d, r0, nrow, off);
+    r0 = uni64(r0);
+    nrow = uni64(nrow);
+    off = uni64(off);
+    const int64_t np = uni64(docs.npairs(d));
+    int td = 0, tq = 0;
+    if (np > 0) {
+      const PairView v = uniform_view(lay.get(uni64(docs.first(d))));
+      td = v.td;
+      tq = v.tq;
+    }
+    const uint32_t nsrc = td > 0 ? (uint32_t)(np * tq) : 0u;
+    if (nsrc > (uint32_t)kDocList) {
+      if (share == 0 && tid == 0) heavy[1 + atomicAdd(&heavy[0], 1u)] = (uint32_t)d;
+      continue;
+    }
+    const int64_t per = (nrow + shares - 1) / shares;
+    const int64_t rend = std::min(nrow, (int64_t)(share + 1) * per);
+    // Sources f = k * tq + t of the document (pair k, query token t): its row
+    // among the rows this document writes (-1: none) and its list entry.
+    int64_t key[kDocKeep];
+    uint2 val[kDocKeep];
+#pragma unroll
+    for (int q = 0; q < kDocKeep; ++q) {
+      const uint32_t f = (uint32_t)(q * kDocThreads + tid);
+      key[q] = -1;
+      if (f < nsrc) {
+        const uint32_t k = f / (uint32_t)tq;
+        const int t = (int)(f - k * (uint32_t)tq);
+        const int64_t p = docs.pair(d, k);
+        const int u = args[p * rows + t];
+        const float dl = delta.at((uint32_t)p);
+        val[q] = make_uint2((uint32_t)(docs.qrow0((uint32_t)p) + t), __float_as_uint(dl));
+        if (u >= 1 && u <= td && dl != 0.0f && docs.qok((uint32_t)p, t)) key[q] = off + u - 1;
+      }
+    }
+    for (int64_t u0 = share * per; u0 < rend; u0 += kDocTile) {
+      const int ut = (int)std::min<int64_t>(kDocTile, rend - u0);
+      if (nsrc > 0) {
+        for (int i = tid; i < ut; i += kDocThreads) cnt[i] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kDocKeep; ++q)
+          if (key[q] >= u0 && key[q] < u0 + ut) atomicAdd(&cnt[key[q] - u0], 1u);
+        __syncthreads();
+        doc_scan_tile(cnt, cur, ut, wsum);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kDocKeep; ++q)
+          if (key[q] >= u0 && key[q] < u0 + ut) list[atomicAdd(&cur[key[q] - u0], 1u)] = val[q];
+        __syncthreads();
+      }
+      for (int i0 = w * rpi; i0 < ut; i0 += (kDocThreads / 64) * rpi) {
+        const int i = i0 + gid;
+        const bool rv = i < ut;
+        const uint32_t n = rv && nsrc > 0 ? cnt[i] : 0u;
+        const uint32_t base = n ? cur[i] - n : 0u;  // (the fill moved cur to the row's end)
+        const uint32_t nmax = nsrc > 0 ? wave_max_u32(n) : 0u;
+        float acc[kCPL][kV];
+#pragma unroll
+        for (int cc = 0; cc < kCPL; ++cc)
+#pragma unroll
+          for (int e = 0; e < kV; ++e) acc[cc][e] = 0.0f;
+        for (uint32_t j = 0; j < nmax; j += kDdUnroll) {
+          uint4 raw[kDdUnroll][kCPL];
+          float dl[kDdUnroll];
+#pragma unroll
+          for (int q = 0; q < kDdUnroll; ++q) {
+            const bool on = j + q < n;
+            const uint2 ent = on ? list[base + j + q] : make_uint2(0u, 0u);
+            dl[q] = __uint_as_float(ent.y);
+            const char* qa = Qbase + (int64_t)ent.x * rb;
+#pragma unroll
+            for (int cc = 0; cc < kCPL; ++cc) {
+              const int ch = c0 + (cc << lg);
+              raw[q][cc] = on && ch < geo.nch ? load16(qa + ch * 16) : make_uint4(0u, 0u, 0u, 0u);
+            }
+          }
+#pragma unroll
+          for (int q = 0; q < kDdUnroll; ++q)
+#pragma unroll
+            for (int cc = 0; cc < kCPL; ++cc) E::fma_chunk(raw[q][cc], dl[q], acc[cc]);
+        }
+        if (rv) {
+#pragma unroll
+          for (int cc = 0; cc < kCPL; ++cc) {
+            const int ch = c0 + (cc << lg);
+            if (ch < geo.nch)
+              *reinterpret_cast<uint4*>(dD + (r0 + u0 + i) * rb + ch * 16) = E::pack(acc[cc]);
+          }
+        }
+      }
+      __syncthreads();  // the counters and lists are rewritten by the next tile
+    }
+  }
+}
+
+// ---- dD of documents with many sources --------------------------------------------------------
+// Past kDocList sources a document, one 1024-thread sort per document into
+// global row lists and a row-sum kernel over all rows are the better split:
+// every row has its own waves however few documents there are (fp32, d = 128,
+// Td = 180, us per pullback with these / with a workgroup per document and
+// share: in-batch 128 x 128 66 / 97, 512 x 512 670 / 916; 64 x 100 candidates
+// on three documents 221 / 389; below kDocList sources, in-batch 64 x 64 73 /
+// 45).  In-batch and long queries the host knows; of candidates the device
+// lists such documents (heavy), and there may be none.
+// Exclusive scan of cnt[0, n) (n <= kCsrTile) into out[]; returns the total.
+// Every thread of the (kCsrThreads) block calls it.
+__device__ uint32_t csr_scan_tile(const uint32_t* cnt, uint32_t* out, int n) {
+  constexpr int kWaves = kCsrThreads / 64, kPer = kCsrTile / kCsrThreads;
   __shared__ uint32_t wsum[kWaves];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int i0 = tid * kPer;
@@ -646,19 +875,19 @@ __device__ uint32_t block_scan_tile(const uint32_t* cnt, uint32_t* out, int n) {
 }
 
 // Sources f = k * tq + t (pair k of the document, query token t) of one
-// document, kDocUnroll per thread at a time: calls fn(p, t, u) for those with
+// document, kCsrUnroll per thread at a time: calls fn(p, t, u) for those with
 // a nonzero delta, a true qmask and a tape entry u0 < u <= u0 + ut.
-template <class Docs, class Fn>
+template <class Docs, class E, class Fn>
 __device__ __forceinline__ void for_doc_sources(const Docs& docs, int64_t d, uint32_t nsrc, int tq,
-                                                const float* delta, const int32_t* args, int rows,
+                                                const DeltaOf<E>& delta, const int32_t* args, int rows,
                                                 int u0, int ut, Fn fn) {
-  for (uint32_t f0 = 0; f0 < nsrc; f0 += kDocUnroll * kDocThreads) {
-    int64_t p[kDocUnroll];
-    int t[kDocUnroll], u[kDocUnroll];
-    bool ok[kDocUnroll];
+  for (uint32_t f0 = 0; f0 < nsrc; f0 += kCsrUnroll * kCsrThreads) {
+    int64_t p[kCsrUnroll];
+    int t[kCsrUnroll], u[kCsrUnroll];
+    bool ok[kCsrUnroll];
 #pragma unroll
-    for (int q = 0; q < kDocUnroll; ++q) {
-      const uint32_t f = f0 + q * kDocThreads + threadIdx.x;
+    for (int q = 0; q < kCsrUnroll; ++q) {
+      const uint32_t f = f0 + q * kCsrThreads + threadIdx.x;
       ok[q] = f < nsrc;
       const uint32_t k = ok[q] ? f / (uint32_t)tq : 0u;
       t[q] = ok[q] ? (int)(f - k * (uint32_t)tq) : 0;
@@ -666,8 +895,8 @@ __device__ __forceinline__ void for_doc_sources(const Docs& docs, int64_t d, uin
       u[q] = ok[q] ? args[p[q] * rows + t[q]] : 0;
     }
 #pragma unroll
-    for (int q = 0; q < kDocUnroll; ++q) {
-      if (ok[q] && u[q] > u0 && u[q] <= u0 + ut && delta[p[q]] != 0.0f &&
+    for (int q = 0; q < kCsrUnroll; ++q) {
+      if (ok[q] && u[q] > u0 && u[q] <= u0 + ut && delta.at((uint32_t)p[q]) != 0.0f &&
           docs.qok((uint32_t)p[q], t[q]))
         fn(p[q], t[q], u[q]);
     }
@@ -676,18 +905,20 @@ __device__ __forceinline__ void for_doc_sources(const Docs& docs, int64_t d, uin
 
 // One workgroup per document (grid-stride): sources of the document with a
 // nonzero delta, a true qmask and a tape entry 1 <= u <= td, sorted by u in
-// LDS tiles of kDocTile rows; writes rstart/rcount of the document's rows and
+// LDS tiles of kCsrTile rows; writes rstart/rcount of the document's rows and
 // each source as (query row, delta bits) into list[slot0(d) ...].
-template <class L, class Docs>
-__global__ void __launch_bounds__(kDocThreads) bwd_doc_csr_kernel(const L lay, const Docs docs,
-                                                                 const float* delta,
+template <class L, class Docs, class E>
+__global__ void __launch_bounds__(kCsrThreads) bwd_doc_csr_kernel(const L lay, const Docs docs,
+                                                                 const DeltaOf<E> delta,
                                                                  const int32_t* args, int rows,
                                                                  const char* Dbase, int64_t rb,
                                                                  uint32_t* rstart, uint32_t* rcount,
-                                                                 uint2* list) {
-  __shared__ uint32_t cnt[kDocTile], cur[kDocTile];
+                                                                 uint2* list, const uint32_t* heavy) {
+  __shared__ uint32_t cnt[kCsrTile], cur[kCsrTile];
   const int tid = threadIdx.x;
-  for (int64_t d = blockIdx.x; d < docs.ndocs; d += gridDim.x) {
+  const int64_t nd = heavy != nullptr ? (int64_t)rfl32(heavy[0]) : docs.ndocs;
+  for (int64_t x = blockIdx.x; x < nd; x += gridDim.x) {
+    const int64_t d = heavy != nullptr ? (int64_t)rfl32(heavy[1 + x]) : x;
     const int64_t np = uni64(docs.npairs(d));
     if (np == 0) continue;
     const PairView v = uniform_view(lay.get(uni64(docs.first(d))));
@@ -695,58 +926,58 @@ __global__ void __launch_bounds__(kDocThreads) bwd_doc_csr_kernel(const L lay, c
     const int td = v.td, tq = v.tq;
     const uint32_t nsrc = (uint32_t)(np * tq);
     int64_t slot = docs.slot0(d);
-    if (nsrc <= (uint32_t)(kDocKeep * kDocThreads) && td <= kDocTile) {
+    if (nsrc <= (uint32_t)(kCsrKeep * kCsrThreads) && td <= kCsrTile) {
       // One tape read: each thread keeps its sources (row, (query row, delta))
       // in registers between the count and the fill.
-      uint32_t key[kDocKeep];
-      uint2 val[kDocKeep];
+      uint32_t key[kCsrKeep];
+      uint2 val[kCsrKeep];
 #pragma unroll
-      for (int q = 0; q < kDocKeep; ++q) {
-        const uint32_t f = q * kDocThreads + tid;
+      for (int q = 0; q < kCsrKeep; ++q) {
+        const uint32_t f = q * kCsrThreads + tid;
         const bool in = f < nsrc;
         const uint32_t k = in ? f / (uint32_t)tq : 0u;
         const int t = in ? (int)(f - k * (uint32_t)tq) : 0;
         const int64_t p = docs.pair(d, k);
         const int u = in ? args[p * rows + t] : 0;
-        const float dl = delta[p];
+        const float dl = delta.at((uint32_t)p);
         const bool ok = in && u >= 1 && u <= td && dl != 0.0f && docs.qok((uint32_t)p, t);
         key[q] = ok ? (uint32_t)(u - 1) : 0xFFFFFFFFu;
         val[q] = make_uint2((uint32_t)(docs.qrow0((uint32_t)p) + t), __float_as_uint(dl));
       }
-      for (int i = tid; i < td; i += kDocThreads) cnt[i] = 0u;
+      for (int i = tid; i < td; i += kCsrThreads) cnt[i] = 0u;
       __syncthreads();
 #pragma unroll
-      for (int q = 0; q < kDocKeep; ++q)
+      for (int q = 0; q < kCsrKeep; ++q)
         if (key[q] != 0xFFFFFFFFu) atomicAdd(&cnt[key[q]], 1u);
       __syncthreads();
-      block_scan_tile(cnt, cur, td);
-      for (int i = tid; i < td; i += kDocThreads) {
+      csr_scan_tile(cnt, cur, td);
+      for (int i = tid; i < td; i += kCsrThreads) {
         rstart[r0 + i] = (uint32_t)slot + cur[i];
         rcount[r0 + i] = cnt[i];
       }
       __syncthreads();  // every start read before the fill moves the cursors
 #pragma unroll
-      for (int q = 0; q < kDocKeep; ++q)
+      for (int q = 0; q < kCsrKeep; ++q)
         if (key[q] != 0xFFFFFFFFu) list[slot + atomicAdd(&cur[key[q]], 1u)] = val[q];
       __syncthreads();
       continue;
     }
-    for (int u0 = 0; u0 < td; u0 += kDocTile) {
-      const int ut = std::min(kDocTile, td - u0);
-      for (int i = tid; i < ut; i += kDocThreads) cnt[i] = 0u;
+    for (int u0 = 0; u0 < td; u0 += kCsrTile) {
+      const int ut = std::min(kCsrTile, td - u0);
+      for (int i = tid; i < ut; i += kCsrThreads) cnt[i] = 0u;
       __syncthreads();
       for_doc_sources(docs, d, nsrc, tq, delta, args, rows, u0, ut,
                       [&](int64_t, int, int u) { atomicAdd(&cnt[u - 1 - u0], 1u); });
       __syncthreads();
-      const uint32_t total = block_scan_tile(cnt, cur, ut);
-      for (int i = tid; i < ut; i += kDocThreads) {
+      const uint32_t total = csr_scan_tile(cnt, cur, ut);
+      for (int i = tid; i < ut; i += kCsrThreads) {
         rstart[r0 + u0 + i] = (uint32_t)slot + cur[i];
         rcount[r0 + u0 + i] = cnt[i];
       }
       __syncthreads();  // every start read before the fill moves the cursors
       for_doc_sources(docs, d, nsrc, tq, delta, args, rows, u0, ut, [&](int64_t p, int t, int u) {
         const uint32_t pos = atomicAdd(&cur[u - 1 - u0], 1u);
-        list[slot + pos] = make_uint2((uint32_t)(docs.qrow0((uint32_t)p) + t), __float_as_uint(delta[p]));
+        list[slot + pos] = make_uint2((uint32_t)(docs.qrow0((uint32_t)p) + t), __float_as_uint(delta.at((uint32_t)p)));
       });
       __syncthreads();
       slot += total;
@@ -754,34 +985,32 @@ __global__ void __launch_bounds__(kDocThreads) bwd_doc_csr_kernel(const L lay, c
   }
 }
 
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = std::max(v, (uint32_t)__shfl_xor((int)v, o));
-  return v;
-}
-
 // dD row r = sum over its listed sources of delta_p * Q[query row].  A wave
 // covers 64 / Lr consecutive rows, Lr lanes per row; every row of [0, nrows)
-// is written.  Each lane of a row group reads one list entry of a batch of Lr
+// (or, with a list of heavy documents of td rows each, every row of theirs) is
+// written.  Each lane of a row group reads one list entry of a batch of Lr
 // (the next batch is loaded while this one is gathered); the group gathers
-// the batch's query rows kDdUnroll at a time, taking row and delta by
+// the batch's query rows kCsrDdUnroll at a time, taking row and delta by
 // ds_bpermute.  Entries are checked against the list and the query rows, so
 // a malformed tape or cu cannot send a read out of bounds.
 template <class E, int kCPL>
 __global__ void __launch_bounds__(kBwdThreads) bwd_dd_vec_kernel(
     const uint32_t* rstart, const uint32_t* rcount, const uint2* list, uint32_t nlist,
-    int64_t nrows, RowGeo geo, int64_t rb, const char* Qbase, int64_t nq_rows, char* dD) {
+    int64_t nrows, RowGeo geo, int64_t rb, const char* Qbase, int64_t nq_rows, char* dD,
+    const uint32_t* heavy, int td) {
   constexpr int kV = E::kV;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lg = geo.lg_lr, lr = 1 << lg, rpi = 64 >> lg;
   const int gid = lane >> lg, c0 = lane & (lr - 1), gbase = gid << lg;
   const int64_t per_block = 4 * (int64_t)rpi;
+  if (heavy != nullptr) nrows = (int64_t)rfl32(heavy[0]) * td;  // row x: of heavy document x / td
   auto fetch = [&](uint32_t jj, uint32_t n, uint32_t base) {
     return (jj < n && base + jj < nlist) ? list[base + jj] : make_uint2(0u, 0u);
   };
   for (int64_t rb0 = (int64_t)blockIdx.x * per_block; rb0 < nrows; rb0 += (int64_t)gridDim.x * per_block) {
-    const int64_t r = rb0 + w * rpi + gid;
+    int64_t r = rb0 + w * rpi + gid;
     const bool rv = r < nrows;
+    if (heavy != nullptr && rv) r = (int64_t)heavy[1 + r / td] * td + r % td;
     const uint32_t n = rv ? rcount[r] : 0u;
     const uint32_t base = n ? rstart[r] : 0u;
     const uint32_t nmax = wave_max_u32(n);
@@ -797,11 +1026,11 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dd_vec_kernel(
       const int qlane = ok ? (int)ent.x : 0;
       ent = fetch(j + lr + c0, n, base);  // next batch
       const uint32_t nb = std::min<uint32_t>(lr, nmax - j);
-      for (uint32_t i0 = 0; i0 < nb; i0 += kDdUnroll) {
-        uint4 raw[kDdUnroll][kCPL];
-        float dl[kDdUnroll];
+      for (uint32_t i0 = 0; i0 < nb; i0 += kCsrDdUnroll) {
+        uint4 raw[kCsrDdUnroll][kCPL];
+        float dl[kCsrDdUnroll];
 #pragma unroll
-        for (int i = 0; i < kDdUnroll; ++i) {
+        for (int i = 0; i < kCsrDdUnroll; ++i) {
           const int sl = gbase + (int)((i0 + i) & (uint32_t)(lr - 1));
           dl[i] = (i0 + i < (uint32_t)lr) ? __shfl(dlane, sl) : 0.0f;
           const char* qa = Qbase + (int64_t)__shfl(qlane, sl) * rb;
@@ -813,7 +1042,7 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dd_vec_kernel(
           }
         }
 #pragma unroll
-        for (int i = 0; i < kDdUnroll; ++i)
+        for (int i = 0; i < kCsrDdUnroll; ++i)
 #pragma unroll
           for (int cc = 0; cc < kCPL; ++cc) {
             E::fma_chunk(raw[i][cc], dl[i], acc[cc]);
@@ -1408,16 +1637,18 @@ DocsInBatch make_docs(const LayInBatch& l, const PullbackArgs& a, void*, hipStre
   d.ndocs = l.Bd;
   d.Bd = (uint32_t)l.Bd;
   d.Bq = (uint32_t)(a.npairs / l.Bd);
-  d.rows = a.rows;
+  d.trows = a.rows;
   d.Tq = l.Tq;
+  d.Td = l.Td;
   d.qm = l.qm;
   return d;
 }
 DocsPaired make_docs(const LayPaired& l, const PullbackArgs& a, void*, hipStream_t, hipError_t*) {
   DocsPaired d;
   d.ndocs = a.npairs;
-  d.rows = a.rows;
+  d.trows = a.rows;
   d.Tq = l.Tq;
+  d.Td = l.Td;
   d.qm = l.qm;
   return d;
 }
@@ -1425,8 +1656,9 @@ DocsCand make_docs(const LayCand& l, const PullbackArgs& a, void* gws, hipStream
   DocsCand d;
   d.ndocs = l.N;
   d.C = (uint32_t)l.C;
-  d.rows = a.rows;
+  d.trows = a.rows;
   d.Tq = l.Tq;
+  d.Td = l.Td;
   d.qm = l.qm;
   *e = group_pairs_by_document(l.idx, l.idx64, a.npairs, l.N, gws, &d.order, &d.end, st);
   return d;
@@ -1434,19 +1666,27 @@ DocsCand make_docs(const LayCand& l, const PullbackArgs& a, void* gws, hipStream
 DocsPacked make_docs(const LayPacked& l, const PullbackArgs& a, void*, hipStream_t, hipError_t*) {
   DocsPacked d;
   d.ndocs = a.npairs;
-  d.rows = a.rows;
+  d.trows = a.rows;
   d.qm = l.qm;
+  d.cu = l.cu;
+  d.ntok = l.ntok;
   return d;
 }
 DocsVarlen make_docs(const LayVarlen& l, const PullbackArgs& a, void*, hipStream_t, hipError_t*) {
   DocsVarlen d;
   d.ndocs = a.npairs;
-  d.rows = a.rows;
+  d.trows = a.rows;
   d.cu_q = l.cu_q;
+  d.cu_d = l.cu_d;
   d.nq = l.nq;
+  d.nd = l.nd;
   return d;
 }
 template <class L> size_t docs_workspace(const L&, int64_t) { return 0; }
+// Most sources one document can have (host; candidates: any number).
+int64_t doc_sources(const LayInBatch& l, const PullbackArgs& a) { return a.npairs / l.Bd * a.rows; }
+int64_t doc_sources(const LayCand&, const PullbackArgs& a) { return a.npairs * a.rows; }
+template <class L> int64_t doc_sources(const L&, const PullbackArgs& a) { return a.rows; }
 template <> size_t docs_workspace<LayCand>(const LayCand& l, int64_t npairs) {
   return al256(group_workspace_bytes(npairs, l.N));
 }
@@ -1457,11 +1697,11 @@ template <class L> int64_t staged_rows(const L&) { return -1; }
 template <> int64_t staged_rows<LayInBatch>(const LayInBatch& l) { return l.Td; }
 
 template <class E, class L>
-void launch_dq_staged(const L&, const PullbackArgs&, const RowGeo&, const float*, int, int, int64_t,
-                      int64_t, float*, hipStream_t) {}
+void launch_dq_staged(const L&, const PullbackArgs&, const RowGeo&, const DeltaOf<E>&, int, int,
+                      int64_t, int64_t, float*, hipStream_t) {}
 template <class E>
 void launch_dq_staged(const LayInBatch& lay, const PullbackArgs& a, const RowGeo& geo,
-                      const float* delta, int ntb, int nsplit, int64_t nitems, int64_t rb, float* part,
+                      const DeltaOf<E>& delta, int ntb, int nsplit, int64_t nitems, int64_t rb, float* part,
                       hipStream_t st) {
   const int64_t nblk = bcdiv(nitems, kIbItems) * nsplit;
   if constexpr (E::kSz != 2) return;  // (16-bit features only, see launch_vec)
@@ -1595,8 +1835,9 @@ bool vec_geometry(int64_t rb, int esz, RowGeo* g) {
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 template <class L, class E>
-hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, const float* delta,
-                      hipStream_t st) {
+hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hipStream_t st) {
+  const DeltaOf<E> delta{static_cast<const char*>(a.Delta), static_cast<const char*>(a.inv_n),
+                         (uint32_t)a.G};
   const int64_t rb = (int64_t)a.dim * E::kSz;
   const int64_t ngroups = a.npairs / a.G;
   const int ntb = (int)bcdiv(a.rows, geo.tpw);
@@ -1620,21 +1861,28 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, co
   }
   while (nsplit > 1 && nsplit * a.nq_rows * a.dim * 4 > ((int64_t)512 << 20)) nsplit /= 2;
   if (nsplit < 1) nsplit = 1;
-  // dD: document lists
+  // Workspace: dQ partials, the lists of documents whose sources pass the LDS
+  // list, the document order of candidates (none for pairs of ordinary size).
   const int64_t nsrc = a.npairs * a.rows;
   const size_t b_part = nsplit > 1 ? al256((size_t)(nsplit * a.nq_rows * a.dim) * 4) : 0;
-  const size_t b_rows = al256((size_t)std::max<int64_t>(a.nd_rows, 1) * 4);
-  const size_t b_list = al256((size_t)std::max<int64_t>(nsrc, 1) * 8);
+  constexpr bool kCand = std::is_same<L, LayCand>::value;
+  const bool many = doc_sources(lay, a) > kDocList;  // (for candidates: possibly)
+  const size_t b_list = many ? al256((size_t)nsrc * 8) : 0;
+  const size_t b_rows = many ? al256((size_t)std::max<int64_t>(a.nd_rows, 1) * 4) : 0;
   const size_t b_docs = docs_workspace(lay, a.npairs);
+  const size_t b_heavy = kCand && many ? al256((size_t)(nsrc / kDocList + 1) * 4) : 0;
+  const size_t b_all = b_part + b_list + 2 * b_rows + b_docs + b_heavy;
   void* ws = nullptr;
-  hipError_t e = workspace_alloc(&ws, b_part + 2 * b_rows + b_list + b_docs, st);
+  hipError_t e = hipSuccess;
+  if (b_all > 0) e = workspace_alloc(&ws, b_all, st);
   if (e != hipSuccess) return e;
   char* w = static_cast<char*>(ws);
   float* part = reinterpret_cast<float*>(w);
-  uint32_t* rstart = reinterpret_cast<uint32_t*>(w + b_part);
-  uint32_t* rcount = reinterpret_cast<uint32_t*>(w + b_part + b_rows);
-  uint2* list = reinterpret_cast<uint2*>(w + b_part + 2 * b_rows);
-  void* gws = w + b_part + 2 * b_rows + b_list;
+  uint2* list = reinterpret_cast<uint2*>(w + b_part);
+  uint32_t* rstart = reinterpret_cast<uint32_t*>(w + b_part + b_list);
+  uint32_t* rcount = reinterpret_cast<uint32_t*>(w + b_part + b_list + b_rows);
+  void* gws = w + b_part + b_list + 2 * b_rows;
+  uint32_t* heavy = b_heavy ? reinterpret_cast<uint32_t*>(w + (b_all - b_heavy)) : nullptr;
 
   if (staged) {
     launch_dq_staged<E>(lay, a, geo, delta, ntb, (int)nsplit, nitems, rb, part, st);
@@ -1642,11 +1890,11 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, co
     const int64_t nblk = nitems * nsplit;
     hipLaunchKernelGGL((bwd_dq_vec_kernel<L, E, true>), dim3((unsigned)nblk), dim3(kBwdThreads), 0, st,
                        lay, delta, a.args, a.G, a.rows, ntb, (int)nsplit, nitems, geo, rb, a.dim,
-                       a.Qbase, a.dQ, part, a.nq_rows);
+                       a.Qbase, a.dQ, part, a.nq_rows, heavy);
   } else {
     hipLaunchKernelGGL((bwd_dq_vec_kernel<L, E, false>), dim3((unsigned)bcdiv(nitems, 4)),
                        dim3(kBwdThreads), 0, st, lay, delta, a.args, a.G, a.rows, ntb, 1, nitems,
-                       geo, rb, a.dim, a.Qbase, a.dQ, part, a.nq_rows);
+                       geo, rb, a.dim, a.Qbase, a.dQ, part, a.nq_rows, heavy);
   }
   if (nsplit > 1) {
     const int64_t nchunks = a.nq_rows * rb / 16;
@@ -1659,24 +1907,47 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, co
     hipError_t eg = hipSuccess;
     const auto docs = make_docs(lay, a, gws, st, &eg);
     if (eg == hipSuccess) {
-      hipLaunchKernelGGL(bwd_zero_kernel, dim3(grid_for(bcdiv(a.nd_rows, 64))), dim3(kBwdThreads), 0,
-                         st, rcount, a.nd_rows);
-      const unsigned dblocks = (unsigned)std::min<int64_t>(std::max<int64_t>(docs.ndocs, 1), 65536);
-      hipLaunchKernelGGL((bwd_doc_csr_kernel<L, decltype(docs)>), dim3(dblocks), dim3(kDocThreads), 0,
-                         st, lay, docs, delta, a.args, a.rows, a.Dbase, rb, rstart, rcount, list);
-      const int64_t per_block = 4 * (int64_t)(64 >> geo.lg_lr);
-      const unsigned rblocks = (unsigned)std::min<int64_t>(1048576, bcdiv(a.nd_rows, per_block));
-      if (geo.cpl == 1)
-        hipLaunchKernelGGL((bwd_dd_vec_kernel<E, 1>), dim3(rblocks), dim3(kBwdThreads), 0, st, rstart,
-                           rcount, list, (uint32_t)nsrc, a.nd_rows, geo, rb, a.Qbase, a.nq_rows, a.dD);
-      else
-        hipLaunchKernelGGL((bwd_dd_vec_kernel<E, 2>), dim3(rblocks), dim3(kBwdThreads), 0, st, rstart,
-                           rcount, list, (uint32_t)nsrc, a.nd_rows, geo, rb, a.Qbase, a.nq_rows, a.dD);
+      const int64_t ndocs = std::max<int64_t>(docs.ndocs, 1);
+      if (kCand || !many) {
+        // Shares of a document's rows: enough workgroups for four on each CU, of
+        // at least 32 rows (ragged stores: on average).
+        const int64_t avg = a.nd_rows / ndocs;
+        const int shares = (int)std::max<int64_t>(1, std::min<int64_t>(bcdiv(1024, ndocs), avg / 32));
+        const unsigned blocks = (unsigned)std::min<int64_t>(ndocs * shares, 65536);
+        if (geo.cpl == 1)
+          hipLaunchKernelGGL((bwd_doc_dd_kernel<L, decltype(docs), E, 1>), dim3(blocks), dim3(kDocThreads),
+                             0, st, lay, docs, delta, a.args, a.rows, geo, rb, a.Qbase, a.dD, shares, heavy);
+        else
+          hipLaunchKernelGGL((bwd_doc_dd_kernel<L, decltype(docs), E, 2>), dim3(blocks), dim3(kDocThreads),
+                             0, st, lay, docs, delta, a.args, a.rows, geo, rb, a.Qbase, a.dD, shares, heavy);
+      }
+      if (many) {
+        // (heavy documents: at most nsrc / kDocList of them, usually none)
+        const int td = kCand ? (int)(a.nd_rows / ndocs) : 0;
+        const int64_t cdocs = kCand ? std::min<int64_t>(256, nsrc / kDocList) : ndocs;
+        const int64_t crows = kCand ? std::min<int64_t>(nsrc / kDocList * td, 8192) : a.nd_rows;
+        const int64_t per_block = 4 * (int64_t)(64 >> geo.lg_lr);
+        const unsigned dblocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(cdocs, 65536));
+        const unsigned rblocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(1048576, bcdiv(crows, per_block)));
+        if (!kCand)
+          hipLaunchKernelGGL(bwd_zero_kernel, dim3(grid_for(bcdiv(a.nd_rows, 64))), dim3(kBwdThreads), 0,
+                             st, rcount, a.nd_rows);
+        hipLaunchKernelGGL((bwd_doc_csr_kernel<L, decltype(docs), E>), dim3(dblocks), dim3(kCsrThreads), 0,
+                           st, lay, docs, delta, a.args, a.rows, a.Dbase, rb, rstart, rcount, list, heavy);
+        if (geo.cpl == 1)
+          hipLaunchKernelGGL((bwd_dd_vec_kernel<E, 1>), dim3(rblocks), dim3(kBwdThreads), 0, st, rstart,
+                             rcount, list, (uint32_t)nsrc, a.nd_rows, geo, rb, a.Qbase, a.nq_rows, a.dD,
+                             heavy, td);
+        else
+          hipLaunchKernelGGL((bwd_dd_vec_kernel<E, 2>), dim3(rblocks), dim3(kBwdThreads), 0, st, rstart,
+                             rcount, list, (uint32_t)nsrc, a.nd_rows, geo, rb, a.Qbase, a.nq_rows, a.dD,
+                             heavy, td);
+      }
     }
     e = eg;
   }
   if (e == hipSuccess) e = hipGetLastError();
-  const hipError_t ef = workspace_free(ws, st);
+  const hipError_t ef = ws ? workspace_free(ws, st) : hipSuccess;
   return e != hipSuccess ? e : ef;
 }
 
@@ -1738,6 +2009,13 @@ hipError_t launch_pullback(const L& lay, const PullbackArgs& a, hipStream_t st) 
                                      : false;
     if (took) return eib;
   }
+  RowGeo geo;
+  if (vec_geometry(rb, esz, &geo) && aligned16(a.dQ) && aligned16(a.dD) && aligned16(a.Qbase) &&
+      aligned16(a.Dbase)) {
+    return a.dtype == 0   ? launch_vec<L, EF32>(lay, a, geo, st)
+           : a.dtype == 1 ? launch_vec<L, EF16>(lay, a, geo, st)
+                          : launch_vec<L, EBF16>(lay, a, geo, st);
+  }
   void* ws = nullptr;
   hipError_t e = workspace_alloc(&ws, al256((size_t)a.npairs * 4), st);
   if (e != hipSuccess) return e;
@@ -1753,16 +2031,7 @@ hipError_t launch_pullback(const L& lay, const PullbackArgs& a, hipStream_t st) 
   else
     hipLaunchKernelGGL(bwd_delta_kernel<EBF16>, dim3(flat), dim3(kBwdThreads), 0, st, Dl, Il, a.npairs, a.G, delta);
   if (a.zero_dq) clear(a.dQ, a.nq_rows);
-  RowGeo geo;
-  const bool vec = vec_geometry(rb, esz, &geo) && aligned16(a.dQ) && aligned16(a.dD) &&
-                   aligned16(a.Qbase) && aligned16(a.Dbase);
-  if (vec) {
-    if (a.dtype == 0) e = launch_vec<L, EF32>(lay, a, geo, delta, st);
-    else if (a.dtype == 1) e = launch_vec<L, EF16>(lay, a, geo, delta, st);
-    else e = launch_vec<L, EBF16>(lay, a, geo, delta, st);
-  } else {
-    e = launch_generic(lay, a, delta, st);
-  }
+  e = launch_generic(lay, a, delta, st);
   const hipError_t ef = workspace_free(ws, st);
   return e != hipSuccess ? e : ef;
 }

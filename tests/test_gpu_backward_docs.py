@@ -1,0 +1,104 @@
+"""The per-document dD kernel of the pullbacks at its edges, against the oracle
+(tolerances of test_gpu_backward.py): documents whose sources fit LDS and do
+not (2048), shared by few and by many queries, row tiles (1024 rows), one and
+several shares of a document's rows, a query with more tokens than the list
+holds, and query / document tokens outside every segment."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import as_feature, tokens
+from test_gpu_backward import DT_ID, DTYPES, _abs, _vals, assert_grad
+
+import flashmaxsim as fm
+from flashmaxsim import backward as bw
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a, device):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(device)
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: DT_ID[d])
+@pytest.mark.parametrize("B,C,N,Tq,Td,dim,hot", [
+    (5, 16, 4, 32, 40, 128, 2),      # 640 sources a document, and none on two
+    (9, 60, 30, 32, 33, 64, 3),      # documents past the LDS list among documents without a pair
+    (2, 64, 2, 32, 1030, 128, 1),    # exactly 4096 sources, two row tiles
+    (1, 64, 1, 32, 70, 768, 1),      # exactly 2048: the largest LDS list; two chunks a lane
+])
+def test_candidates_sources_per_document(device, dtype, B, C, N, Tq, Td, dim, hot):
+    rng = np.random.default_rng([B, C, N, Td])
+    Qt, Qo, bf = as_feature(tokens(rng, (B, Tq, dim)), dtype)
+    Gt, Go, _ = as_feature(tokens(rng, (N, Td, dim)), dtype)
+    idx = rng.integers(1, hot + 1, size=(B, C)).astype(np.int64)
+    args = rng.integers(0, Td + 2, size=(B, C, Tq)).astype(np.int32)  # 0 and Td + 1: no source
+    Dl_t, Dl = _vals(rng, (B, C), dtype, device)
+    qm = rng.random((B, Tq)) < (0.9 if N > 2 else 2.0)
+    iv_t, iv = _vals(rng, (B,), dtype, device, positive=True)
+    want = oracle.candidates_backward(Qo, Go, idx, args, Dl, iv, qm, bf16=bf)
+    mag = oracle.candidates_backward(_abs(Qo, bf), _abs(Go, bf), idx, args, np.abs(Dl), iv, qm, bf16=bf)
+    dQ, dG = bw.candidates_pullback(Dl_t, Qt.to(device), Gt.to(device), _dev(idx, device),
+                                    _dev(qm, device), _dev(args, device), iv_t)
+    torch.cuda.synchronize()
+    assert_grad(dQ, want[0], mag[0], dtype, "dQ")
+    assert_grad(dG, want[1], mag[1], dtype, "dG")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: DT_ID[d])
+@pytest.mark.parametrize("Tq,Td,B", [(2048, 35, 2), (2049, 1100, 2), (3, 1, 700), (33, 257, 300)])
+def test_paired_long_queries_and_many_pairs(device, dtype, Tq, Td, B):
+    rng = np.random.default_rng([Tq, Td, B])
+    dim = 64
+    Qt, Qo, bf = as_feature(tokens(rng, (B, Tq, dim)), dtype)
+    Dt, Do, _ = as_feature(tokens(rng, (B, Td, dim)), dtype)
+    args = rng.integers(0, Td + 2, size=(B, Tq)).astype(np.int32)
+    Dl_t, Dl = _vals(rng, (B,), dtype, device)
+    want = oracle.paired_backward(Qo, Do, args, Dl, None, None, bf16=bf)
+    mag = oracle.paired_backward(_abs(Qo, bf), _abs(Do, bf), args, np.abs(Dl), None, None, bf16=bf)
+    dQ, dD = bw.paired_pullback(Dl_t, Qt.to(device), Dt.to(device), None, _dev(args, device))
+    torch.cuda.synchronize()
+    assert_grad(dQ, want[0], mag[0], dtype, "dQ")
+    assert_grad(dD, want[1], mag[1], dtype, "dD")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: DT_ID[d])
+def test_ragged_tokens_outside_every_segment(device, dtype):
+    """A device cu is trusted as given: segments that start late, end early or leave
+    nothing in between; rows of no segment get zero gradients."""
+    rng = np.random.default_rng(5)
+    dim, nq, nd = 64, 40, 90
+    Qt, Qo, bf = as_feature(tokens(rng, (nq, dim)), dtype)
+    Dt, Do, _ = as_feature(tokens(rng, (nd, dim)), dtype)
+    cu_q = np.array([4, 9, 9, 30], np.int32)
+    cu_d = np.array([6, 40, 41, 70], np.int32)
+    max_q = 13  # shorter than the last query segment
+    args = rng.integers(1, 3, size=(3, max_q)).astype(np.int32)
+    Dl_t, Dl = _vals(rng, (3,), dtype, device)
+    P = fm.PackedSeq(Qt.to(device), _dev(cu_q, device), max_q)
+    R = fm.PackedSeq(Dt.to(device), _dev(cu_d, device), 34)
+    dQ, dD = bw.varlen_pullback(Dl_t, P, R, _dev(args, device))
+    q, d = Qt.double().numpy(), Dt.double().numpy()
+    wQ, wD = np.zeros_like(q), np.zeros_like(d)
+    mQ, mD = np.zeros_like(q), np.zeros_like(d)
+    for n in range(3):
+        tq, td = min(cu_q[n + 1] - cu_q[n], max_q), cu_d[n + 1] - cu_d[n]
+        for t in range(tq):
+            u = args[n, t]
+            if u <= td:
+                i, j = cu_q[n] - 1 + t, cu_d[n] - 1 + u - 1
+                wQ[i] += Dl[n] * d[j]
+                wD[j] += Dl[n] * q[i]
+                mQ[i] += abs(Dl[n] * d[j])
+                mD[j] += abs(Dl[n] * q[i])
+    torch.cuda.synchronize()
+    assert_grad(dQ, wQ, mQ, dtype, "dQ")
+    assert_grad(dD, wD, mD, dtype, "dD")
+    q1 = Qt[:7].to(device)
+    tape = rng.integers(1, 3, size=(3, 7)).astype(np.int32)
+    dq, dP = bw.packed_pullback(Dl_t, q1, R, None, _dev(tape, device))
+    torch.cuda.synchronize()
+    g = dP.float().cpu().numpy()
+    assert np.isfinite(g).all() and (g[:5] == 0).all() and (g[69:] == 0).all()
+    assert (g[5:7] != 0).any()
