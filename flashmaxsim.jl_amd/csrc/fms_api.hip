@@ -781,6 +781,15 @@ fms_status fms_varlen_normalize(float* scores, const int32_t* cu_q, int64_t N, v
   return from_hip(varlen_normalize(scores, cu_q, N, as_stream(stream)));
 }
 
+fms_status fms_inverse_counts(int32_t dtype, void* inv_n, const uint8_t* qmask, const int32_t* cu,
+                              int64_t Tq, int64_t n, void* stream) {
+  if (elem_bytes(dtype) == 0) return FMS_EUNSUPPORTED;
+  if (Tq < 0 || n < 0) return FMS_EINVAL;
+  if (n == 0) return FMS_OK;
+  if (!inv_n) return FMS_EINVAL;
+  return from_hip(inverse_counts(dtype, inv_n, qmask, cu, Tq, n, as_stream(stream)));
+}
+
 fms_status fms_topk(const float* scores, int64_t nrows, int64_t ncols, int64_t k, float* vals,
                     int32_t* idx, void* stream) {
   if (nrows < 0 || ncols < 0 || k < 0 || k > ncols) return FMS_EINVAL;

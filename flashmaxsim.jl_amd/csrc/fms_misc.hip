@@ -180,6 +180,46 @@ hipError_t varlen_normalize(float* scores, const int32_t* cu_q, int64_t N, hipSt
   return hipGetLastError();
 }
 
+// Inverse query lengths for the pullbacks, one wave per query (one launch; as
+// tensor operations on the host's side they took one to five).
+__global__ void __launch_bounds__(256) inverse_counts_kernel(int dtype, void* inv_n,
+                                                             const uint8_t* qmask, const int32_t* cu,
+                                                             int64_t Tq, int64_t n) {
+  const int lane = threadIdx.x & 63;
+  const int64_t nw = (int64_t)gridDim.x * 4;
+  for (int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); i < n; i += nw) {
+    int64_t c = Tq;
+    if (cu != nullptr) {
+      c = (int64_t)cu[i + 1] - (int64_t)cu[i];
+    } else if (qmask != nullptr) {
+      c = 0;
+      for (int64_t t0 = 0; t0 < Tq; t0 += 64) {
+        const int64_t t = t0 + lane;
+        c += __builtin_popcountll(__ballot(t < Tq && qmask[i * Tq + t] != 0));
+      }
+    }
+    const float inv = 1.0f / (float)(c > 1 ? c : 1);
+    if (lane != 0) continue;
+    if (dtype == 0) {
+      static_cast<float*>(inv_n)[i] = inv;
+    } else if (dtype == 1) {
+      static_cast<_Float16*>(inv_n)[i] = (_Float16)inv;
+    } else {  // bf16, to nearest even (inv is finite)
+      const uint32_t u = __builtin_bit_cast(uint32_t, inv);
+      static_cast<uint16_t*>(inv_n)[i] = (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
+    }
+  }
+}
+
+hipError_t inverse_counts(int dtype, void* inv_n, const uint8_t* qmask, const int32_t* cu, int64_t Tq,
+                          int64_t n, hipStream_t stream) {
+  int64_t blocks = (n + 3) / 4;
+  if (blocks > 65536) blocks = 65536;
+  hipLaunchKernelGGL(inverse_counts_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, dtype, inv_n,
+                     qmask, cu, Tq, n);
+  return hipGetLastError();
+}
+
 // Accumulator layout probe: one wave, one 32x32 MFMA per feature type.
 // Pass 0 puts A[i][0] = i+1, B[0][j] = 1 (result = row+1); pass 1 puts
 // A[i][0] = 1, B[0][j] = j+1 (result = column+1).  "k = 0" is element 0 of

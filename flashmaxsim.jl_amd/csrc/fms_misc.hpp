@@ -15,6 +15,9 @@ hipError_t length_normalize(float* scores, const uint8_t* qmask, int64_t Tq, int
                             int64_t ncols, const void* idx, int idx64, int64_t N, float neg,
                             hipStream_t stream);
 hipError_t varlen_normalize(float* scores, const int32_t* cu_q, int64_t N, hipStream_t stream);
+// inv_n[i] = 1 / max(count_i, 1) as dtype (0 fp32, 1 fp16, 2 bf16).
+hipError_t inverse_counts(int dtype, void* inv_n, const uint8_t* qmask, const int32_t* cu, int64_t Tq,
+                          int64_t n, hipStream_t stream);
 hipError_t mfma_layout_probe(float* out, int op, hipStream_t stream);
 hipError_t cross_lane_probe(float* out, hipStream_t stream);
 hipError_t read_bandwidth(const void* p, int64_t bytes, uint32_t* out, int blocks,

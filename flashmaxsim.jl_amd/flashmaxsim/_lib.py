@@ -51,6 +51,7 @@ SIGNATURES = {
     "fms_int8_dots": [_p, _p, _p, _i64, _i64, _i64, _p],
     "fms_length_normalize": [_p, _p, _i64, _i64, _i64, _p, _i32, _i64, _f, _p],
     "fms_varlen_normalize": [_p, _p, _i64, _p],
+    "fms_inverse_counts": [_i32, _p, _p, _p, _i64, _i64, _p],
     "fms_debug_mfma_layout": [_p, _i32, _p],
     "fms_debug_read_bandwidth": [_p, _i64, _p, _i32, _p],
     "fms_debug_gather_bandwidth": [_p, _i64, _i64, _p, _i64, _p, _p],

@@ -305,6 +305,20 @@ def topk_rows(vals, idx, scores, k):
     _lib.check(st, "topk")
 
 
+def inverse_counts(inv_n, qmask, cu, Tq):
+    """inv_n (n,) = 1 / max(count, 1) rounded to its eltype: count = the true entries of
+    row i of qmask (n, Tq), cu[i + 1] - cu[i], or Tq (inv_token_counts, normalize.jl:4-10;
+    varlen_inv_n_kernel!, kernels_packed.jl:277-282)."""
+    n = inv_n.numel()
+    if cu is not None:
+        _cu(cu, "cu", n + 1)
+    dev = require_device(inv_n, qmask, cu)
+    st = _lib.lib().fms_inverse_counts(
+        dtype_code(inv_n), ptr(inv_n), ptr(_maskn(qmask, "qmask", n * Tq)), ptr(cu), int(Tq), n,
+        stream_handle(dev))
+    _lib.check(st, "inverse_counts")
+
+
 def launch_varlen_scan(args, partial, Qp, Dp, cu_q, cu_d, scores=None, normalize=False,
                        max_q=None):
     """The shapes come from args (N, max_q), as in the reference method; without a

@@ -1,7 +1,7 @@
 """Layout drivers: allocate outputs, call the boundary, finalize.
 
 Each ``*_forward`` mirrors the reference's device driver ``*_forward_ka``
-(outputs allocated with zeros_like, one scan launch, scores kept on device)
+(outputs allocated, one scan launch that writes them in full, scores kept on device)
 and returns ``(scores, argmax_tape)``.  Σ_t, the candidate ``neg`` fill and,
 with ``normalize=True``, the length normalisation are fused into the scan
 kernel's score write (the reference runs ``sum(partial; dims=1)``,
@@ -25,8 +25,10 @@ from .quant import Int8Index, quantize_int8_symmetric, require_int8_index
 SCORE_DTYPE = torch.float32
 
 
-def _zeros(like: torch.Tensor, dtype, *shape):
-    return torch.zeros(shape, dtype=dtype, device=like.device)
+def _out(like: torch.Tensor, dtype, *shape):
+    """An output buffer.  Not cleared: the scans write every score, tape and partial entry
+    of their pairs (empty documents and masked tokens included)."""
+    return torch.empty(shape, dtype=dtype, device=like.device)
 
 
 # ---- shape checks (DimensionMismatch, as in the reference) ---------------------------
@@ -108,9 +110,9 @@ def pair_forward(q, d, qmask=None, dmask=None, neg=None, normalize=False, tape=T
     dispatch.jl:44-287)."""
     boundary.require_device(q, d, qmask, dmask)
     _, Tq, _ = require_pair_shapes(q, d, qmask, dmask)
-    argmax_u = _zeros(q, torch.int32, Tq) if tape else None
-    partial = _zeros(q, SCORE_DTYPE, Tq) if tape else None
-    score = _zeros(q, SCORE_DTYPE, 1)
+    argmax_u = _out(q, torch.int32, Tq) if tape else None
+    partial = _out(q, SCORE_DTYPE, Tq) if tape else None
+    score = _out(q, SCORE_DTYPE, 1)
     boundary.launch_pair_scan(argmax_u, partial, q, d, qmask, dmask, score, normalize)
     return score, argmax_u
 
@@ -119,8 +121,8 @@ def paired_forward(Q, D, qmask=None, dmask=None, neg=None, normalize=False, tape
     """paired_forward_ka (forward_layouts.jl:112-124): (scores (B,), args (B,Tq))."""
     boundary.require_device(Q, D, qmask, dmask)
     _, Tq, _, B = require_paired_shapes(Q, D, qmask, dmask)
-    args = _zeros(Q, torch.int32, B, Tq) if tape else None
-    scores = _zeros(Q, SCORE_DTYPE, B)
+    args = _out(Q, torch.int32, B, Tq) if tape else None
+    scores = _out(Q, SCORE_DTYPE, B)
     boundary.launch_paired_scan(args, None, Q, D, qmask, dmask, scores, normalize)
     return scores, args
 
@@ -133,10 +135,10 @@ def inbatch_forward(Q, D, qmask=None, dmask=None, neg=None, normalize=False, tap
     it the kernel keeps a running maximum alone (the same S)."""
     boundary.require_device(Q, D, qmask, dmask)
     _, Tq, Bq, Td, Bd = require_inbatch_shapes(Q, D, qmask, dmask)
-    S = _zeros(Q, SCORE_DTYPE, Bq, Bd)
-    args = _zeros(Q, torch.int32, Bq, Bd, Tq) if tape else None
+    S = _out(Q, SCORE_DTYPE, Bq, Bd)
+    args = _out(Q, torch.int32, Bq, Bd, Tq) if tape else None
     if Bd == 0 or Bq == 0 or Tq == 0 or Td == 0:
-        return S, args
+        return S.zero_(), args.zero_() if tape else None
     boundary.inbatch_device_scan(S, args, Q, D, qmask, dmask, normalize)
     return S, args
 
@@ -148,8 +150,8 @@ def candidates_forward(Q, gallery, idxs, qmask=None, dmask=None, neg=-1.0e4, nor
     _, Tq, B, _, N = require_candidates_shapes(Q, gallery, idxs, qmask, dmask)
     idx = indices_on(Q, idxs)
     C = idx.shape[1]
-    args = _zeros(Q, torch.int32, B, C, Tq) if tape else None
-    S = _zeros(Q, SCORE_DTYPE, B, C)
+    args = _out(Q, torch.int32, B, C, Tq) if tape else None
+    S = _out(Q, SCORE_DTYPE, B, C)
     boundary.launch_candidates_scan(args, None, Q, gallery, idx, qmask, dmask, N, S, neg,
                                     normalize)
     return S, args
@@ -164,8 +166,8 @@ def packed_forward(q, P: PackedSeq, qmask=None, neg=None, normalize=False, tape=
     if qmask is not None and qmask.numel() != Tq:
         raise DimensionMismatch("qmask")
     B = P.nseq()
-    args = _zeros(q, torch.int32, B, Tq) if tape else None
-    scores = _zeros(q, SCORE_DTYPE, B)
+    args = _out(q, torch.int32, B, Tq) if tape else None
+    scores = _out(q, SCORE_DTYPE, B)
     boundary.launch_packed_scan(args, None, q, P.tokens, P.cu, qmask, scores, normalize)
     return scores, args
 
@@ -187,8 +189,8 @@ def packed_multi_forward(Q, P: PackedSeq, qmask=None, neg=None, normalize=False,
     if qmask is not None and tuple(qmask.shape) != (nq, Tq):
         raise DimensionMismatch("qmask")
     B = P.nseq()
-    S = _zeros(Q, SCORE_DTYPE, nq, B)
-    args = _zeros(Q, torch.int32, nq, B, Tq) if tape else None
+    S = _out(Q, SCORE_DTYPE, nq, B)
+    args = _out(Q, torch.int32, nq, B, Tq) if tape else None
     if nq == 0 or B == 0:
         return S, args
     boundary.launch_packed_multi_scan(args, S, Q, P.tokens, P.cu, qmask, P.max_len, normalize)
@@ -234,8 +236,8 @@ def varlen_forward(Qp: PackedSeq, Dp: PackedSeq, neg=None, normalize=False, tape
     if Qp.tokens.shape[1] != Dp.tokens.shape[1]:
         raise DimensionMismatch("feature dim")
     max_q = Qp.max_len
-    args = _zeros(Qp.tokens, torch.int32, N, max_q) if tape else None
-    scores = _zeros(Qp.tokens, SCORE_DTYPE, N)
+    args = _out(Qp.tokens, torch.int32, N, max_q) if tape else None
+    scores = _out(Qp.tokens, SCORE_DTYPE, N)
     boundary.launch_varlen_scan(args, None, Qp.tokens, Dp.tokens, Qp.cu, Dp.cu, scores, normalize,
                                 max_q=max_q)
     return scores, args
@@ -256,8 +258,8 @@ def int8_pair_forward(q, d: Int8Index, qmask=None, dmask=None, normalize=False, 
         raise DimensionMismatch("qmask")
     if dmask is not None and dmask.numel() != Td:
         raise DimensionMismatch("dmask")
-    args = _zeros(q, torch.int32, Tq) if tape else None
-    score = _zeros(q, SCORE_DTYPE, 1)
+    args = _out(q, torch.int32, Tq) if tape else None
+    score = _out(q, SCORE_DTYPE, 1)
     boundary.launch_int8_pair_scan(args, None, qq.codes, qq.scales, d.codes, d.scales, qmask,
                                    dmask, score, normalize)
     return score, args
@@ -280,8 +282,8 @@ def int8_paired_forward(Q, D: Int8Index, qmask=None, dmask=None, normalize=False
         raise DimensionMismatch("qmask")
     if dmask is not None and tuple(dmask.shape) != (B, Td):
         raise DimensionMismatch("dmask")
-    args = _zeros(Q, torch.int32, B, Tq) if tape else None
-    scores = _zeros(Q, SCORE_DTYPE, B)
+    args = _out(Q, torch.int32, B, Tq) if tape else None
+    scores = _out(Q, SCORE_DTYPE, B)
     boundary.launch_int8_paired_scan(args, None, QQ.codes, QQ.scales, D.codes, D.scales, qmask,
                                      dmask, scores, normalize)
     return scores, args
@@ -306,8 +308,8 @@ def int8_candidates_forward(Q, G: Int8Index, idxs, qmask=None, dmask=None, neg=-
         raise DimensionMismatch("dmask")
     idx = indices_on(Q, idxs)
     C = idx.shape[1]
-    args = _zeros(Q, torch.int32, B, C, Tq) if tape else None
-    S = _zeros(Q, SCORE_DTYPE, B, C)
+    args = _out(Q, torch.int32, B, C, Tq) if tape else None
+    S = _out(Q, SCORE_DTYPE, B, C)
     boundary.launch_int8_candidates_scan(args, None, QQ.codes, QQ.scales, G.codes, G.scales, idx,
                                          qmask, dmask, N, S, neg, normalize)
     return S, args

@@ -3,7 +3,7 @@ autograd binding.
 
 ``rrule(cfg, *args)`` mirrors ``ChainRulesCore.rrule(maxsim, cfg, args...)``
 (rrule.jl:38-143): it runs the forward once (scores and argmax tape, no dense
-similarity matrix), applies the ``normalize`` finalisation, and returns
+similarity matrix), with the ``normalize`` finalisation in the scan, and returns
 ``(y, pullback)``.  ``pullback(Δ)`` returns one tangent per positional
 argument after the config (``None`` where the reference returns
 ``NoTangent()``); feature tangents are device arrays of the feature eltype,
@@ -26,25 +26,26 @@ from __future__ import annotations
 import torch
 
 from . import backward as BW
+from . import boundary
 from . import forward as F
 from .errors import ArgumentError, DimensionMismatch
 from .packed import PackedSeq
 from .quant import Int8Index
 
 
-def _inv_counts(qmask, B: int, Tq: int, device) -> torch.Tensor:
-    """inv_token_counts (normalize.jl:4-10): fp32 (B,) = 1 / max(count(qmask[:, b]), 1)."""
-    if qmask is None:
-        return torch.full((B,), 1.0 / max(Tq, 1), dtype=torch.float32, device=device)
-    c = qmask.reshape(B, Tq).to(torch.float32).sum(1).clamp(min=1.0)
-    return 1.0 / c
+def _inv_counts(qmask, B: int, Tq: int, proto: torch.Tensor, dtype=None) -> torch.Tensor:
+    """inv_token_counts (normalize.jl:4-10): (B,) = 1 / max(count(qmask[:, b]), 1) in fp32,
+    rounded to the feature eltype (or ``dtype``)."""
+    inv = torch.empty(B, dtype=dtype or proto.dtype, device=proto.device)
+    boundary.inverse_counts(inv, qmask, None, Tq)
+    return inv
 
 
 def _varlen_inv(Q: PackedSeq) -> torch.Tensor:
-    """varlen_inv_n_kernel! (kernels_packed.jl:277-282): 1 / max(Tq_n, 1) per pair."""
-    cu = Q.cu
-    n = (cu[1:] - cu[:-1]).clamp(min=1).to(torch.float32)
-    return 1.0 / n
+    """varlen_inv_n_kernel! (kernels_packed.jl:277-282): 1 / max(Tq_n, 1) per pair, as above."""
+    inv = torch.empty(Q.nseq(), dtype=Q.tokens.dtype, device=Q.tokens.device)
+    boundary.inverse_counts(inv, None, Q.cu, 0)
+    return inv
 
 
 def _cotangent(delta, y: torch.Tensor) -> torch.Tensor:
@@ -90,24 +91,22 @@ def rrule(cfg, *args):
     if isinstance(a, PackedSeq):
         if not isinstance(b, PackedSeq) or rest:
             raise ArgumentError("varlen maxsim takes two PackedSeq")
-        scores, tape = F.varlen_forward(a, b, cfg.neg)
+        y, tape = F.varlen_forward(a, b, cfg.neg, norm)
         inv = _varlen_inv(a) if norm else None
-        y = scores * inv if norm else scores
         T = a.tokens.dtype
 
         def pullback(delta):
             dh = _cotangent(delta, y).to(T)
-            dQ, dD = BW.varlen_pullback(dh, a, b, tape, None if inv is None else inv.to(T), mode)
+            dQ, dD = BW.varlen_pullback(dh, a, b, tape, inv, mode)
             return _pad((dQ, dD), nargs)
         return y, pullback
 
     # ---- several queries against one PackedSeq (extension): per-query pullbacks ----
     if isinstance(b, PackedSeq) and a.dim() == 3:
         qmask = rest[0] if rest else None
-        S, tape = F.packed_multi_forward(a, b, qmask, cfg.neg)
+        y, tape = F.packed_multi_forward(a, b, qmask, cfg.neg, norm)
         nq, Tq = a.shape[0], a.shape[1]
-        inv = _inv_counts(qmask, nq, Tq, a.device) if norm else None
-        y = S * inv[:, None] if norm else S
+        inv = _inv_counts(qmask, nq, Tq, a) if norm else None
         T = a.dtype
 
         def pullback(delta):
@@ -116,7 +115,7 @@ def rrule(cfg, *args):
             dP = None
             for i in range(nq):
                 qi = None if qmask is None else qmask[i].contiguous()
-                iv = None if inv is None else inv[i:i + 1].to(T)
+                iv = None if inv is None else inv[i:i + 1]
                 dq, dp = BW.packed_pullback(dh[i].contiguous(), a[i], b, qi, tape[i].contiguous(),
                                             iv, mode)
                 dQ[i] = dq
@@ -127,15 +126,13 @@ def rrule(cfg, *args):
     # ---- packed (rrule.jl:119-130) ----
     if isinstance(b, PackedSeq):
         qmask = rest[0] if rest else None
-        scores, tape = F.packed_forward(a, b, qmask, cfg.neg)
-        inv = _inv_counts(qmask, 1, a.shape[0], a.device) if norm else None
-        y = scores * inv if norm else scores
+        y, tape = F.packed_forward(a, b, qmask, cfg.neg, norm)
+        inv = _inv_counts(qmask, 1, a.shape[0], a) if norm else None
         T = a.dtype
 
         def pullback(delta):
             dh = _cotangent(delta, y).to(T)
-            dq, dP = BW.packed_pullback(dh, a, b, qmask, tape, None if inv is None else inv.to(T),
-                                        mode)
+            dq, dP = BW.packed_pullback(dh, a, b, qmask, tape, inv, mode)
             return _pad((dq, dP), nargs)
         return y, pullback
 
@@ -156,38 +153,31 @@ def rrule(cfg, *args):
     if rest and _is_index(rest[0]) and not inbatch:
         idxs, masks = rest[0], rest[1:]
         qmask, dmask = (masks + [None, None])[:2]
-        S, tape = F.candidates_forward(a, b, idxs, qmask, dmask, cfg.neg)
-        B, Tq = a.shape[0], a.shape[1]
-        inv = _inv_counts(qmask, B, Tq, a.device) if norm else None
-        y = F.length_normalize_candidates(S, qmask, Tq, idxs, b.shape[0], cfg.neg) if norm else S
+        y, tape = F.candidates_forward(a, b, idxs, qmask, dmask, cfg.neg, norm)
+        inv = _inv_counts(qmask, a.shape[0], a.shape[1], a) if norm else None
 
         def pullback(delta):
             dh = _cotangent(delta, y).to(T)
-            dQ, dG = BW.candidates_pullback(dh, a, b, idxs, qmask, tape,
-                                            None if inv is None else inv.to(T), mode)
+            dQ, dG = BW.candidates_pullback(dh, a, b, idxs, qmask, tape, inv, mode)
             return _pad((dQ, dG), nargs)
         return y, pullback
 
     qmask, dmask = (rest + [None, None])[:2]
     # ---- in-batch (rrule.jl:84-99) ----
     if inbatch:
-        S, tape = F.inbatch_forward(a, b, qmask, dmask, cfg.neg)
-        Bq, Tq = a.shape[0], a.shape[1]
-        inv = _inv_counts(qmask, Bq, Tq, a.device) if norm else None
-        y = S * inv[:, None] if norm else S
+        y, tape = F.inbatch_forward(a, b, qmask, dmask, cfg.neg, norm)
+        inv = _inv_counts(qmask, a.shape[0], a.shape[1], a) if norm else None
 
         def pullback(delta):
             dh = _cotangent(delta, y).to(T)
-            dQ, dD = BW.inbatch_pullback(dh, a, b, qmask, tape,
-                                         None if inv is None else inv.to(T), mode)
+            dQ, dD = BW.inbatch_pullback(dh, a, b, qmask, tape, inv, mode)
             return _pad((dQ, dD), nargs)
         return y, pullback
 
     # ---- pair (rrule.jl:38-66) ----
     if a.dim() == 2:
-        score, tape = F.pair_forward(a, b, qmask, dmask, cfg.neg)
-        inv = _inv_counts(qmask, 1, a.shape[0], a.device) if norm else None
-        y = score * inv if norm else score
+        y, tape = F.pair_forward(a, b, qmask, dmask, cfg.neg, norm)
+        inv = _inv_counts(qmask, 1, a.shape[0], a, torch.float32) if norm else None
 
         def pullback(delta):
             d32 = _cotangent(delta, y)
@@ -197,15 +187,12 @@ def rrule(cfg, *args):
         return y, pullback
 
     # ---- paired (rrule.jl:68-82) ----
-    scores, tape = F.paired_forward(a, b, qmask, dmask, cfg.neg)
-    B, Tq = a.shape[0], a.shape[1]
-    inv = _inv_counts(qmask, B, Tq, a.device) if norm else None
-    y = scores * inv if norm else scores
+    y, tape = F.paired_forward(a, b, qmask, dmask, cfg.neg, norm)
+    inv = _inv_counts(qmask, a.shape[0], a.shape[1], a) if norm else None
 
     def pullback(delta):
         dh = _cotangent(delta, y).to(T)
-        dQ, dD = BW.paired_pullback(dh, a, b, qmask, tape, None if inv is None else inv.to(T),
-                                    mode)
+        dQ, dD = BW.paired_pullback(dh, a, b, qmask, tape, inv, mode)
         return _pad((dQ, dD), nargs)
     return y, pullback
 

@@ -345,6 +345,15 @@ fms_status fms_length_normalize(float* scores, const uint8_t* qmask, int64_t Tq,
 fms_status fms_varlen_normalize(float* scores, const int32_t* cu_q, int64_t N, void* stream);
 
 /*
+ * The inverse query lengths a pullback takes as inv_n (src/normalize.jl:4-10,
+ * src/kernels_packed.jl:277-282): inv_n[i] = 1/max(count_i, 1) in fp32, rounded
+ * to dtype (fp32, fp16 or bf16), i < n; count_i = cu[i+1]-cu[i] when cu is
+ * given, else the true entries of qmask[:,i] (Tq,n), else Tq.
+ */
+fms_status fms_inverse_counts(int32_t dtype, void* inv_n, const uint8_t* qmask,
+                              const int32_t* cu, int64_t Tq, int64_t n, void* stream);
+
+/*
  * Backward on the argmax tape (paper Eqs. 2-3).  For every pair p and query
  * token t with qmask[t] and a tape entry 1 <= u = args[t,p] <= Td(p):
  *     dQ[:, t of p's query]     += delta_p * D[:, u of p's document]
