@@ -745,6 +745,10 @@ int32_t fms_candidates_grouping(int32_t mode) {
   return prev;
 }
 
+void fms_workspace_lend(void* ptr, int64_t bytes) { workspace_lend(ptr, bytes > 0 ? (size_t)bytes : 0); }
+
+int64_t fms_workspace_return(void) { return (int64_t)workspace_return(); }
+
 uint64_t fms_debug_workspace_allocs(void) { return workspace_alloc_count(); }
 
 int32_t fms_debug_inbatch_kernel(int32_t dtype, int64_t dim, int64_t Tq, int64_t Td, int64_t Bq,

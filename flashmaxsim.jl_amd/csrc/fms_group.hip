@@ -411,12 +411,40 @@ hipError_t stream_device(hipStream_t stream, int* dev) {
 
 namespace {
 std::atomic<uint64_t> g_workspace_allocs{0};
+
+struct Loan {
+  char* p = nullptr;
+  size_t bytes = 0, used = 0, wanted = 0;
+};
+thread_local Loan t_loan;
 }  // namespace
+
+void workspace_lend(void* ptr, size_t bytes) {
+  t_loan = Loan();
+  if (ptr != nullptr && (reinterpret_cast<uintptr_t>(ptr) & 255u) == 0) {
+    t_loan.p = static_cast<char*>(ptr);
+    t_loan.bytes = bytes;
+  }
+}
+
+size_t workspace_return() {
+  const size_t wanted = t_loan.wanted;
+  t_loan = Loan();
+  return wanted;
+}
 
 uint64_t workspace_alloc_count() { return g_workspace_allocs.load(std::memory_order_relaxed); }
 
 hipError_t workspace_alloc(void** ptr, size_t bytes, hipStream_t stream) {
   g_workspace_allocs.fetch_add(1, std::memory_order_relaxed);
+  Loan& loan = t_loan;
+  const size_t need = align256(bytes);
+  loan.wanted += need;
+  if (loan.p != nullptr && need <= loan.bytes - loan.used) {
+    *ptr = loan.p + loan.used;
+    loan.used += need;
+    return hipSuccess;
+  }
   int dev = 0;
   hipError_t e = stream_device(stream, &dev);
   if (e != hipSuccess) return e;
@@ -426,6 +454,10 @@ hipError_t workspace_alloc(void** ptr, size_t bytes, hipStream_t stream) {
   return hipMallocFromPoolAsync(ptr, bytes, pool, stream);
 }
 
-hipError_t workspace_free(void* ptr, hipStream_t stream) { return hipFreeAsync(ptr, stream); }
+hipError_t workspace_free(void* ptr, hipStream_t stream) {
+  const uintptr_t off = reinterpret_cast<uintptr_t>(ptr) - reinterpret_cast<uintptr_t>(t_loan.p);
+  if (t_loan.p != nullptr && off < t_loan.bytes) return hipSuccess;
+  return hipFreeAsync(ptr, stream);
+}
 
 }  // namespace fms

@@ -57,6 +57,8 @@ SIGNATURES = {
     "fms_debug_gather_bandwidth": [_p, _i64, _i64, _p, _i64, _p, _p],
     "fms_candidates_grouping": [_i32],
     "fms_debug_workspace_allocs": [],
+    "fms_workspace_lend": [_p, _i64],
+    "fms_workspace_return": [],
     "fms_debug_inbatch_kernel": [_i32, _i64, _i64, _i64, _i64, _i64, _p, _p],
     "fms_debug_cross_lane": [_p, _p],
     "fms_topk": [_p, _i64, _i64, _i64, _p, _p, _p],
@@ -77,6 +79,8 @@ _RESTYPES = {
     "fms_arch_supported": ctypes.c_int,
     "fms_version": ctypes.c_char_p,
     "fms_debug_workspace_allocs": ctypes.c_uint64,
+    "fms_workspace_lend": None,
+    "fms_workspace_return": ctypes.c_int64,
 }
 
 _lib = None

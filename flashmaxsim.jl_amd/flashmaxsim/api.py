@@ -24,12 +24,15 @@ Scores are Float32 for every feature type (score_eltype).
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import forward as F
 from .errors import ArgumentError
 from .packed import PackedSeq
 from .quant import Int8Index
+from .rrule import maxsim_autograd, needs_grad
 
 
 class InBatch:
@@ -59,11 +62,12 @@ def score_eltype(dtype):
 dot_accum = score_eltype
 
 
-def _cast_neg(neg, dtype) -> float:
+@functools.lru_cache(maxsize=64)
+def _cast_neg(neg: float, dtype) -> float:
     """MaxSim{T} stores T(neg) (types.jl:35-38); scores report it as Float32."""
     if dtype in (torch.float16, torch.bfloat16, torch.float32, torch.float64):
-        return float(torch.tensor(float(neg), dtype=dtype).to(torch.float32))
-    return float(torch.tensor(float(neg), dtype=torch.float32))
+        return float(torch.tensor(neg, dtype=dtype).to(torch.float32))
+    return float(torch.tensor(neg, dtype=torch.float32))
 
 
 class MaxSim:
@@ -72,7 +76,7 @@ class MaxSim:
     def __init__(self, dtype=torch.float32, *, neg=-1.0e4, normalize: bool = False,
                  backward=AtomicUnified):
         self.dtype = dtype
-        self.neg = _cast_neg(neg, dtype)
+        self.neg = _cast_neg(float(neg), dtype)
         self.normalize = bool(normalize)
         self.backward = backward() if isinstance(backward, type) else backward
 
@@ -120,7 +124,6 @@ def maxsim(*args, neg=None, normalize=None, backward=None):
             raise ArgumentError("MaxSim feature eltype must match the callable's parameter")
 
     # ---- differentiable call: record the tape and the pullback (rrule.jl) ----
-    from .rrule import maxsim_autograd, needs_grad
     if needs_grad(args):
         return maxsim_autograd(cfg, args)
 

@@ -33,6 +33,8 @@ holds, since both strategies compute the same sums.
 """
 from __future__ import annotations
 
+import threading
+
 import torch
 
 from . import _lib
@@ -60,7 +62,8 @@ def ptr(t):
 
 
 def stream_handle(device: torch.device):
-    return torch.cuda.current_stream(device).cuda_stream
+    """The raw handle of torch's current stream on `device` (no Stream object is built)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def require_device(*ts):
@@ -71,7 +74,7 @@ def require_device(*ts):
             continue
         if not isinstance(t, torch.Tensor):
             raise ArgumentError(f"expected a torch.Tensor, got {type(t).__name__}")
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise ArgumentError(
                 "FlashMaxSim requires colocated arrays (same KernelAbstractions backend) for "
                 "features and masks; the MI355X path needs every array on the HIP device")
@@ -103,6 +106,37 @@ def _idx_bytes(idx: torch.Tensor) -> int:
 def _norm(normalize) -> int:
     """The scans' fused normalize=true epilogue flag (0 or 1)."""
     return 1 if normalize else 0
+
+
+# ---- workspace -------------------------------------------------------------------------
+# The library takes its workspace from a stream-ordered pool of its own, whose
+# allocation holds the host until earlier work on the stream is done (a 64 x 64
+# in-batch call returned after its 64 us on the GPU).  A call that is lent memory
+# uses it instead: a torch allocation on the same stream, as large as the entry
+# point last asked for on this thread, given back when the call returns (the
+# caching allocator reuses it in stream order).  What does not fit, and every
+# allocation under graph capture, comes from the library's pool.
+
+_wanted = threading.local()  # entry point -> bytes its last call on this thread asked for
+
+
+def _call_with_workspace(fn, device, *args):
+    """fn(*args) with lent workspace on `device` (torch's current stream); its status."""
+    L = _lib.lib()
+    wanted = _wanted.__dict__
+    name = fn.__name__
+    n = wanted.get(name, 0)
+    ws = None
+    if n and not torch._C._cuda_isCurrentStreamCapturing():
+        try:
+            ws = torch.empty(n, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            pass  # the library's pool decides
+    L.fms_workspace_lend(ptr(ws), 0 if ws is None else n)
+    try:
+        return fn(*args)
+    finally:
+        wanted[name] = L.fms_workspace_return()
 
 
 # ---- argument checks ---------------------------------------------------------------
@@ -207,7 +241,8 @@ def launch_candidates_scan(args, partial, Q, gallery, idx, qmask, dmask, N, scor
     dev = require_device(args, partial, Q, gallery, idx, qmask, dmask, scores)
     fn = (_lib.lib().fms_launch_candidates_scan_noalloc if noalloc
           else _lib.lib().fms_launch_candidates_scan)
-    st = fn(
+    st = _call_with_workspace(
+        fn, dev,
         dtype_code(Q), ptr(args), ptr(partial), ptr(Q), ptr(gallery), ptr(idx), _idx_bytes(idx),
         ptr(_maskn(qmask, "qmask", B * Tq)), ptr(_maskn(dmask, "dmask", N * Td)), dim, Tq, B, Td, N,
         C, ptr(scores), float(neg), _norm(normalize), stream_handle(dev))
@@ -241,7 +276,8 @@ def inbatch_device_scan(S, args, Q, D, qmask, dmask, normalize=False):
     _buf(S, "S", torch.float32, Bq * Bd)
     _buf(args, "args", torch.int32, Bq * Bd * Tq)
     dev = require_device(S, args, Q, D, qmask, dmask)
-    st = _lib.lib().fms_inbatch_device_scan(
+    st = _call_with_workspace(
+        _lib.lib().fms_inbatch_device_scan, dev, 
         dtype_code(Q), ptr(S), ptr(args), ptr(Q), ptr(D), ptr(_maskn(qmask, "qmask", Bq * Tq)),
         ptr(_maskn(dmask, "dmask", Bd * Td)), dim, Tq, Bq, Td, Bd, _norm(normalize),
         stream_handle(dev))
@@ -281,7 +317,8 @@ def launch_packed_multi_scan(args, scores, Q, tokens, cu, qmask, max_len, normal
     _buf(scores, "scores", torch.float32, nq * B)
     _buf(args, "args", torch.int32, nq * B * Tq)
     dev = require_device(args, scores, Q, tokens, cu, qmask)
-    st = _lib.lib().fms_launch_packed_multi_scan(
+    st = _call_with_workspace(
+        _lib.lib().fms_launch_packed_multi_scan, dev, 
         dtype_code(Q), ptr(args), ptr(scores), ptr(Q), ptr(tokens), ptr(cu),
         ptr(_maskn(qmask, "qmask", nq * Tq)), dim, Tq, nq, B, tokens.shape[0], int(max_len),
         _norm(normalize), stream_handle(dev))
@@ -300,7 +337,8 @@ def topk_rows(vals, idx, scores, k):
         _buf(vals, "vals", torch.float32, nrows * k)
         _buf(idx, "idx", torch.int32, nrows * k)
     dev = require_device(vals, idx, scores)
-    st = _lib.lib().fms_topk(ptr(scores), nrows, ncols, int(k), ptr(vals), ptr(idx),
+    st = _call_with_workspace(
+        _lib.lib().fms_topk, dev, ptr(scores), nrows, ncols, int(k), ptr(vals), ptr(idx),
                              stream_handle(dev))
     _lib.check(st, "topk")
 
@@ -418,7 +456,8 @@ def launch_int8_candidates_scan(args, partial, Qc, Qs, Gc, Gs, idx, qmask, dmask
     _buf(partial, "partial", torch.float32, B * C * Tq)
     _buf(scores, "scores", torch.float32, B * C)
     dev = require_device(args, partial, Qc, Qs, Gc, Gs, idx, qmask, dmask, scores)
-    st = _lib.lib().fms_launch_int8_candidates_scan(
+    st = _call_with_workspace(
+        _lib.lib().fms_launch_int8_candidates_scan, dev, 
         ptr(args), ptr(partial), ptr(Qc), ptr(Qs), qsc, ptr(Gc), ptr(Gs), dsc, ptr(idx),
         _idx_bytes(idx), ptr(_maskn(qmask, "qmask", B * Tq)), ptr(_maskn(dmask, "dmask", N * Td)),
         dim, Tq, B, Td, N, C, ptr(scores), float(neg), _norm(normalize), stream_handle(dev))
@@ -499,7 +538,8 @@ def pair_apply_pullback(dq, dd, q, d, qmask, argmax_u, delta):
     Td = d.shape[0]
     for t, w in ((dq, "dq"), (dd, "dd"), (d, "d"), (delta, "delta")):
         _like(t, q, w)
-    st = _lib.lib().fms_pair_pullback(
+    st = _call_with_workspace(
+        _lib.lib().fms_pair_pullback, dev, 
         dtype_code(q), ptr(dq), ptr(dd), ptr(q), ptr(d), ptr(_mask(qmask)), ptr(_tape(argmax_u)),
         ptr(delta), dim, Tq, Td, stream_handle(dev))
     _lib.check(st, "pair_apply_pullback")
@@ -511,7 +551,8 @@ def paired_apply_pullback(dQ, dD, Q, D, qmask, args, Delta, inv_n):
     Td = D.shape[1]
     for t, w in ((dQ, "dQ"), (dD, "dD"), (D, "D"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, Q, w)
-    st = _lib.lib().fms_paired_pullback(
+    st = _call_with_workspace(
+        _lib.lib().fms_paired_pullback, dev, 
         dtype_code(Q), ptr(dQ), ptr(dD), ptr(Q), ptr(D), ptr(_mask(qmask)), ptr(_tape(args)),
         ptr(Delta), ptr(inv_n), dim, Tq, Td, B, stream_handle(dev))
     _lib.check(st, "paired_apply_pullback")
@@ -524,7 +565,8 @@ def inbatch_apply_pullback(dQ, dD, Q, D, qmask, args, Delta, inv_n):
     Bd, Td = D.shape[0], D.shape[1]
     for t, w in ((dQ, "dQ"), (dD, "dD"), (D, "D"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, Q, w)
-    st = _lib.lib().fms_inbatch_pullback(
+    st = _call_with_workspace(
+        _lib.lib().fms_inbatch_pullback, dev, 
         dtype_code(Q), ptr(dQ), ptr(dD), ptr(Q), ptr(D), ptr(_mask(qmask)), ptr(_tape(args)),
         ptr(Delta), ptr(inv_n), dim, Tq, Td, Bq, Bd, stream_handle(dev))
     _lib.check(st, "inbatch_apply_pullback")
@@ -538,7 +580,8 @@ def candidates_apply_pullback(dQ, dG, Q, gallery, idx, qmask, args, Delta, inv_n
     C = idx.shape[1]
     for t, w in ((dQ, "dQ"), (dG, "dG"), (gallery, "gallery"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, Q, w)
-    st = _lib.lib().fms_candidates_pullback(
+    st = _call_with_workspace(
+        _lib.lib().fms_candidates_pullback, dev, 
         dtype_code(Q), ptr(dQ), ptr(dG), ptr(Q), ptr(gallery), ptr(idx), _idx_bytes(idx),
         ptr(_mask(qmask)), ptr(_tape(args)), ptr(Delta), ptr(inv_n), dim, Tq, B, Td, N, C,
         stream_handle(dev))
@@ -553,7 +596,8 @@ def packed_apply_pullback(dq, dP, q, tokens, cu, qmask, args, Delta, inv_n):
         raise ArgumentError("PackedSeq cu must be Int32 on device")
     for t, w in ((dq, "dq"), (dP, "dP"), (tokens, "tokens"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, q, w)
-    st = _lib.lib().fms_packed_pullback(
+    st = _call_with_workspace(
+        _lib.lib().fms_packed_pullback, dev, 
         dtype_code(q), ptr(dq), ptr(dP), ptr(q), ptr(tokens), ptr(cu), ptr(_mask(qmask)),
         ptr(_tape(args)), ptr(Delta), ptr(inv_n), dim, Tq, B, tokens.shape[0],
         stream_handle(dev))
@@ -569,7 +613,8 @@ def varlen_apply_pullback(dQ, dD, Qp, Dp, cu_q, cu_d, args, Delta, inv_n):
         raise ArgumentError("PackedSeq cu must be Int32 on device")
     for t, w in ((dQ, "dQ"), (dD, "dD"), (Dp, "D tokens"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, Qp, w)
-    st = _lib.lib().fms_varlen_pullback(
+    st = _call_with_workspace(
+        _lib.lib().fms_varlen_pullback, dev, 
         dtype_code(Qp), ptr(dQ), ptr(dD), ptr(Qp), ptr(Dp), ptr(cu_q), ptr(cu_d),
         ptr(_tape(args)), ptr(Delta), ptr(inv_n), dim, max_q, N, Qp.shape[0], Dp.shape[0],
         stream_handle(dev))

@@ -451,8 +451,23 @@ fms_status fms_debug_mfma_layout(float* out, int32_t dtype_or_int8, void* stream
 fms_status fms_debug_cross_lane(float* out, void* stream);
 
 /*
- * Test-only: the number of workspace allocations the library has requested
- * from its stream-ordered pool in this process (no reference counterpart).
+ * Workspace lent to the calling host thread's next calls (no reference
+ * counterpart).  An entry point that needs workspace takes it from the library's
+ * stream-ordered pool; allocating there holds the host until earlier work on the
+ * stream is done.  Between fms_workspace_lend(ptr, bytes) and
+ * fms_workspace_return() it uses the lent device memory first (256-byte aligned,
+ * on the device of the calls' stream; NULL or 0 bytes lends none) and the pool
+ * for what does not fit.  Work that uses the memory is enqueued on the calls'
+ * streams: the owner may reuse it in stream order, or once that work is done.
+ * fms_workspace_return ends the loan and returns the bytes asked for since it
+ * began, i.e. what would have fitted everything.
+ */
+void fms_workspace_lend(void* ptr, int64_t bytes);
+int64_t fms_workspace_return(void);
+
+/*
+ * Test-only: the number of workspace allocations the library's calls have made
+ * in this process, from its stream-ordered pool or from lent memory (no reference counterpart).
  * Lets a test show that fms_launch_candidates_scan_noalloc takes none.
  */
 uint64_t fms_debug_workspace_allocs(void);
