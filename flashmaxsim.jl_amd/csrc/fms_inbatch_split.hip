@@ -8,29 +8,31 @@
 // the reference materialises D'Q chunks and runs an argmax-accumulate); the
 // same fused scores and argmax tape as the other in-batch kernel.
 //
-// Work item = one document j x kRows query rows (a query row is a 32-token
-// tile of a query: query v / ntq, tokens 32 (v % ntq) ..).  Blocks of 4
+// A plan lists the call's document chunks that hold a valid row, in document
+// order (a document without one keeps one chunk, all masked, so that it
+// closes), and cuts the list into R ranges of equal length at document
+// boundaries.  Work item = one range x kRows query rows (a query row is a
+// 32-token tile of a query: query v / ntq, tokens 32 (v % ntq) ..).  Blocks of 4
 // waves, one per CU for 16-bit features and two for fp32, each walk their
-// items in turn (a persistent grid).  An item's document chunks are taken
-// kCg at a time (a chunk group: 6 chunks for 16-bit features, 3 for fp32);
-// per group the block runs the whole K loop:
+// items in turn (a persistent grid).  An item's chunks are taken kCg at a time
+// whatever documents they belong to (a chunk group: 6 chunks for 16-bit
+// features, 3 for fp32); per group the block runs the whole K loop:
 //   * K advances by a slice of 128 bytes of every row (64 features of a
-//     16-bit type, 32 of fp32).  The document's slice (shared by the four
-//     waves) goes HBM/L2 -> LDS with direct buffer-to-LDS loads (no
-//     registers in between), in MFMA fragment order: 1 KB per (chunk, unit
-//     pair m), lane l's 16 bytes at l * 16 = row l % 32, 16-byte unit
-//     2m + l / 32 of the slice, so a fragment read is 1 KB contiguous over
-//     the wave (no bank conflicts).  A wave's own query rows' fragments are
-//     loaded straight into registers in the same order.  Rows past the
-//     document or the query, and units past the row (the last slice of a
-//     dim that is not a multiple of it) read zeros (buffer bounds);
+//     16-bit type, 32 of fp32).  The chunks' slice (shared by the four
+//     waves) goes HBM/L2 -> LDS with direct buffer-to-LDS loads of whole rows
+//     (layout below).  A wave's own query rows' fragments are loaded straight
+//     into registers.  Rows past the document or the query, and units past the
+//     row (the last slice of a dim that is not a multiple of it) read zeros
+//     (buffer bounds);
 //   * the block's slices (items, their groups, their K slices, in order)
 //     form one stream with three stages: slice task p + 2 is requested
 //     while task p is multiplied, across group and item boundaries, so an
 //     item's first slices arrive while the previous item folds and closes;
-//     one barrier per task (every wave's share of task p has landed, and
-//     every wave is done with the stage task p - 1 used, which the request
-//     of task p + 2 then refills);
+//     one barrier per task (every wave's share of task p + 1 has landed, and
+//     every wave is done with the stage of task p, which the request of task
+//     p + 3 then refills).  It stands before the last quarter of task p's
+//     MFMAs, and task p + 1's first fragments are read behind it, so neither
+//     the barrier nor the LDS latency holds up the matrix cores;
 //   * wave w holds the accumulators of query rows 2w, 2w + 1 for the whole
 //     chunk group (2 x kCg 32x32 tiles): each query fragment read feeds kCg
 //     MFMA chains and each document fragment read two;
@@ -40,16 +42,24 @@
 //     bijection for both operands, so the four MFMAs sum the 8 features of
 //     the unit pair;
 //   * after a group's last slice each accumulator tile is folded, chunk by
-//     chunk in document order, into the running max / argmax exactly as the
-//     scans fold (first valid row taken, then strictly greater; chunk valid
-//     words from a plan kernel over dmask and Td), and the item's last group
-//     closes the tiles: wave halves merged, tape rows and the score written
-//     straight to global memory.
-// Item -> (document, query group) is XCD-aware: each XCD takes every 8th
-// document, in bands of kBand documents; within a band the document runs
-// fastest, so the XCD's 32 CUs hold kBand documents x 32 / kBand query groups
-// at a time, and the band's documents stay in that XCD's L2 while all query
-// groups pass over them.
+//     chunk in list order, into the running max / argmax exactly as the
+//     scans fold (first valid row taken, then strictly greater), and a
+//     document's last chunk closes it: wave halves merged, tape rows and the
+//     score written straight to global memory.  Without a tape (args null) the
+//     fold is the max3 tree alone.
+// Item -> (range, query group) is XCD-aware: an XCD's 32 CUs hold a few query
+// groups x several ranges at a time: a chunk is read by the CUs of several query
+// groups and a query row by those of several ranges (split_slot, split_cut).
+//
+// Measured, us per call on documents of U[Td / 3, Td] tokens, scores alone / with
+// the tape, against one document per item, all its chunks multiplied and a
+// task's loads ahead of its MFMAs: bf16, d = 768, 256 x 256, Td = 180: 655 / 656 ->
+// 408 / 451 (0.96 PFLOP/s on valid tokens); 512 x 512 2591 / 2605 -> 1532 / 1710;
+// fp16, d = 256, 512 x 512, Td = 300 1980 / 1990 -> 1019 / 1260; fp32, d = 128, 512 x
+// 512 3289 / 3308 -> 2116 / 2209; 64 x 64 bf16, d = 768 47 -> 45.  Full documents: bf16
+// 256 x 256 663 -> 543.  Bound by the MFMAs and, in 16 bits, by the one wave per
+// SIMD that the accumulators leave: its fold and close run with the matrix cores
+// idle.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -97,7 +107,6 @@ struct SplitShape {
 constexpr int kMaxCg = SplitShape<2>::kCg;  // the largest group (range checks)
 static_assert(SplitShape<4>::kCg <= kMaxCg, "range checks cover every shape");
 constexpr int kSpXcds = 8;
-constexpr int kBand = 8;  // documents an XCD keeps in flight together
 
 // The block's waves have all landed their loads of the slice to be read next
 // (each leaves only its kVm most recent loads in flight) and finished their
@@ -123,6 +132,25 @@ __device__ __forceinline__ typename Op::Acc mma_pair(u32x4 a, u32x4 b, typename 
   } else {
     return Op::mma(a, b, acc);
   }
+}
+
+// base[at] = v for at < n (wave-uniform base and n), nothing past it.  The task
+// loop's stores go through this, none under a branch on the lane: divergent
+// control flow there makes the compiler restructure the whole loop.  (A device
+// function: a resource local to a lambda keeps the host compile from emitting
+// the kernel's launch stub.)
+__device__ __forceinline__ void store_below(const void* base, int n, int at, uint32_t v) {
+  __builtin_amdgcn_raw_buffer_store_b32(v, make_rsrc_u(base, (uint32_t)n * 4u), at * 4, 0, 0);
+}
+
+// A wave's 16 bytes per lane HBM/L2 -> LDS, and into registers, with a scalar
+// offset (device functions, not lambdas, for the same reason).
+__device__ __forceinline__ void copy16_lds(rsrc_t r, u32x4* dst, int voff, int soff) {
+  typedef __attribute__((address_space(3))) void* lds_void_t;
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t)dst, 16, voff, soff, 0, 0);
+}
+__device__ __forceinline__ u32x4 load16_at(rsrc_t r, int voff, int soff) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
 // Valid-row words of the call, one launch before the scan: plan[j * nch + c]
@@ -154,56 +182,136 @@ __global__ void __launch_bounds__(256) split_plan_kernel(const uint8_t* dm, cons
   }
 }
 
-// Slot x of the block order -> (document, query group).  Slots are dealt
-// round-robin to the 8 XCDs (slot x runs on XCD x % 8: the grid is a multiple
-// of 8 and each block walks slots blockIdx.x + n * gridDim.x); XCD x serves
-// documents 8 dl + x, dl < ndx, in bands of kBand consecutive dl: inside a
-// band dl runs fastest, then the query group.  A document index >= Bd marks
-// a slot with no work (the last band when Bd is not a multiple of 8).
-__device__ __forceinline__ int split_slot_doc(int x, int nqg, int ndx, int& qg) {
-  const int xcd = x % kSpXcds, kx = x / kSpXcds;
-  const int band = kx / (kBand * nqg);
-  const int bsz = std::min(kBand, ndx - band * kBand);
-  const int within = kx - band * kBand * nqg;
-  qg = within / bsz;
-  return (band * kBand + within % bsz) * kSpXcds + xcd;
+// The chunk list, one block: entry {valid rows, document, chunk | last << 31, 0}
+// per listed chunk (see above), and rs[r], the first entry of range r (rs[R]: the
+// entries' number).  byDocs: range r starts at document r Bd / R; otherwise at the
+// first document whose first entry is at or past r / R of the list.
+constexpr int kListThreads = 1024;
+__global__ void __launch_bounds__(kListThreads) split_list_kernel(const uint32_t* plan, int Bd, int nch,
+                                                                  int R, int byDocs, uint4* list,
+                                                                  int32_t* rs) {
+  __shared__ int wsum[kListThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  constexpr int kWords = 8;  // plan words in flight per thread
+  // f(chunk, valid rows) for the chunks of document j with a valid row
+  auto each_chunk = [&](int j, auto f) {
+    const uint32_t* const words = plan + (int64_t)j * nch;
+    for (int c0 = 0; c0 < nch; c0 += kWords) {
+      uint32_t m[kWords];
+#pragma unroll
+      for (int i = 0; i < kWords; ++i) m[i] = c0 + i < nch ? words[c0 + i] : 0u;
+#pragma unroll
+      for (int i = 0; i < kWords; ++i)
+        if (m[i] != 0u) f(c0 + i, m[i]);
+    }
+  };
+  auto chunks_of = [&](int j) {
+    int n = 0;
+    each_chunk(j, [&](int, uint32_t) { ++n; });
+    return n > 0 ? n : 1;
+  };
+  // exclusive prefix of v over the block and its total (two barriers)
+  auto scan = [&](int v, int& total) {
+    int x = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[w] = x;
+    __syncthreads();
+    int before = x - v;
+    total = 0;
+#pragma unroll
+    for (int i = 0; i < kListThreads / 64; ++i) {
+      if (i < w) before += wsum[i];
+      total += wsum[i];
+    }
+    __syncthreads();
+    return before;
+  };
+  int all = 0;
+  if (!byDocs)
+    for (int j0 = 0; j0 < Bd; j0 += kListThreads) {
+      int t;
+      scan(j0 + tid < Bd ? chunks_of(j0 + tid) : 0, t);
+      all += t;
+    }
+  // the range that document j, first entry e, belongs to
+  auto range_of = [&](int j, int e) {
+    return byDocs ? (int)(((int64_t)j * R + R - 1) / Bd) : (int)(((int64_t)e * R) / all);
+  };
+  int base = 0;
+  for (int j0 = 0; j0 < Bd; j0 += kListThreads) {
+    const int j = j0 + tid;
+    const int n = j < Bd ? chunks_of(j) : 0;
+    int t;
+    const int e0 = base + scan(n, t);
+    base += t;
+    if (n == 0) continue;
+    int e = e0;
+    each_chunk(j, [&](int c, uint32_t m) {
+      list[e] = make_uint4(m, (uint32_t)j, (uint32_t)c | ((e + 1 == e0 + n) ? 0x80000000u : 0u), 0u);
+      ++e;
+    });
+    if (e == e0) list[e] = make_uint4(0u, (uint32_t)j, 0x80000000u, 0u);
+    // the ranges that start at the next document (or, past the last one, at the end)
+    const int en = e0 + n, lo = range_of(j, e0), hi = j + 1 == Bd ? R : range_of(j + 1, en);
+    if (j == 0) rs[0] = 0;
+    for (int r = lo + 1; r <= hi; ++r) rs[r] = en;
+  }
+}
+
+// Slot x of the block order -> (range, query group); qg = nqg marks a slot with
+// no work.  Slots are dealt round-robin to the 8 XCDs (slot x runs on XCD x % 8:
+// the grid is a multiple of 8 and each block walks slots blockIdx.x + n *
+// gridDim.x).  XCD x takes every xq-th query group and every (8 / xq)-th range,
+// and goes through its ranges for one query group before the next.
+__device__ __forceinline__ int split_slot(int x, int nqg, int R, int xq, int& qg) {
+  const int xcd = x % kSpXcds, k = x / kSpXcds, xr = kSpXcds / xq;
+  const int nrx = (R + xr - 1) / xr;
+  const int r = (k % nrx) * xr + xcd / xq;
+  const int g = (k / nrx) * xq + xcd % xq;
+  qg = r < R && g < nqg ? g : nqg;
+  return r;
 }
 
 // kWhole: rows are whole slices (rowbytes a multiple of kSliceBytes, as at
 // d = 768 in 16 bits or d = 128 in fp32), so no unit lies past a row's end
 // and the slice's byte offset goes to the loads' scalar offset.
-template <class Op, bool kWhole>
+template <class Op, bool kWhole, bool kTape>
 __global__ void __launch_bounds__(64 * kSpWaves, SplitShape<Op::kEsz>::kBlocks)
     inbatch_split(const InBatchSplitArgs A) {
   typedef typename Op::Acc Acc;
   typedef SplitShape<Op::kEsz> Shape;
   constexpr int kCg = Shape::kCg, kDFrags = Shape::kDFrags, kAfterCopies = Shape::kAfterCopies;
-  constexpr int kMmaPerPair = Op::kEsz == 4 ? 4 : 1;
-  typedef __attribute__((address_space(3))) void* lds_void_t;
-  __shared__ u32x4 dbuf[kStages][kDFrags * 64];
+  // three arrays, not one indexed by stage: the compiler then sees that a copy
+  // into one stage cannot alias reads of another
+  __shared__ u32x4 dbuf0[kDFrags * 64], dbuf1[kDFrags * 64], dbuf2[kDFrags * 64];
+  static_assert(kStages == 3, "three stages, and the task loop below is unrolled by three");
 
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
   const int r32 = lane & 31, h = lane >> 5;
 
-  const int rowbytes = A.rowbytes, Tq = A.Tq, Td = A.Td, ntq = A.ntq, Bd = A.Bd, nqg = A.nqg;
+  const int rowbytes = A.rowbytes, Tq = A.Tq, Td = A.Td, ntq = A.ntq, Bd = A.Bd, nqg = A.nqg, R = A.R, xq = A.xq;
   const int nslices = (rowbytes + kSliceBytes - 1) / kSliceBytes;
-  const int nch = Td > 0 ? (Td + kTile - 1) / kTile : 0;
-  const int ngroups = (nch + kCg - 1) / kCg;
   const int nqv = A.Bq * ntq;
-  const int ndx = (Bd + kSpXcds - 1) / kSpXcds;
   const int G = gridDim.x;
-  // The plan words are read through the constant address space: scalar
-  // loads (wave-uniform words, lgkmcnt), nothing in the vector-memory count
-  // that the slice waits rely on.  The kernel never writes them.
+  // The plan is read through the constant address space: scalar loads
+  // (wave-uniform words, lgkmcnt), nothing in the vector-memory count that the
+  // slice waits rely on.  The kernel never writes it.
   typedef __attribute__((address_space(4))) const uint32_t* cword_ptr;
-  const cword_ptr cmask = (cword_ptr)(uintptr_t)A.plan;
-  const cword_ptr qmask = cmask + (int64_t)Bd * nch;
+  typedef __attribute__((address_space(4))) const int32_t* cint_ptr;
+  const cword_ptr clist = (cword_ptr)(uintptr_t)A.list;
+  const cint_ptr crs = (cint_ptr)(uintptr_t)A.rs;
+  const cword_ptr qmask = (cword_ptr)(uintptr_t)A.qwords;
 
-  // This block's slots with a document, in order.
+  // This block's slots with work, in order: the first at or after x.
   auto next_slot = [&](int x) {
     for (; x < A.nslots; x += G) {
       int qg;
-      if (split_slot_doc(x, nqg, ndx, qg) < Bd) break;
+      const int r = split_slot(x, nqg, R, xq, qg);
+      if (qg < nqg && crs[r] < crs[r + 1]) break;
     }
     return x;
   };
@@ -213,31 +321,28 @@ __global__ void __launch_bounds__(64 * kSpWaves, SplitShape<Op::kEsz>::kBlocks)
     int qv[2], qi[2], qt0[2], qtn[2];
   };
   auto rows_of = [&](int qg) {
-    Rows R;
+    Rows Rw;
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       const int v = qg * kRows + 2 * wave + q;
       const bool live = v < nqv;
-      R.qv[q] = live ? v : -1;
-      R.qi[q] = live ? v / ntq : 0;
-      R.qt0[q] = live ? (v - R.qi[q] * ntq) * kTile : 0;
-      R.qtn[q] = live ? std::min(kTile, Tq - R.qt0[q]) : 0;
+      Rw.qv[q] = live ? v : -1;
+      Rw.qi[q] = live ? v / ntq : 0;
+      Rw.qt0[q] = live ? (v - Rw.qi[q] * ntq) * kTile : 0;
+      Rw.qtn[q] = live ? std::min(kTile, Tq - Rw.qt0[q]) : 0;
     }
-    return R;
+    return Rw;
   };
 
   // ---- the load stream ---------------------------------------------------------
-  // A block's work is one sequence of slice tasks: its slots (items) in order,
-  // each item its chunk groups in order, each group its K slices.  The stream
-  // requests task p + 2 while task p is multiplied, across group and item
-  // boundaries, so a new item's first slices arrive while the previous item
-  // folds and closes.  Per task and wave: kCg document copies into LDS (the
-  // four waves together copy the whole slice), then this wave's own query
-  // fragments (2 rows x kPairs unit pairs) into registers, lane l reading
-  // row l % 32, unit 2m + l / 32 of the slice.  Rows past the document or
-  // query and units past the row read out of range (zeros).  Past the last
-  // task the resources are empty: the same operations, no memory traffic.
-  // Document copies read whole rows: a wave's copy of chunk c is its rows
+  // Per task and wave: kCg document copies into LDS (the four waves together
+  // copy the whole slice), then this wave's own query fragments (2 rows x
+  // kPairs unit pairs) into registers, lane l reading row l % 32, unit 2m +
+  // l / 32 of the slice.  Each chunk of the group has a buffer resource of its
+  // own (its rows up to the document's end; empty past the item's last chunk
+  // and past the block's last task: the same operations, no memory traffic), so
+  // a lane's offset is the same for every chunk, group and slice.
+  // Document copies read whole rows: a wave's copy of a chunk is its rows
   // 8w .. 8w + 7 (1 KB, 8 cache lines), lane l taking row 8w + l / 8 and the
   // unit that leaves the chunk row-major with each row's 8 units
   // XOR-swizzled: unit u of row r at r * 8 + (u ^ key(r)), key(r) =
@@ -245,235 +350,274 @@ __global__ void __launch_bounds__(64 * kSpWaves, SplitShape<Op::kEsz>::kBlocks)
   // on 16 distinct 16-byte bank groups for any 16 consecutive lanes.
   const int crow = 8 * wave + (lane >> 3);
   const int copy_off = ((lane & 7) ^ ((crow >> 1) & 7)) * 16;
+  const int dvoff = crow * rowbytes, qvoff = r32 * rowbytes + h * 16;
   int roff[kPairs];  // fragment m of a chunk: u32x4 index in the chunk's 4 KB
 #pragma unroll
   for (int m = 0; m < kPairs; ++m) roff[m] = r32 * 8 + ((2 * m + h) ^ ((r32 >> 1) & 7));
-  int is_slot = next_slot(blockIdx.x), is_g = 0, is_s = 0;
-  rsrc_t rdoc, rq[2];
+  int is_slot = next_slot(blockIdx.x), is_e = 0, is_end = 0, is_s = 0;
+  rsrc_t rdoc[kCg], rq[2];
+  auto set_issue_group = [&]() {
+#pragma unroll
+    for (int c = 0; c < kCg; ++c) {
+      const bool in = is_e + c < is_end;
+      const int64_t e = in ? is_e + c : 0;
+      const int j = (int)clist[e * 4 + 1], ch = (int)(clist[e * 4 + 2] & 0x7fffffffu);
+      const int rows = in ? std::min(kTile, Td - ch * kTile) : 0;
+      rdoc[c] = make_rsrc_u(A.D + ((int64_t)j * Td + ch * kTile) * rowbytes,
+                            rows > 0 ? (uint32_t)rows * (uint32_t)rowbytes : 0u);
+    }
+  };
   auto set_issue_item = [&]() {
     if (is_slot < A.nslots) {
       int qg;
-      const int j = split_slot_doc(is_slot, nqg, ndx, qg);
-      const Rows R = rows_of(qg);
-      rdoc = make_rsrc_u(A.D + (int64_t)j * Td * rowbytes, (uint32_t)Td * (uint32_t)rowbytes);
+      const int r = split_slot(is_slot, nqg, R, xq, qg);
+      is_e = crs[r];
+      is_end = crs[r + 1];
+      const Rows Rw = rows_of(qg);
 #pragma unroll
       for (int q = 0; q < 2; ++q)
-        rq[q] = make_rsrc_u(A.Q + ((int64_t)R.qi[q] * Tq + R.qt0[q]) * rowbytes,
-                            (uint32_t)R.qtn[q] * (uint32_t)rowbytes);
+        rq[q] = make_rsrc_u(A.Q + ((int64_t)Rw.qi[q] * Tq + Rw.qt0[q]) * rowbytes,
+                            (uint32_t)Rw.qtn[q] * (uint32_t)rowbytes);
     } else {
-      rdoc = make_rsrc_u(A.D, 0u);
+      is_e = is_end = 0;
       rq[0] = rq[1] = make_rsrc_u(A.Q, 0u);
     }
+    set_issue_group();
   };
   set_issue_item();
   // Query fragments of kStages tasks in flight: set k holds tasks 3n + k.
   u32x4 qf[kStages][2][kPairs];
-  auto issue = [&](auto SETc) {
-    constexpr int kSet = decltype(SETc)::value;
-    // A unit past the row end is pushed out of range with all low 31 bits set
-    // (branch-free: a select here became divergent branches around the loads).
-    if constexpr (kWhole) {
-      const int so = is_s * kSliceBytes;  // uniform: the loads' scalar offset
-#pragma unroll
-      for (int c = 0; c < kCg; ++c) {
-        const int row = (is_g * kCg + c) * kTile + crow;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rdoc, (lds_void_t)&dbuf[kSet][c * 256 + wave * 64],
-                                                 16, row * rowbytes + copy_off, so, 0, 0);
+  // Load i of a task (0 .. kOpsPerSlice - 1): a document copy or a query fragment.
+  auto issue_one = [&](auto SETc, auto Ic) {
+    constexpr int kSet = decltype(SETc)::value, i = decltype(Ic)::value;
+    u32x4* const dst = kSet == 0 ? dbuf0 : kSet == 1 ? dbuf1 : dbuf2;
+    const int s0 = is_s * kSliceBytes;  // uniform: the loads' scalar offset
+    if constexpr (i < kCg) {
+      if constexpr (kWhole) {
+        copy16_lds(rdoc[i], &dst[i * 256 + wave * 64], dvoff + copy_off, s0);
+      } else {
+        // A unit past the row end is pushed out of range with all low 31 bits set
+        // (branch-free: a select here became divergent branches around the loads).
+        const int past = -(int)(s0 + copy_off >= rowbytes) & 0x7fffffff;
+        copy16_lds(rdoc[i], &dst[i * 256 + wave * 64], (dvoff + s0 + copy_off) | past, 0);
       }
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int m = 0; m < kPairs; ++m)
-          qf[kSet][q][m] = __builtin_bit_cast(
-              u32x4, __builtin_amdgcn_raw_buffer_load_b128(rq[q], r32 * rowbytes + (2 * m + h) * 16,
-                                                           so, 0));
     } else {
-      const int so = is_s * kSliceBytes + copy_off;
-      const int dpast = -(int)(so >= rowbytes) & 0x7fffffff;
-#pragma unroll
-      for (int c = 0; c < kCg; ++c) {
-        const int row = (is_g * kCg + c) * kTile + crow;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rdoc, (lds_void_t)&dbuf[kSet][c * 256 + wave * 64], 16, (row * rowbytes + so) | dpast,
-            0, 0, 0);
+      constexpr int q = (i - kCg) / kPairs, m = (i - kCg) % kPairs;
+      if constexpr (kWhole) {
+        qf[kSet][q][m] = load16_at(rq[q], qvoff + m * 32, s0);
+      } else {
+        const int past = -(int)(s0 + (2 * m + h) * 16 >= rowbytes) & 0x7fffffff;
+        qf[kSet][q][m] = load16_at(rq[q], (qvoff + s0 + m * 32) | past, 0);
       }
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int m = 0; m < kPairs; ++m) {
-          const int o = is_s * kSliceBytes + (2 * m + h) * 16;
-          const int qpast = -(int)(o >= rowbytes) & 0x7fffffff;
-          qf[kSet][q][m] = buf_load16(rq[q], (r32 * rowbytes + o) | qpast);
-        }
     }
-    if (++is_s == nslices) {
-      is_s = 0;
-      if (++is_g == ngroups) {
-        is_g = 0;
-        is_slot = next_slot(is_slot + G);
-        set_issue_item();
-      }
+  };
+  auto advance = [&]() {
+    if (++is_s < nslices) return;
+    is_s = 0;
+    is_e += kCg;
+    if (is_e < is_end) {
+      set_issue_group();
+    } else {
+      is_slot = next_slot(is_slot + G);
+      set_issue_item();
     }
   };
 
   // ---- the compute side -----------------------------------------------------------
-  int c_slot = next_slot(blockIdx.x), c_g = 0, c_s = 0;
-  int j = 0;
-  Rows R{};
+  int c_slot = next_slot(blockIdx.x), c_e = 0, c_end = 0, c_s = 0;
+  Rows Rw{};
   auto set_compute_item = [&]() {
     int qg = 0;
-    j = c_slot < A.nslots ? split_slot_doc(c_slot, nqg, ndx, qg) : 0;
-    R = rows_of(qg);
+    c_e = c_end = 0;
+    if (c_slot < A.nslots) {
+      const int r = split_slot(c_slot, nqg, R, xq, qg);
+      c_e = crs[r];
+      c_end = crs[r + 1];
+    }
+    Rw = rows_of(qg);
   };
   set_compute_item();
-  float mx[2] = {-INFINITY, -INFINITY};
-  int slot[2] = {-1, -1};
+  if (c_slot >= A.nslots) return;
+  int64_t ntasks = 0;  // (items x groups x slices can pass 2^31 at extreme shapes)
+  for (int x = c_slot; x < A.nslots; x = next_slot(x + G)) {
+    int qg;
+    const int r = split_slot(x, nqg, R, xq, qg);
+    ntasks += (int64_t)((crs[r + 1] - crs[r] + kCg - 1) / kCg) * nslices;
+  }
 
-  // Close the item's document for both query rows: wave halves merged, tape
-  // row and score written straight to global memory.  Both rows' running
-  // max starts again for the block's next item, a row past the last query
-  // (whose folds saw zeros) included.
-  auto close_item = [&]() {
+  // Running max of both rows.  With a tape: (max, slot) as the scans keep them.
+  // Without: the max alone, the score of the document's first valid row (which
+  // stands when it is NaN, see take_first_row) and whether there was one.
+  float mx[2] = {-INFINITY, -INFINITY}, first[2] = {-INFINITY, -INFINITY};
+  int slot[2] = {-1, -1};
+  bool any = false;
+
+  // Close document j for both query rows: wave halves merged, tape row and
+  // score written straight to global memory.  Both rows' running max starts
+  // again, a row past the last query (whose folds saw zeros) included.
+  auto close_doc = [&](int j) {
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-      if (R.qv[q] < 0) {
-        mx[q] = -INFINITY;
-        slot[q] = -1;
-        continue;
-      }
-      const uint32_t qw = qmask[R.qv[q]];
-      const bool tv = ((qw >> r32) & 1u) != 0u;
-      int tok = slot_to_token(slot[q], h);
-      float m = mx[q];
-      merge_halves(m, tok, h);
-      const float part = (tv && tok != 0) ? m : 0.0f;
-      const int64_t p = (int64_t)R.qi[q] * Bd + j;
-      if (A.args && h == 0 && r32 < R.qtn[q]) A.args[p * Tq + R.qt0[q] + r32] = tv ? tok : 0;
-      const float score = half_sum(part);
-      if (ntq > 1) {
-        if (lane == 0) A.St[(int64_t)R.qv[q] * Bd + j] = score;
-      } else {
+      if (Rw.qv[q] >= 0) {
+        const uint32_t qw = qmask[Rw.qv[q]];
+        const bool tv = ((qw >> r32) & 1u) != 0u;
+        const int64_t p = (int64_t)Rw.qi[q] * Bd + j;
+        float part;
+        if constexpr (kTape) {
+          int tok = slot_to_token(slot[q], h);
+          float m = mx[q];
+          merge_halves(m, tok, h);
+          part = (tv && tok != 0) ? m : 0.0f;
+          store_below(A.args + p * Tq + Rw.qt0[q], Rw.qtn[q], lane, (uint32_t)(tv ? tok : 0));
+        } else {
+          const float m = merge_halves_max(mx[q]);
+          const uint32_t nf = is_nan_bits(first[q]) ? 1u : 0u;
+          const bool nan_first = (nf | lane_xor32(nf, h)) != 0u;
+          part = tv && any ? (nan_first ? __builtin_bit_cast(float, 0x7fc00000u) : m) : 0.0f;
+        }
+        const float score = half_sum(part);
         const float nf = (float)__builtin_popcount(qw);
         const float inv = 1.0f / (nf > 1.0f ? nf : 1.0f);
-        if (lane == 0) A.S[p] = A.norm ? score * inv : score;
+        const float sc = A.norm && ntq == 1 ? score * inv : score;
+        const float* const out = ntq > 1 ? A.St + ((int64_t)Rw.qv[q] * Bd + j) : A.S + p;
+        store_below(out, 1, lane, __builtin_bit_cast(uint32_t, sc));
       }
       mx[q] = -INFINITY;
+      first[q] = -INFINITY;
       slot[q] = -1;
+    }
+    any = false;
+  };
+
+  // Fold one chunk's scores of query row q (valid rows m32, chunk ch).
+  auto fold = [&](float (&s)[16], uint32_t m32, int ch, int q) {
+    if constexpr (kTape) {
+      take_first_row(s, m32, h, ch, mx[q], slot[q]);
+      if (m32 == 0xffffffffu) fold_tree<true>(s, ch * 16, mx[q], slot[q]);
+      else update_chunk(s, m32, h, ch, mx[q], slot[q]);
+    } else {
+      if (!any) {  // (m32 != 0)
+        const int row = __builtin_ctz(m32);
+        const int reg = ((row >> 3) << 2) | (row & 3);
+        f32x16 sv;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sv[r] = s[r];
+        const float v = sv[reg];
+        first[q] = h == ((row >> 2) & 1) ? v : -INFINITY;
+      }
+      if (m32 != 0xffffffffu) {
+        const uint32_t bits = m32 >> (4 * h);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = ((bits >> acc_row(r, 0)) & 1u) ? s[r] : -INFINITY;
+      }
+      fold_max(s, mx[q]);
     }
   };
 
-  if (ngroups == 0) {  // Td = 0: every pair scores 0 with an all-zero tape
-    for (; c_slot < A.nslots; c_slot = next_slot(c_slot + G)) {
-      set_compute_item();
-      close_item();
-    }
-    return;
-  }
-
-  int64_t ntasks = 0;  // (items x groups x slices can pass 2^31 at extreme shapes)
-  for (int x = c_slot; x < A.nslots; x = next_slot(x + G)) ntasks += (int64_t)ngroups * nslices;
-  if (ntasks == 0) return;
-
   Acc acc[kCg][2];
-  uint32_t gmask[kCg];  // the group's chunk words (scalar loads at its first slice)
+  u32x4 a[2][kCg];  // document fragments of two unit pairs
+  auto read_pair = [&](auto SETc, int m, int c, u32x4& dst) {
+    constexpr int kSet = decltype(SETc)::value;
+    const u32x4* const B = kSet == 0 ? dbuf0 : kSet == 1 ? dbuf1 : dbuf2;
+    dst = B[c * 256 + roff[m]];
+  };
 
-  // Task p: wait for its copies (exactly kAfterCopies vector operations were
-  // issued after them: its own query loads and the whole of task p + 1), a
-  // barrier makes every wave's share visible and frees the stage task p - 1
-  // read, task p + 2 is requested into that stage and query set, and task p
-  // is multiplied; after a group's last slice the group folds, after an
-  // item's last group the item closes.  Chunks past the document read zeros:
-  // their MFMAs run unguarded and their accumulators are never folded.
+  // Task p.  On entry its slice is in LDS and its pair 0 fragments are in a[0].
+  // Pair m's MFMAs run while pair m + 1's fragments are read; task p + 2's loads
+  // go out one by one between the first MFMAs; before pair 3's, the wait and
+  // barrier for task p + 1's slice (exactly kAfterCopies vector operations were
+  // issued after its copies: its own query loads and the whole of task p + 2),
+  // then task p + 1's pair 0 fragments are read.  Each unit (a fragment read, a
+  // load, the MFMAs of one chunk) is fenced: the compiler otherwise puts every
+  // read right before its MFMAs and all loads ahead of them.
   auto step = [&](auto SETc) {
     constexpr int kSet = decltype(SETc)::value;
-    slice_barrier<kAfterCopies>();
-    issue(std::integral_constant<int, (kSet + 2) % kStages>());
-    if (c_s == 0) {
+    typedef std::integral_constant<int, (kSet + 1) % kStages> NextSet;
+    typedef std::integral_constant<int, (kSet + 2) % kStages> IssueSet;
+    constexpr int kOps = Shape::kOpsPerSlice;
+    auto pair_mma = [&](auto Mc, auto FIRSTc) {
+      constexpr int m = decltype(Mc)::value;
+      constexpr bool kZero = decltype(FIRSTc)::value;
+      static_for<0, kCg>([&](auto Cc) {
+        constexpr int c = decltype(Cc)::value;
+        if constexpr (m + 1 < kPairs) read_pair(SETc, m + 1, c, a[(m + 1) & 1][c]);
+        else read_pair(NextSet(), 0, c, a[0][c]);
+        // loads of task p + 2: spread over pairs 0 .. kPairs - 2
+        constexpr int units = kCg * (kPairs - 1), u = m * kCg + c;
+        if constexpr (m < kPairs - 1)
+          static_for<u * kOps / units, (u + 1) * kOps / units>(
+              [&](auto Ic) { issue_one(IssueSet(), Ic); });
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int c = 0; c < kCg; ++c) {
-        const int ch = std::min(c_g * kCg + c, nch - 1);
-        gmask[c] = cmask[(int64_t)j * nch + ch];
-      }
-    }
-    // Document fragments of unit pair m + 1 are read while pair m's MFMAs run
-    // (two register sets); a group's first slice starts its accumulators.
+        for (int q = 0; q < 2; ++q)
+          acc[c][q] = mma_pair<Op>(a[m & 1][c], qf[kSet][q][m], kZero ? Acc{} : acc[c][q]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+    };
+    static_assert(kPairs == 4, "pair 3 reads into the fragment set pair 0 used");
     auto multiply = [&](auto FIRSTc) {
-      constexpr bool kFirst = decltype(FIRSTc)::value;
-      const u32x4* B = &dbuf[kSet][0];
-      u32x4 a[2][kCg];
-#pragma unroll
-      for (int c = 0; c < kCg; ++c) a[0][c] = B[c * 256 + roff[0]];
-#pragma unroll
-      for (int m = 0; m < kPairs; ++m) {
-        if (m + 1 < kPairs) {
-#pragma unroll
-          for (int c = 0; c < kCg; ++c) a[(m + 1) & 1][c] = B[c * 256 + roff[m + 1]];
-        }
-#pragma unroll
-        for (int c = 0; c < kCg; ++c)
-#pragma unroll
-          for (int q = 0; q < 2; ++q)
-            acc[c][q] = mma_pair<Op>(a[m & 1][c], qf[kSet][q][m],
-                                     (kFirst && m == 0) ? Acc{} : acc[c][q]);
-      }
-      // Schedule: the first pair's reads, then per chunk of each pair one read
-      // of the next pair and the chunk's MFMAs (the compiler otherwise puts
-      // every read right before its MFMAs and waits for it there).
-      __builtin_amdgcn_sched_group_barrier(0x100, kCg, 0);
-#pragma unroll
-      for (int m = 0; m < kPairs; ++m)
-#pragma unroll
-        for (int c = 0; c < kCg; ++c) {
-          if (m + 1 < kPairs) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x008, 2 * kMmaPerPair, 0);
-        }
+      pair_mma(std::integral_constant<int, 0>(), FIRSTc);
+      pair_mma(std::integral_constant<int, 1>(), std::false_type());
+      pair_mma(std::integral_constant<int, 2>(), std::false_type());
+      slice_barrier<kAfterCopies>();
+      pair_mma(std::integral_constant<int, 3>(), std::false_type());
     };
     if (c_s == 0) multiply(std::true_type());
     else multiply(std::false_type());
+    advance();
 
     if (++c_s == nslices) {
       c_s = 0;
-      // fold the group's chunks in document order
 #pragma unroll
       for (int c = 0; c < kCg; ++c) {
-        const int ch = c_g * kCg + c;
-        if (ch >= nch) continue;
-        const uint32_t m32 = gmask[c];
+        if (c_e + c >= c_end) continue;
+        const int64_t e = c_e + c;
+        const uint32_t m32 = clist[e * 4], j = clist[e * 4 + 1], ci = clist[e * 4 + 2];
+        if (m32 != 0u) {
+          const int ch = (int)(ci & 0x7fffffffu);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          float s[16];
+          for (int q = 0; q < 2; ++q) {
+            float s[16];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) s[r] = acc[c][q][r];
-          take_first_row(s, m32, h, ch, mx[q], slot[q]);
-          if (m32 == 0xffffffffu)
-            fold_tree<true>(s, ch * 16, mx[q], slot[q]);
-          else
-            update_chunk(s, m32, h, ch, mx[q], slot[q]);
+            for (int r = 0; r < 16; ++r) s[r] = acc[c][q][r];
+            fold(s, m32, ch, q);
+          }
+          any = true;
         }
+        if (ci >> 31) close_doc((int)j);
       }
-      if (++c_g == ngroups) {
-        c_g = 0;
-        close_item();
+      c_e += kCg;
+      if (c_e >= c_end) {
         c_slot = next_slot(c_slot + G);
         set_compute_item();
       }
     }
   };
 
-  issue(std::integral_constant<int, 0>());
-  issue(std::integral_constant<int, 1>());
-  // Whole rounds of three steps, then the one or two tasks left: no branch
-  // around a step inside a round, so the compiler's wait counts see every
-  // step's loads (a skip edge made it drain the loads of later tasks).
-  static_assert(kStages == 3, "the task loop below is unrolled by three");
-  int64_t p = 0;
-  for (; p + kStages <= ntasks; p += kStages) {
+  // The first two tasks' loads, then the steps (past the block's last task the
+  // loads are empty).  The only branches between steps leave the loop: none
+  // skips a step.
+  auto issue_all = [&](auto SETc) {
+    static_for<0, Shape::kOpsPerSlice>([&](auto Ic) {
+      issue_one(SETc, Ic);
+      __builtin_amdgcn_sched_barrier(0);  // in this order: the waits count them
+    });
+  };
+  issue_all(std::integral_constant<int, 0>());
+  advance();
+  issue_all(std::integral_constant<int, 1>());
+  advance();
+  slice_barrier<kAfterCopies>();
+#pragma unroll
+  for (int c = 0; c < kCg; ++c) read_pair(std::integral_constant<int, 0>(), 0, c, a[0][c]);
+  for (int64_t p = 0;;) {
     step(std::integral_constant<int, 0>());
+    if (++p == ntasks) break;
     step(std::integral_constant<int, 1>());
+    if (++p == ntasks) break;
     step(std::integral_constant<int, 2>());
+    if (++p == ntasks) break;
   }
-  if (p < ntasks) step(std::integral_constant<int, 0>());
-  if (p + 1 < ntasks) step(std::integral_constant<int, 1>());
   slice_barrier<0>();  // the empty requests past the last task
 }
 
@@ -512,12 +656,13 @@ bool inbatch_split_supported(int esz, int64_t dim, int64_t Tq, int64_t Td, int64
   const int64_t rowbytes = dim * esz;
   const int64_t ntq = Tq > kTile ? (Tq + kTile - 1) / kTile : 1;
   const int64_t nqg = (Bq * ntq + kRows - 1) / kRows, ndx = (Bd + kSpXcds - 1) / kSpXcds;
-  // 32-bit buffer offsets: a document's rows, a query tile's rows, the slot count
+  // 32-bit buffer offsets: a chunk's rows, a query tile's rows; 32-bit counts:
+  // the chunk list, the slots (ranges are at most as many as documents)
   const int64_t lim = ((int64_t)1 << 31) - 4096;
   return (esz == 2 || esz == 4) && dim > 0 && rowbytes % 16 == 0 && al && Tq >= 1 && Td >= 0 &&
          Bq >= 1 && Bd >= 1 && Bq * ntq <= ((int64_t)1 << 30) && Bd <= ((int64_t)1 << 26) &&
          (Td + kTile * kMaxCg) * rowbytes < lim && kTile * rowbytes < lim &&
-         nqg <= lim / kSpXcds / ndx;
+         Bd * ((Td + kTile - 1) / kTile + 1) < lim && nqg <= lim / kSpXcds / ndx;
 }
 
 namespace {
@@ -538,6 +683,42 @@ int device_cus() {
   return n;
 }
 
+// How the items are cut and dealt: R ranges of the chunk list, and xq (see
+// split_slot).  The pair that makes the longest sequence of items on one block
+// shortest, taking every document as its nch chunks (an item counts its chunk
+// groups and half a group more), and more where an XCD would draw on the memory
+// behind its L2 faster than it delivers: per K slice, the chunks of the ranges
+// that it holds together and the rows of its query groups.
+struct SplitCut {
+  int R, xq;
+};
+SplitCut split_cut(int nqg, int Bd, int nch, int xcd_blocks, int cg, bool f32) {
+  constexpr double kXcdBytesPerUs = 0.7e6;                // memory bandwidth share of an XCD
+  const double slice_us = f32 ? 6.1 : 0.77;               // a block's MFMAs per slice at 2 GHz
+  const int docch = std::max(nch, 1);
+  SplitCut best{1, 8};
+  double best_cost = 0.0;
+  for (int xq = 1; xq <= kSpXcds; xq *= 2) {
+    const int xr = kSpXcds / xq, nqx = (nqg + xq - 1) / xq;
+    const int rmax = std::min(Bd, xr * xcd_blocks * 2);
+    for (int R = 1; R <= rmax; ++R) {
+      const int nrx = (R + xr - 1) / xr;
+      const int64_t passes = ((int64_t)nqx * nrx + xcd_blocks - 1) / xcd_blocks;
+      const int64_t groups = ((int64_t)((Bd + R - 1) / R) * docch + cg - 1) / cg;
+      const int held_r = std::min(nrx, xcd_blocks);
+      const int held_q = std::min(nqx, std::max(1, xcd_blocks / nrx));
+      const double bytes = (double)(held_r * cg + held_q * kRows) * kTile * kSliceBytes;
+      const double cost = (double)passes * ((double)groups + 0.5) *
+                          std::max(1.0, bytes / slice_us / kXcdBytesPerUs) * (1.0 + 1e-9 * bytes);
+      if (best_cost == 0.0 || cost < best_cost) {
+        best = SplitCut{R, xq};
+        best_cost = cost;
+      }
+    }
+  }
+  return best;
+}
+
 }  // namespace
 
 hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
@@ -545,44 +726,61 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   InBatchSplitArgs A = args_in;
   A.ntq = A.Tq > kTile ? (A.Tq + kTile - 1) / kTile : 1;
   A.nqg = (int)(((int64_t)A.Bq * A.ntq + kRows - 1) / kRows);
-  const int ndx = (A.Bd + kSpXcds - 1) / kSpXcds;
-  A.nslots = A.nqg * ndx * kSpXcds;
-  // One workspace: the plan words (documents' chunk words, then query rows'
-  // words), then, with several tiles per query, the tile scores St.
-  const int nch = A.Td > 0 ? (A.Td + kTile - 1) / kTile : 0;
-  const int64_t nwords = (int64_t)A.Bd * nch + (int64_t)A.Bq * A.ntq;
-  const size_t plan_bytes = ((size_t)nwords * sizeof(uint32_t) + 255) / 256 * 256;
-  const size_t st_bytes = A.ntq > 1 ? (size_t)A.Bq * A.ntq * A.Bd * sizeof(float) : 0;
-  void* ws = nullptr;
-  hipError_t e = workspace_alloc(&ws, plan_bytes + st_bytes, stream);
-  if (e != hipSuccess) return e;
-  A.plan = static_cast<uint32_t*>(ws);
-  if (A.ntq > 1) A.St = reinterpret_cast<float*>(static_cast<char*>(ws) + plan_bytes);
-  hipLaunchKernelGGL(split_plan_kernel, dim3((unsigned)std::min<int64_t>((nwords + 7) / 8, 1024)),
-                     dim3(256), 0, stream, A.dm, A.qm, A.Bd, A.Td, nch, A.Bq, A.Tq, A.ntq,
-                     static_cast<uint32_t*>(ws));
-  e = hipGetLastError();
-  // kBlocks blocks per CU (CUs a multiple of 8, so slot x stays on XCD
-  // x % 8), each walking its slots.
+  // kBlocks blocks per CU (CUs a multiple of 8, so slot x stays on XCD x % 8).
   const int cus = std::max(kSpXcds, device_cus() / kSpXcds * kSpXcds);
   const int per_cu = dtype == 0 ? SplitShape<4>::kBlocks : SplitShape<2>::kBlocks;
+  const int cg = dtype == 0 ? SplitShape<4>::kCg : SplitShape<2>::kCg;
+  const int nch = A.Td > 0 ? (A.Td + kTile - 1) / kTile : 0;
+  const SplitCut cut = split_cut(A.nqg, A.Bd, nch, cus * per_cu / kSpXcds, cg, dtype == 0);
+  A.R = cut.R;
+  A.xq = cut.xq;
+  const int xr = kSpXcds / A.xq;
+  A.nslots = kSpXcds * ((A.nqg + A.xq - 1) / A.xq) * ((A.R + xr - 1) / xr);
+  // Ranges of few documents are cut by their number: cut by chunks, one of them
+  // could hold two long documents and its neighbour none.
+  const int by_docs = A.Bd < 4 * A.R ? 1 : 0;
+  // One workspace: the plan words (documents' chunk words, then query rows'
+  // words), the chunk list, the ranges, then, with several tiles per query, the
+  // tile scores St.
+  const int64_t ndw = (int64_t)A.Bd * nch, nwords = ndw + (int64_t)A.Bq * A.ntq;
+  auto al = [](size_t v) { return (v + 255) / 256 * 256; };
+  const size_t plan_bytes = al((size_t)nwords * sizeof(uint32_t));
+  const size_t list_bytes = al((size_t)A.Bd * std::max(nch, 1) * sizeof(uint4));
+  const size_t rs_bytes = al((size_t)(A.R + 1 + kSpXcds) * sizeof(int32_t));  // (slots past R look there)
+  const size_t st_bytes = A.ntq > 1 ? (size_t)A.Bq * A.ntq * A.Bd * sizeof(float) : 0;
+  void* ws = nullptr;
+  hipError_t e = workspace_alloc(&ws, plan_bytes + list_bytes + rs_bytes + st_bytes, stream);
+  if (e != hipSuccess) return e;
+  uint32_t* const plan = static_cast<uint32_t*>(ws);
+  uint4* const list = reinterpret_cast<uint4*>(static_cast<char*>(ws) + plan_bytes);
+  int32_t* const rs = reinterpret_cast<int32_t*>(static_cast<char*>(ws) + plan_bytes + list_bytes);
+  A.qwords = plan + ndw;
+  A.list = list;
+  A.rs = rs;
+  if (A.ntq > 1)
+    A.St = reinterpret_cast<float*>(static_cast<char*>(ws) + plan_bytes + list_bytes + rs_bytes);
+  hipLaunchKernelGGL(split_plan_kernel, dim3((unsigned)std::min<int64_t>((nwords + 7) / 8, 1024)),
+                     dim3(256), 0, stream, A.dm, A.qm, A.Bd, A.Td, nch, A.Bq, A.Tq, A.ntq, plan);
+  hipLaunchKernelGGL(split_list_kernel, dim3(1), dim3(kListThreads), 0, stream, plan, A.Bd, nch, A.R,
+                     by_docs, list, rs);
+  e = hipGetLastError();
   const dim3 grid((unsigned)std::min(A.nslots, cus * per_cu)), block(64 * kSpWaves);
   if (e == hipSuccess) {
-    const bool whole = A.rowbytes % kSliceBytes == 0;
-    switch (dtype) {
-      case 1:
-        if (whole) hipLaunchKernelGGL((inbatch_split<OpF16, true>), grid, block, 0, stream, A);
-        else hipLaunchKernelGGL((inbatch_split<OpF16, false>), grid, block, 0, stream, A);
-        break;
-      case 2:
-        if (whole) hipLaunchKernelGGL((inbatch_split<OpBF16, true>), grid, block, 0, stream, A);
-        else hipLaunchKernelGGL((inbatch_split<OpBF16, false>), grid, block, 0, stream, A);
-        break;
-      default:
-        if (whole) hipLaunchKernelGGL((inbatch_split<OpF32, true>), grid, block, 0, stream, A);
-        else hipLaunchKernelGGL((inbatch_split<OpF32, false>), grid, block, 0, stream, A);
-        break;
-    }
+    auto go = [&](auto op, auto whole, auto tape) {
+      hipLaunchKernelGGL((inbatch_split<decltype(op), decltype(whole)::value, decltype(tape)::value>), grid,
+                         block, 0, stream, A);
+    };
+    auto by_tape = [&](auto op, auto whole) {
+      if (A.args) go(op, whole, std::true_type());
+      else go(op, whole, std::false_type());
+    };
+    auto by_whole = [&](auto op) {
+      if (A.rowbytes % kSliceBytes == 0) by_tape(op, std::true_type());
+      else by_tape(op, std::false_type());
+    };
+    if (dtype == 1) by_whole(OpF16());
+    else if (dtype == 2) by_whole(OpBF16());
+    else by_whole(OpF32());
     e = hipGetLastError();
   }
   if (e == hipSuccess && A.ntq > 1) {

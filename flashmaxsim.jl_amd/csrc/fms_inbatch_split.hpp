@@ -20,13 +20,16 @@ struct InBatchSplitArgs {
   int norm = 0;
   // filled by the launcher: query rows are 32-token tiles, ntq per query
   // (scored into St (Bq * ntq, Bd) and summed into S when ntq > 1); nqg
-  // groups of 8 query rows per document
+  // groups of 8 query rows
   int ntq = 1, nqg = 1;
   float* St = nullptr;
-  // filled by the launcher: the plan words (valid rows of every 32-row
-  // document chunk, then valid tokens of every query row) and the number of
-  // block-order slots (nqg x 8 x ceil(Bd / 8), some past Bd)
-  const uint32_t* plan = nullptr;
+  // filled by the launcher: valid tokens of every query row, the list of
+  // document chunks (see split_list_kernel), the first entry of each of its R
+  // ranges, and the number of block-order slots (see split_slot)
+  const uint32_t* qwords = nullptr;
+  const uint4* list = nullptr;
+  const int32_t* rs = nullptr;
+  int R = 1, xq = 8;
   int nslots = 0;
 };
 
