@@ -56,6 +56,9 @@ hipError_t launch_runs(const RunArgs& A, hipStream_t stream) {
   constexpr int b = (Op::kKb == 16) ? 4 : 2;
   const int nkb = fast_nkb<Op>(A.nkb);
   if (nkb == b) return launch_nkb<Op, b>(A, stream);
+  if constexpr (Op::kKb == 16) {
+    if (nkb == 6) return launch_nkb<Op, 6>(A, stream);
+  }
   if (nkb == 2 * b) return launch_nkb<Op, 2 * b>(A, stream);
   if (nkb == 4 * b) return launch_nkb<Op, 4 * b>(A, stream);
   return hipErrorInvalidValue;

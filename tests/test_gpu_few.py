@@ -132,3 +132,23 @@ def test_ragged_layouts_match_the_wave_per_pair_scan(device, dtype, dim):
     S, args = fm.varlen_forward(*fm.pack_pairs(q, d), normalize=True)
     S_b, args_b = fm.varlen_forward(fm.pack_docs(q * rep), many, normalize=True)
     assert _same(S, S_b[: len(dl)]) and torch.equal(args, args_b[: len(dl)])
+
+
+@pytest.mark.parametrize("grouping", ["never", "always"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_d96_matches_padded_rows(device, dtype, grouping):
+    """d = 96 against the same features padded with zeros to d = 128 (the added products are
+    +0), in output order and as document batches, past the sizes of the few-pair scan."""
+    B, C, N, Tq, Td = 5, 130, 40, 37, 70
+    _, G, _, dm = _case(dtype, N, Tq, Td, 96, device)
+    Q, _, qm, _ = _case(dtype, B, Tq, Td, 96, device, seed=1)
+    g = torch.Generator(device=device).manual_seed(2)
+    idx = torch.randint(0, N + 1, (B, C), generator=g, device=device)
+    pad = torch.nn.functional.pad
+    prev = boundary.candidates_grouping(grouping)
+    try:
+        S, a = fm.candidates_forward(Q, G, idx, qm, dm, neg=-7.0)
+        S_p, a_p = fm.candidates_forward(pad(Q, (0, 32)), pad(G, (0, 32)), idx, qm, dm, neg=-7.0)
+    finally:
+        boundary.candidates_grouping(prev)
+    assert torch.equal(S, S_p) and torch.equal(a, a_p)
