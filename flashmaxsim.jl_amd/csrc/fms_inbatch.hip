@@ -89,6 +89,11 @@ constexpr int kIbMaxChunkMasks = 512;            // documents x chunks per block
 constexpr int kIbMaxDocs = 40;                   // documents per block
 constexpr int kIbMaxChunks = 64;                 // chunks per document (Td <= 2048)
 constexpr int kIbMaxList = (kIbMaxChunkMasks + kIbBufs - 1) / kIbBufs * kIbBufs;  // padded stream
+// Query rows packed across queries (kFlat): queries per wave at most, and
+// documents per block (less than kIbMaxDocs: the scores of more queries and the
+// token maxima being summed take LDS of two blocks per CU).
+constexpr int kIbFlatQueries = 8;
+constexpr int kIbFlatDocs = 32;
 constexpr int kIbBlocksPerCu = 2;                // occupancy the launch bounds ask for
 constexpr int kIbBalanceMaxDocs = 6144;          // partition weights fit the result area
 // List entry: chunk (6 bits) | document in block (6) | last chunk of its
@@ -272,9 +277,19 @@ __device__ int block_exclusive_scan_i32(int v, int* total) {
 // is kNkb k-blocks of 1 KB; wave w copies k-block w mod kNkb of every chunk
 // (with fewer k-blocks than waves, two waves copy the same bytes to the same
 // place, so every wave issues the same loads per step).
+// kFlat: the same packing for any Tq (flat_queries): a wave's A.qpw queries
+// are consecutive tokens over its four tiles, with the steps of a query per
+// tile; only the close differs (flat_sums).  Bound by the MFMAs, of which a
+// query per tile spends (32 - Tq) / 32 on padding.  us per call, query per tile ->
+// packed: 512 x 512 documents of 60..180 tokens, bf16, d = 128, scores alone / with
+// the tape: Tq = 16 212 / 253 -> 119 / 140, 20 214 / 252 -> 154 / 181, 25 213 / 254 ->
+// 179 / 212, 40 377 / 448 -> 292 / 341; 64 queries x 10000 packed documents of
+// 570..900 tokens: Tq = 9 2412 -> 1259, 16 2822 -> 1391, 25 2806 -> 2521.
+// (Summed inside the last tile's close, the sums spilled query fragments at
+// d = 128, whose reloads then waited for the chunk loads: Tq = 20 340.)
 // kTape = false: args is null (scores only, as the reference's maxsim keeps
 // them, dispatch.jl:124): the fold keeps the running maximum alone.
-template <class Op, bool kPacked, bool kT24, int kNkb, bool kTape>
+template <class Op, bool kPacked, bool kT24, int kNkb, bool kTape, bool kFlat>
 __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(const InBatchArgs A) {
   typedef typename Op::Acc Acc;
   typedef typename Op::Frag Frag;
@@ -282,6 +297,9 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
   // The in-batch layout streams 16-row units; the packed layouts (long
   // documents, little tail to save) stream whole 32-row document chunks.
   constexpr bool kHalf = !kPacked && !kT24;
+  static_assert(!(kT24 && kFlat), "one query packing");
+  constexpr int kMaxDocs = kFlat ? kIbFlatDocs : kIbMaxDocs;  // documents per block
+  constexpr int kScoreQ = kFlat ? kIbFlatQueries : kIbQpw;    // queries per wave
   constexpr int kIbNkb = kNkb;
   constexpr int kIbRowBytes = kNkb * 32;                                // bytes per token row
   constexpr int kIbFrags = kNkb * 64;                                   // 16-byte fragments per chunk
@@ -292,27 +310,34 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
   __shared__ u32x4 cbuf0[kIbFrags], cbuf1[kIbFrags], cbuf2[kIbFrags];
   __shared__ u32x4 cbuf3[kIbBufs == 4 ? kIbFrags : 1];
   __shared__ uint32_t chunk_mask[kIbMaxChunkMasks];  // valid rows per (doc, chunk)
-  __shared__ int32_t doc_first[kIbMaxDocs];          // plan value: first valid token | flag
+  __shared__ int32_t doc_first[kMaxDocs];          // plan value: first valid token | flag
   __shared__ uint32_t lst_mask[kIbMaxList];          // compacted chunk list
   __shared__ uint32_t lst_info[kIbMaxList];
   __shared__ int32_t lst_row0[kPacked ? kIbMaxList : 1];  // packed: document's first row
   __shared__ uint32_t lst_first[kHalf ? kIbMaxList : 1];  // units: first valid tokens
-  __shared__ int unit_start[kHalf ? kIbMaxDocs + 1 : 1];  // units: a document's first entry unit
-  __shared__ int unit_first[kHalf ? kIbMaxDocs : 1];      //   and its first unit
-  __shared__ int32_t doc_row0[kPacked ? kIbMaxDocs + 1 : 1];
+  __shared__ int unit_start[kHalf ? kMaxDocs + 1 : 1];  // units: a document's first entry unit
+  __shared__ int unit_first[kHalf ? kMaxDocs : 1];      //   and its first unit
+  __shared__ int32_t doc_row0[kPacked ? kMaxDocs + 1 : 1];
   __shared__ int lst_count;
   __shared__ int any_nf;  // some document's first valid row is not finite
-  __shared__ int16_t res_tape[kIbWaves][kIbQpw][kIbMaxDocs][kTile];  // Td <= 2048
+  __shared__ int16_t res_tape[kIbWaves][kIbQpw][kMaxDocs][kTile];  // Td <= 2048
   // Scores per (wave, query tile, document), then (units) 64 sink floats
   // for the branch-free close: lane 31 stores the score, the other lanes
   // store to the sink.  One array, so the compiler can tell the store from
   // the chunk buffers the loads to LDS write (a store through a pointer
   // that may point into either of two arrays made it wait for every load
   // in flight at each close).
-  constexpr int kScoreWords = kIbWaves * kIbQpw * kIbMaxDocs;
-  __shared__ float score_buf[kScoreWords + (kHalf ? 64 : 0)];
-  float (&res_score)[kIbWaves][kIbQpw][kIbMaxDocs] =
-      *reinterpret_cast<float(*)[kIbWaves][kIbQpw][kIbMaxDocs]>(score_buf);
+  constexpr int kScoreWords = kIbWaves * kScoreQ * kMaxDocs;
+  __shared__ float score_buf[kScoreWords + (kHalf || kFlat ? 64 : 0)];
+  float (&res_score)[kIbWaves][kScoreQ][kMaxDocs] =
+      *reinterpret_cast<float(*)[kIbWaves][kScoreQ][kMaxDocs]>(score_buf);
+  // kFlat: token maxima of the documents being closed, per wave, parity of the
+  // entry that closes them and kind of close (0: a split entry's first document,
+  // 1: an entry's last): tiles 0, 1 close entry i's documents in step i, tiles 2,
+  // 3 in step i + 1, at whose end they are summed.  (The sums read up to 47
+  // entries past a query's first token.)
+  constexpr int kTokMax = kIbQpw * kTile;
+  __shared__ float tok_max[kFlat ? kIbWaves * 4 * kTokMax + 48 : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
   const int r32 = lane & 31, h = lane >> 5;
@@ -322,13 +347,17 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
   // fastest, so the nqb blocks of one document range are dispatched together
   // on one XCD and stream the range's chunks through that XCD's L2 at about
   // the same time: HBM delivers each range about once, not once per query
-  // block.  Document range db = (k / nqb) * 8 + XCD (the grid is padded to
-  // whole rows of 8 ranges).
+  // block.  Document range db = (k / nqb) * 8 + XCD where the ranges are a
+  // multiple of 8; otherwise an XCD takes an eighth of the (range, query block)
+  // pairs in order, so that no XCD gets a whole row of ranges more than another
+  // (100 x 100 documents of 80..250 tokens: 7 query blocks x 73 ranges were 70
+  // blocks on some XCDs' 64 slots).
   const int nqb = A.nqb, ndb = A.ndb;
   const int id = blockIdx.x;
   const int xcd = id % kXcds, kx = id / kXcds;
-  const int qb = kx % nqb;
-  const int db = (kx / nqb) * kXcds + xcd;
+  const int eighth = gridDim.x / kXcds;
+  const int item = ndb % kXcds == 0 ? (kx / nqb * kXcds + xcd) * nqb + kx % nqb : xcd * eighth + kx;
+  const int qb = item % nqb, db = item / nqb;
   if (db >= ndb) return;
 
   // ---- this block's documents -------------------------------------------------
@@ -429,7 +458,24 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
     qt0[q] = (qi[q] - qrow[q] * ntq) * kTile;
     qtn[q] = std::min(kTile, Tq - qt0[q]);
   }
-  if constexpr (!kT24) {
+  // kFlat: the wave's queries are consecutive rows of Q (qf0 the first, nflat of
+  // them): tile t, lane r32 holds token 32t + r32 of theirs; the rest read 0.
+  const int qf0 = (qb * kIbWaves + wave) * A.qpw;
+  const int nflat = std::max(0, std::min(A.qpw, A.Bq - qf0));
+  uint32_t vbits = 0u;  // kFlat: bit t = this lane's token of tile t is valid
+  if constexpr (kFlat) {
+    const int64_t tok0 = nflat > 0 ? (int64_t)qf0 * Tq : 0;
+    const rsrc_t rq = make_rsrc(A.Q + tok0 * kIbRowBytes, (uint32_t)(nflat * Tq * kIbRowBytes));
+    const rsrc_t rm = make_rsrc(A.qm ? (const void*)(A.qm + tok0) : (const void*)A.Q,
+                                A.qm ? (uint32_t)(nflat * Tq) : 0u);
+#pragma unroll
+    for (int t = 0; t < kIbQpw; ++t) {
+      const int base = (32 * t + r32) * kIbRowBytes + h * 16;
+#pragma unroll
+      for (int kb = 0; kb < kIbNkb; ++kb) qf[t][kb] = Op::load(rq, base + kb * 32);
+      qmb[t] = buf_load1(rm, 32 * t + r32);
+    }
+  } else if constexpr (!kT24) {
 #pragma unroll
     for (int q = 0; q < kIbQpw; ++q) {
       const bool live = qlive[q];
@@ -459,6 +505,7 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
   }
   const bool has_qm = A.qm != nullptr;
   auto token_valid = [&](int q) {
+    if constexpr (kFlat) return ((vbits >> q) & 1u) != 0u;
     return qlive[q] && r32 < qtn[q] && (!has_qm || qmb[q] != 0u);
   };
   // kT24: the query (0..3 in the wave) and token (0..23) of this lane in tile t,
@@ -486,13 +533,17 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
     for (int k = 0; k < (int)(sizeof(res_tape) / (16 * 64 * kIbWaves)); ++k)
       reinterpret_cast<u32x4*>(&res_tape[0][0][0][0])[tid + k * 64 * kIbWaves] = u32x4{0u, 0u, 0u, 0u};
   }
-  for (int e = tid; e < kIbWaves * kIbQpw * kIbMaxDocs; e += 64 * kIbWaves)
-    (&res_score[0][0][0])[e] = 0.0f;
+  for (int e = tid; e < kScoreWords; e += 64 * kIbWaves) (&res_score[0][0][0])[e] = 0.0f;
+  if constexpr (kFlat) {
+#pragma unroll
+    for (int t = 0; t < kIbQpw; ++t)
+      vbits |= (32 * t + r32 < nflat * Tq && (!has_qm || qmb[t] != 0u)) ? 1u << t : 0u;
+  }
   __syncthreads();  // chunk_mask, doc_first complete
   if (tid < ndoc && dfv >= 0 && ((dfv >> kPlanNfBit) & 1)) any_nf = 1;
   if (tid < ndoc && dfv == kPlanTooLong) {  // packed document longer than max_len: NaN
     for (int w = 0; w < kIbWaves; ++w)
-      for (int q = 0; q < kIbQpw; ++q)
+      for (int q = 0; q < kScoreQ; ++q)
         res_score[w][q][tid] = __builtin_bit_cast(float, 0x7fc00000u);
   }
 
@@ -686,17 +737,73 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
 #pragma unroll
   for (int q = 0; q < kIbQpw; ++q) { mx[q] = -INFINITY; slot[q] = kNoSlot; }
 
-  // Close query q's document jj: merge the wave halves, map a winning
+  // Close query q's (kFlat: tile q's) document jj: merge the wave halves, map a winning
   // substituted row back to the first valid token f, reduce the score,
   // stage tape and score in LDS, reset the running max.  (A document whose
   // scores are all -Inf closes on f with -Inf, as the reference's first-token
   // rule gives; the NaN case of that rule is settled after the loop.)
-  auto close = [&](int q, int jj, int f) {
+  // kFlat: a tile's lanes hold tokens of several queries, so a close leaves its
+  // token maxima in tok_max, and at the end of the step that closes tiles 2 and 3
+  // (close_flat, where the fewest registers are in use) every query is summed:
+  // lanes 8g .. 8g + 7 take query g, 8 tokens at a time, added in the order
+  // half_sum_in_lanes adds a tile's 32 tokens (and tile after tile), so scores
+  // are bit for bit those of a query per tile.  kind: 0 = the first document of
+  // a split entry, 1 = an entry's last document.
+  int fpar = 0;  // parity of the entry whose documents a close belongs to
+  auto flat_sums = [&](int jj, int par, int kind) {
+    const int ln = lane_id_here(), g = ln >> 3, p = ln & 7;
+    const float* const x = &tok_max[(wave * 4 + par * 2 + kind) * kTokMax + std::min(g, A.qpw - 1) * Tq + p];
+    constexpr int kN = 6;  // Tq <= 42 (flat_queries)
+    float v[kN];
+#pragma unroll
+    for (int k = 0; k < kN; ++k) {
+      const float m = x[8 * k];
+      v[k] = p + 8 * k < Tq ? m : 0.0f;
+    }
+#pragma unroll
+    for (int k = 0; k < kN; ++k) v[k] = dpp_add<0xB1>(v[k]);   // lane ^ 1
+#pragma unroll
+    for (int k = 0; k < kN; ++k) v[k] = dpp_add<0x4E>(v[k]);   // lane ^ 2
+#pragma unroll
+    for (int k = 0; k < kN; ++k) v[k] = dpp_add<0x141>(v[k]);  // row_half_mirror: the other quad
+    const float score = ((v[2] + v[3]) + (v[0] + v[1])) + (v[4] + v[5]);
+    score_buf[p == 0 ? (wave * kScoreQ + g) * kMaxDocs + jj : kScoreWords + ln] = score;
+  };
+  // The sums of the documents that entry `inf` closed.
+  auto close_flat = [&](uint32_t inf, int par) {
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kHalf) {
+      if (inf & (1u << kHSplitBit)) flat_sums((int)((inf >> kHDoc0Shift) & kInfoDocMask), par, 0);
+      if (inf & (1u << kHLastBit)) flat_sums((int)((inf >> kHDoc1Shift) & kInfoDocMask), par, 1);
+    } else {
+      if (inf & (1u << kInfoLastBit)) flat_sums((int)((inf >> kInfoDocShift) & kInfoDocMask), par, 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto close = [&](int q, int jj, int f, int kind) {
+    if constexpr (kFlat) {
+      float m;
+      const bool tv = token_valid(q);
+      if constexpr (kTape) {
+        int tok = slot[q] + tok_off();
+        m = mx[q];
+        merge_halves_all(m, tok);
+        tok = tok > f + 1 ? tok : f + 1;  // (as below)
+        res_tape[wave][q][jj][lane_id_here() & 31] = (int16_t)(tv ? tok : 0);
+      } else {
+        m = merge_halves_max(mx[q]);
+      }
+      // (both halves: the same value to the same place)
+      tok_max[(wave * 4 + fpar * 2 + kind) * kTokMax + q * kTile + (lane_id_here() & 31)] = tv ? m : 0.0f;
+      mx[q] = -INFINITY;
+      slot[q] = kNoSlot;
+      return;
+    }
     if constexpr (!kTape) {
       // scores only: the maximum of both halves, summed as below
       const float m = merge_halves_max(mx[q]);
       const float score = half_sum_in_lanes(token_valid(q) ? m : 0.0f);
-      if constexpr (kHalf) score_buf[lane == 31 ? (wave * kIbQpw + q) * kIbMaxDocs + jj : kScoreWords + lane] = score;
+      if constexpr (kHalf) score_buf[lane == 31 ? (wave * kIbQpw + q) * kMaxDocs + jj : kScoreWords + lane] = score;
       else if (lane == 31) res_score[wave][q][jj] = score;
       mx[q] = -INFINITY;
       return;
@@ -717,7 +824,7 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
       // without branches: both halves hold the merged token and store it to
       // the same place; lanes other than 31 store the score to a sink
       res_tape[wave][q][jj][r32] = (int16_t)(tv ? tok : 0);
-      score_buf[lane == 31 ? (wave * kIbQpw + q) * kIbMaxDocs + jj : kScoreWords + lane] = score;
+      score_buf[lane == 31 ? (wave * kIbQpw + q) * kMaxDocs + jj : kScoreWords + lane] = score;
     } else {
       if (h == 0) res_tape[wave][q][jj][r32] = (int16_t)(tv ? tok : 0);
       if (lane == 31) res_score[wave][q][jj] = score;
@@ -739,8 +846,8 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
     if (inf & (1u << kInfoLastBit)) {
       const int jj = (inf >> kInfoDocShift) & kInfoDocMask;
       const int f = (int)((inf >> kInfoFirstShift) & kInfoFirstMask) - 1;
-      close(q0, jj, f);
-      close(q1, jj, f);
+      close(q0, jj, f, 1);
+      close(q1, jj, f, 1);
     }
   };
 
@@ -852,12 +959,14 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
     Acc n0, n1, n2, n3;
     mma_fold_pinned(a, n0, n1, 0, 1, lag2, lag3, 2, 3, (int)(pinfo & 63u) * kTile);
     close_if_last(2, 3, pinfo);
+    if constexpr (kFlat) fpar = i & 1;
     __builtin_amdgcn_s_setprio(2);
     mma_fold_pinned(a, n2, n3, 2, 3, n0, n1, 0, 1, (int)(info & 63u) * kTile);
     close_if_last(0, 1, info);
     __builtin_amdgcn_s_setprio(1);
     lag2 = n2;
     lag3 = n3;
+    if constexpr (kFlat) close_flat(pinfo, (i + 1) & 1);
     prev_info = info;
     cur_info = next_info;
     // Entry i+1's loads were issued before those of entries i+2 .. i+kIbBufs-1,
@@ -882,8 +991,8 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
         const int jj = (int)((inf >> kHDoc0Shift) & kInfoDocMask);
         fold_max8<false>(s0, mx[q0]);
         fold_max8<false>(s1, mx[q1]);
-        close(q0, jj, 0);
-        close(q1, jj, 0);
+        close(q0, jj, 0, 0);
+        close(q1, jj, 0, 0);
         fold_max8<true>(s0, mx[q0]);
         fold_max8<true>(s1, mx[q1]);
       } else {
@@ -896,8 +1005,8 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
       const int f = uniform(doc_first[jj]) & 0xffff;
       fold_tree8<false, true>(s0, (v0 + 1) * 16, mx[q0], slot[q0]);
       fold_tree8<false, true>(s1, (v0 + 1) * 16, mx[q1], slot[q1]);
-      close(q0, jj, f);
-      close(q1, jj, f);
+      close(q0, jj, f, 0);
+      close(q1, jj, f, 0);
       fold_tree8<true, true>(s0, (v1 + 1) * 16 + 16, mx[q0], slot[q0]);
       fold_tree8<true, true>(s1, (v1 + 1) * 16 + 16, mx[q1], slot[q1]);
     } else {
@@ -910,8 +1019,8 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
     if (inf & (1u << kHLastBit)) {
       const int jj = (int)((inf >> kHDoc1Shift) & kInfoDocMask);
       const int f = uniform(doc_first[jj]) & 0xffff;
-      close(q0, jj, f);
-      close(q1, jj, f);
+      close(q0, jj, f, 1);
+      close(q1, jj, f, 1);
     }
   };
   // A phase whose folded entry is split: tiles (qa, qb) x the chunk as two
@@ -940,8 +1049,8 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
       else nb = Op::mma(a[k / 2], qf[qb][k / 2], nb);
       static_for<(kU * k + kM - 1) / kM, (kU * (k + 1) + kM - 1) / kM>([&](auto uc) {
         constexpr int u = decltype(uc)::value;
-        if constexpr (u == 8) close(fa, jj, f);
-        else if constexpr (u == 9) close(fb, jj, f);
+        if constexpr (u == 8) close(fa, jj, f, 0);
+        else if constexpr (u == 9) close(fb, jj, f, 0);
         else if constexpr (!kTape) {
           if constexpr (u < 4) fold_max_piece8<u, false>(xla, s0, mx[fa]);
           else if constexpr (u < 8) fold_max_piece8<u - 4, false>(xlb, s1, mx[fb]);
@@ -986,6 +1095,7 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
     if (pinfo & (1u << kHSplitBit)) phase1(std::true_type());
     else phase1(std::false_type());
     close_units(2, 3, pinfo);
+    if constexpr (kFlat) fpar = i & 1;
     __builtin_amdgcn_s_setprio(2);
     auto phase2 = [&](auto split) {
       if constexpr (!decltype(split)::value) {
@@ -1000,6 +1110,7 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
     __builtin_amdgcn_s_setprio(1);
     lag2 = n2;
     lag3 = n3;
+    if constexpr (kFlat) close_flat(pinfo, (i + 1) & 1);
     prev_info = info;
     cur_info = next_info;
     dma_barrier<(kIbBufs - 2) * kIbKbPerWave>();
@@ -1109,10 +1220,12 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
       if (pinfo & (1u << kHSplitBit)) fold_units(2, 3, lag2, lag3, pinfo, std::true_type());
       else fold_units(2, 3, lag2, lag3, pinfo, std::false_type());
       close_units(2, 3, pinfo);
+      if constexpr (kFlat) close_flat(pinfo, fpar);
     } else {  // tiles 2,3 of the last entry
       fold_close(2, lag2, pinfo);
       fold_close(3, lag3, pinfo);
       close_if_last(2, 3, pinfo);
+      if constexpr (kFlat) close_flat(pinfo, fpar);
     }
   }
 
@@ -1196,7 +1309,11 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
           const bool fix = token_valid(q) && is_nan_bits(s0);
           if (__ballot(fix) == 0ull) continue;
           if (kTape && (fix & (h == 0))) res_tape[wave][q][jj][r32] = (int16_t)(f + 1);
-          if (lane == 0) res_score[wave][q][jj] = __builtin_bit_cast(float, 0x7fc00000u);
+          if constexpr (kFlat) {
+            if (fix) res_score[wave][(q * kTile + r32) / Tq][jj] = __builtin_bit_cast(float, 0x7fc00000u);
+          } else {
+            if (lane == 0) res_score[wave][q][jj] = __builtin_bit_cast(float, 0x7fc00000u);
+          }
         }
       }
     }
@@ -1207,6 +1324,36 @@ __global__ void __launch_bounds__(64 * kIbWaves, kIbBlocksPerCu) inbatch_mfma(co
   // Query row qi's tape for documents j0..j1-1 is ndoc runs of its qtn tokens
   // (one contiguous run of ndoc * Tq int32 when a row is a whole query); its
   // scores are ndoc contiguous floats in A.S (A.St, unnormalised, for tiles).
+  if constexpr (kFlat) {
+    const int n = ndoc * Tq;
+    const uint64_t mg = ((uint64_t)1 << 32) / (uint64_t)Tq + (((uint64_t)1 << 32) % (uint64_t)Tq != 0);
+    for (int g = 0; g < nflat; ++g) {
+      const int64_t p0 = (int64_t)(qf0 + g) * A.Bd + j0;
+      if (kTape && A.args) {
+        int32_t* const out = A.args + p0 * Tq;
+#pragma unroll 4
+        for (int e = lane; e < n; e += 64) {  // (e / Tq as below)
+          const int jj = (int)(((uint64_t)(uint32_t)e * mg) >> 32), row = g * Tq + e - jj * Tq;
+          out[e] = res_tape[wave][row / kTile][jj][row % kTile];
+        }
+      }
+      float inv = 1.0f;
+      if (A.norm) {
+        int c = 0;
+#pragma unroll
+        for (int t = 0; t < kIbQpw; ++t) {
+          const int row = 32 * t + r32;
+          c += __builtin_popcountll(__ballot(h == 0 && row >= g * Tq && row < (g + 1) * Tq && token_valid(t)));
+        }
+        inv = 1.0f / (float)(c > 1 ? c : 1);
+      }
+      if (lane < ndoc) {
+        const float sc = res_score[wave][g][lane];
+        A.S[p0 + lane] = A.norm ? sc * inv : sc;
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int q = 0; q < kIbQpw; ++q) {
     if (!qlive[q]) continue;
@@ -1291,10 +1438,22 @@ __global__ void __launch_bounds__(256) inbatch_tile_sum_kernel(const float* St, 
   }
 }
 
+// Queries of a wave's four tiles (128 rows) when they are packed row after row,
+// 0 where that holds no more than whole tiles do: 4 queries up to Tq = 32 (5 in
+// effect at Tq = 24, which has its own packing), 2 up to 64.  So Tq <= 25 but 24,
+// and 33 .. 42.
+static int flat_queries(int Tq) {
+  if (Tq < 1 || Tq > 64 || Tq == 24) return 0;
+  const int flat = std::min(kIbFlatQueries, kIbQpw * kTile / Tq);
+  return flat > (Tq > kTile ? kIbQpw / 2 : kIbQpw) ? flat : 0;
+}
+
 hipError_t launch_inbatch_mfma(int dtype_bf16, const InBatchArgs& args_in, hipStream_t stream) {
   InBatchArgs A = args_in;
-  A.ntq = A.Tq > kTile ? (A.Tq + kTile - 1) / kTile : 1;
-  A.nqb = (int)(((int64_t)A.Bq * A.ntq + kIbQueries - 1) / kIbQueries);
+  A.qpw = flat_queries(A.Tq);
+  A.ntq = A.qpw == 0 && A.Tq > kTile ? (A.Tq + kTile - 1) / kTile : 1;
+  const int block_rows = A.qpw > 0 ? kIbWaves * A.qpw : kIbQueries;
+  A.nqb = (int)(((int64_t)A.Bq * A.ntq + block_rows - 1) / block_rows);
   // Documents per block: the grid should be a whole number of rounds of the
   // resident block slots (kIbBlocksPerCu per CU) -- a last round that
   // fills only part of the GPU idles the rest -- as few blocks as that
@@ -1307,7 +1466,7 @@ hipError_t launch_inbatch_mfma(int dtype_bf16, const InBatchArgs& args_in, hipSt
     cus = 256;
   const int64_t slots = (int64_t)cus * kIbBlocksPerCu;
   const int nch = A.Td > 0 ? (A.Td + kTile - 1) / kTile : 1;
-  const int db_cap = std::min(kIbMaxDocs, std::max(1, kIbMaxChunkMasks / nch));
+  const int db_cap = std::min(A.qpw > 0 ? kIbFlatDocs : kIbMaxDocs, std::max(1, kIbMaxChunkMasks / nch));
   // With the balanced split (blocks of equal work) one round is enough; the
   // uniform split keeps two, so the dispatcher can even out lengths.
   const int balance = A.Bd <= kIbBalanceMaxDocs ? 1 : 0;
@@ -1330,7 +1489,7 @@ hipError_t launch_inbatch_mfma(int dtype_bf16, const InBatchArgs& args_in, hipSt
   A.db = (int)((A.Bd + ndb - 1) / ndb);  // most documents of a range
   A.dbcap = db_cap;
   A.balance = balance;
-  A.tilt = balance && kIbBlocksPerCu == 2 && (int64_t)A.nqb * ndb == slots && ndb % 2 == 0 ? 1 : 0;
+  A.tilt = balance && kIbBlocksPerCu == 2 && (int64_t)A.nqb * ndb == slots && ndb % kXcds == 0 ? 1 : 0;
 
   // Plan workspace: chunk masks, chunk counts, first tokens.
   auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
@@ -1356,32 +1515,33 @@ hipError_t launch_inbatch_mfma(int dtype_bf16, const InBatchArgs& args_in, hipSt
                        A.dm, A.D, dtype_bf16, rb, A.Bd, A.Td, nch, cmask, dcount, dfirst);
   e = hipGetLastError();
   if (e == hipSuccess) {
-    const dim3 grid((unsigned)(A.nqb * ((A.ndb + kXcds - 1) / kXcds) * kXcds)), block(64 * kIbWaves);
-    // Tq == 24: four queries fill three tiles (kT24)
+    const dim3 grid((unsigned)(((int64_t)A.nqb * A.ndb + kXcds - 1) / kXcds * kXcds)), block(64 * kIbWaves);
+    // Tq == 24: four queries fill three tiles (kT24); A.qpw > 0: kFlat
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, block, 0, stream, A); };
     // args null: the scores-only kernels (running maximum, no argmax)
-    auto by_nkb = [&](auto op, auto packed, auto t24, auto tape) {
+    auto by_nkb = [&](auto op, auto packed, auto t24, auto flat, auto tape) {
       typedef decltype(op) O;
       constexpr bool P = decltype(packed)::value, T = decltype(t24)::value;
-      constexpr bool K = decltype(tape)::value;
+      constexpr bool K = decltype(tape)::value, F = decltype(flat)::value;
       switch (A.dim / 16) {
-        case 2: go(inbatch_mfma<O, P, T, 2, K>); break;
-        case 4: go(inbatch_mfma<O, P, T, 4, K>); break;
-        case 6: go(inbatch_mfma<O, P, T, 6, K>); break;
-        default: go(inbatch_mfma<O, P, T, 8, K>); break;
+        case 2: go(inbatch_mfma<O, P, T, 2, K, F>); break;
+        case 4: go(inbatch_mfma<O, P, T, 4, K, F>); break;
+        case 6: go(inbatch_mfma<O, P, T, 6, K, F>); break;
+        default: go(inbatch_mfma<O, P, T, 8, K, F>); break;
       }
     };
-    auto by_tape = [&](auto op, auto packed, auto t24) {
-      if (A.args) by_nkb(op, packed, t24, std::true_type());
-      else by_nkb(op, packed, t24, std::false_type());
+    auto by_tape = [&](auto op, auto packed, auto t24, auto flat) {
+      if (A.args) by_nkb(op, packed, t24, flat, std::true_type());
+      else by_nkb(op, packed, t24, flat, std::false_type());
     };
-    auto by_t24 = [&](auto op, auto packed) {
-      if (A.Tq == 24) by_tape(op, packed, std::true_type());
-      else by_tape(op, packed, std::false_type());
+    auto by_packing = [&](auto op, auto packed) {
+      if (A.Tq == 24) by_tape(op, packed, std::true_type(), std::false_type());
+      else if (A.qpw > 0) by_tape(op, packed, std::false_type(), std::true_type());
+      else by_tape(op, packed, std::false_type(), std::false_type());
     };
     auto by_packed = [&](auto op) {
-      if (A.cu) by_t24(op, std::true_type());
-      else by_t24(op, std::false_type());
+      if (A.cu) by_packing(op, std::true_type());
+      else by_packing(op, std::false_type());
     };
     if (dtype_bf16) by_packed(OpBF16());
     else by_packed(OpF16());

@@ -24,6 +24,7 @@ struct InBatchArgs {
   int ntq = 1;
   float* St = nullptr;        // S *= 1 / max(valid tokens of query i, 1)
   // filled by the launcher
+  int qpw = 0;         // queries packed into a wave's rows (0: whole tiles per query)
   int nqb, ndb;        // query blocks, document blocks
   int db;              // most documents of a block (uniform partition: ranges of floor or ceil of Bd/ndb)
   int dbcap;           // most documents a block can hold

@@ -1,0 +1,70 @@
+"""Queries packed row after row into a wave's tiles (16-bit in-batch and multi-query
+packed scans) against the same queries padded with masked tokens to whole tiles, which
+takes the kernel with a query per tile: the sums run in the same order, so scores and
+tapes are equal bit for bit.  Lengths at both ends of each count of queries per wave,
+query counts that leave a wave or a block part filled, documents without a valid token,
+documents that share a chunk, and Inf / NaN tokens."""
+import pytest
+import torch
+
+import flashmaxsim as fm
+
+pytestmark = pytest.mark.gpu
+
+
+def _padded(Q, qm):
+    B, Tq, dim = Q.shape
+    T = 32 if Tq <= 32 else 64
+    Qp = torch.zeros(B, T, dim, dtype=Q.dtype, device=Q.device)
+    mp = torch.zeros(B, T, dtype=torch.bool, device=Q.device)
+    Qp[:, :Tq] = Q
+    mp[:, :Tq] = True if qm is None else qm
+    return Qp, mp
+
+
+def _same(x, y):
+    return torch.equal(torch.nan_to_num(x, nan=12345.0), torch.nan_to_num(y, nan=12345.0))
+
+
+def _check(forward, Q, D, qm, *masks):
+    Qp, mp = _padded(Q, qm)
+    for norm in (False, True):
+        S, a = forward(Q, D, qm, *masks, normalize=norm)
+        Sp, ap = forward(Qp, D, mp, *masks, normalize=norm)
+        assert _same(S, Sp) and torch.equal(a, ap[..., :Q.shape[1]])
+        S0, _ = forward(Q, D, qm, *masks, normalize=norm, tape=False)
+        assert _same(S, S0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim", [32, 64, 96, 128])
+@pytest.mark.parametrize("Tq", [1, 8, 9, 15, 16, 17, 18, 19, 21, 22, 23, 25, 33, 42])
+def test_packed_queries_match_a_query_per_tile(device, dtype, dim, Tq):
+    g = torch.Generator(device=device).manual_seed(Tq * 1000 + dim)
+    for Bq, Bd, Td in ((1, 1, 1), (33, 90, 50), (130, 40, 33), (7, 700, 180)):
+        Q = torch.randn(Bq, Tq, dim, generator=g, device=device).to(dtype)
+        D = torch.randn(Bd, Td, dim, generator=g, device=device).to(dtype)
+        qm = torch.rand(Bq, Tq, generator=g, device=device) < 0.8
+        dm = torch.rand(Bd, Td, generator=g, device=device) < 0.6
+        if Bd > 2:
+            dm[0] = dm[Bd - 1] = False
+        _check(fm.inbatch_forward, Q, D, qm, dm)
+        _check(fm.inbatch_forward, Q, D, None, None)
+        lens = torch.randint(0, Td + 1, (Bd,), generator=g, device=device)
+        cu = torch.ones(Bd + 1, dtype=torch.int32, device=device)
+        cu[1:] += lens.cumsum(0).to(torch.int32)
+        P = fm.PackedSeq(D.reshape(-1, dim)[:max(1, int(lens.sum()))].contiguous(), cu, int(max(1, lens.max())))
+        if int(lens.sum()) > 0:
+            _check(fm.packed_multi_forward, Q, P, qm)
+
+
+@pytest.mark.parametrize("Tq", [11, 20, 40])
+def test_non_finite_tokens(device, Tq):
+    g = torch.Generator(device=device).manual_seed(Tq)
+    Q = torch.randn(21, Tq, 64, generator=g, device=device).half()
+    D = torch.randn(50, 70, 64, generator=g, device=device).half()
+    Q[3, Tq - 1, 5], Q[4, 0, 0], Q[20, Tq // 2, 1] = float("nan"), float("inf"), float("-inf")
+    D[7, 0, 2], D[8, 30, 2], D[49, 0] = float("nan"), float("inf"), float("-inf")
+    _check(fm.inbatch_forward, Q, D, None, None)
+    cu = torch.arange(51, dtype=torch.int32, device=device) * 70 + 1
+    _check(fm.packed_multi_forward, Q, fm.PackedSeq(D.reshape(-1, 64), cu, 70), None)
