@@ -279,7 +279,16 @@ __device__ __forceinline__ int split_slot(int x, int nqg, int R, int xq, int& qg
 // kWhole: rows are whole slices (rowbytes a multiple of kSliceBytes, as at
 // d = 768 in 16 bits or d = 128 in fp32), so no unit lies past a row's end
 // and the slice's byte offset goes to the loads' scalar offset.
-template <class Op, bool kWhole, bool kTape>
+// kFlat: the queries' tokens are one run of A.Tq = Bq * qtok tokens (A.Bq = 1), cut
+// into tiles whatever query they belong to, so short queries (and the last tile of
+// long ones) multiply no padding; a close stores each token's maximum (A.St), and
+// split_token_sum_kernel sums the queries.  The launcher says when.  us per call
+// against a query per tile, scores alone / with the tape, documents of Td / 3 .. Td
+// tokens: bf16, d = 256, 512 x 512, Td = 300: 978 / 1179 -> 314 / 379 at 9 query tokens,
+// 659 / 826 at 20, and 40 tokens (two tiles) about 1960 / 2360 -> 1225 / 1502; bf16,
+// d = 768, 200 x 200, Td = 180: 289 / 316 -> 112 / 122 at 9, 177 / 195 at 16; fp32, d = 128,
+// 200 x 200: 386 / 401 -> 174 / 184 at 9, 278 / 292 at 20.
+template <class Op, bool kWhole, bool kTape, bool kFlat>
 __global__ void __launch_bounds__(64 * kSpWaves, SplitShape<Op::kEsz>::kBlocks)
     inbatch_split(const InBatchSplitArgs A) {
   typedef typename Op::Acc Acc;
@@ -319,6 +328,7 @@ __global__ void __launch_bounds__(64 * kSpWaves, SplitShape<Op::kEsz>::kBlocks)
   // Query rows of a wave for query group qg: query, first token, token count.
   struct Rows {
     int qv[2], qi[2], qt0[2], qtn[2];
+    int tq0[2];  // kFlat tape: the first token's query
   };
   auto rows_of = [&](int qg) {
     Rows Rw;
@@ -330,6 +340,7 @@ __global__ void __launch_bounds__(64 * kSpWaves, SplitShape<Op::kEsz>::kBlocks)
       Rw.qi[q] = live ? v / ntq : 0;
       Rw.qt0[q] = live ? (v - Rw.qi[q] * ntq) * kTile : 0;
       Rw.qtn[q] = live ? std::min(kTile, Tq - Rw.qt0[q]) : 0;
+      if constexpr (kFlat && kTape) Rw.tq0[q] = Rw.qt0[q] / A.qtok;
     }
     return Rw;
   };
@@ -468,19 +479,33 @@ __global__ void __launch_bounds__(64 * kSpWaves, SplitShape<Op::kEsz>::kBlocks)
           float m = mx[q];
           merge_halves(m, tok, h);
           part = (tv && tok != 0) ? m : 0.0f;
-          store_below(A.args + p * Tq + Rw.qt0[q], Rw.qtn[q], lane, (uint32_t)(tv ? tok : 0));
+          if constexpr (kFlat) {
+            // (row / qtok by a 16-bit reciprocal, exact below 2^16 / qtok; computed
+            // here, not kept: two more registers a lane made the accumulators move)
+            const int row = r32 + (Rw.qt0[q] - Rw.tq0[q] * A.qtok);
+            const int i = (int)(((uint32_t)row * A.qrecip) >> 16);
+            const int past = -(int)(lane >= Rw.qtn[q]) & 0x1fffffff;
+            store_below(A.args + ((int64_t)Rw.tq0[q] * Bd + j) * A.qtok, (kTile + 1) * Bd * A.qtok,
+                        (i * (Bd - 1) * A.qtok + row) | past, (uint32_t)(tv ? tok : 0));
+          } else
+            store_below(A.args + p * Tq + Rw.qt0[q], Rw.qtn[q], lane, (uint32_t)(tv ? tok : 0));
         } else {
           const float m = merge_halves_max(mx[q]);
           const uint32_t nf = is_nan_bits(first[q]) ? 1u : 0u;
           const bool nan_first = (nf | lane_xor32(nf, h)) != 0u;
           part = tv && any ? (nan_first ? __builtin_bit_cast(float, 0x7fc00000u) : m) : 0.0f;
         }
-        const float score = half_sum(part);
-        const float nf = (float)__builtin_popcount(qw);
-        const float inv = 1.0f / (nf > 1.0f ? nf : 1.0f);
-        const float sc = A.norm && ntq == 1 ? score * inv : score;
-        const float* const out = ntq > 1 ? A.St + ((int64_t)Rw.qv[q] * Bd + j) : A.S + p;
-        store_below(out, 1, lane, __builtin_bit_cast(uint32_t, sc));
+        if constexpr (kFlat) {
+          store_below(A.St + ((int64_t)j * ntq * kTile + Rw.qt0[q]), Rw.qtn[q], lane,
+                      __builtin_bit_cast(uint32_t, part));
+        } else {
+          const float score = half_sum(part);
+          const float nf = (float)__builtin_popcount(qw);
+          const float inv = 1.0f / (nf > 1.0f ? nf : 1.0f);
+          const float sc = A.norm && ntq == 1 ? score * inv : score;
+          const float* const out = ntq > 1 ? A.St + ((int64_t)Rw.qv[q] * Bd + j) : A.S + p;
+          store_below(out, 1, lane, __builtin_bit_cast(uint32_t, sc));
+        }
       }
       mx[q] = -INFINITY;
       first[q] = -INFINITY;
@@ -648,6 +673,47 @@ __global__ void __launch_bounds__(256) split_tile_sum_kernel(const float* St, in
   }
 }
 
+// S[i, j] = the sum of query i's token maxima St[j][i * Tq ..] (rows of nr tokens), a
+// thread per (i, j), added as half_sum adds a tile's 32 tokens and tile after tile,
+// so scores are bit for bit those of a query per tile; normalised as above.
+__global__ void __launch_bounds__(256) split_token_sum_kernel(const float* St, int64_t nr, int Bq, int Bd,
+                                                              const uint8_t* qm, int Tq, int norm,
+                                                              float* S) {
+  const int64_t n = (int64_t)Bq * Bd;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (int64_t)gridDim.x * 256) {
+    const int64_t j = e / Bq;
+    const int i = (int)(e - j * Bq);
+    const float* const x = St + j * nr + (int64_t)i * Tq;
+    float s = 0.0f;
+    for (int t0 = 0; t0 < Tq; t0 += kTile) {
+      float row[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float quad[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          float v[4];
+#pragma unroll
+          for (int l = 0; l < 4; ++l) {
+            const int t = t0 + 16 * h + 4 * k + l;
+            v[l] = t < Tq ? x[t] : 0.0f;
+          }
+          quad[k] = (v[0] + v[1]) + (v[2] + v[3]);
+        }
+        row[h] = (quad[0] + quad[3]) + (quad[2] + quad[1]);
+      }
+      s += row[0] + row[1];
+    }
+    if (norm) {
+      int c = qm ? 0 : Tq;
+      if (qm)
+        for (int t = 0; t < Tq; ++t) c += qm[(int64_t)i * Tq + t] != 0;
+      s *= 1.0f / (float)(c > 1 ? c : 1);
+    }
+    S[(int64_t)i * Bd + j] = s;
+  }
+}
+
 }  // namespace
 
 bool inbatch_split_supported(int esz, int64_t dim, int64_t Tq, int64_t Td, int64_t Bq,
@@ -726,6 +792,26 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   InBatchSplitArgs A = args_in;
   A.ntq = A.Tq > kTile ? (A.Tq + kTile - 1) / kTile : 1;
   A.nqg = (int)(((int64_t)A.Bq * A.ntq + kRows - 1) / kRows);
+  // Tokens in one run (kFlat) where that saves a fifth of the query groups, up to 8
+  // of them counted as the power of two that the XCDs are dealt: less is used up
+  // by the token maxima's way through memory and the sum's launch (fp32, d = 64, 60 x
+  // 60: 8 groups 50 us, as 5 groups of one run 53, as 4 37).  The maxima's array is
+  // bounded, and a tile's tape entries lie within 2^30 bytes.
+  const int Bq = A.Bq, Tq = A.Tq;
+  const int64_t ntok = (int64_t)Bq * Tq, ftiles = (ntok + kTile - 1) / kTile;
+  const int64_t fgroups = (ftiles + kRows - 1) / kRows;
+  auto dealt = [](int64_t n) { return n <= 2 ? n : n <= 4 ? 4 : n <= kSpXcds ? kSpXcds : n; };
+  const bool flat = dealt(fgroups) * 5 <= dealt(A.nqg) * 4 && ntok <= ((int64_t)1 << 30) && (Tq + kTile) * Tq < 65536 &&
+                    ftiles * kTile * A.Bd <= ((int64_t)1 << 26) &&
+                    (int64_t)(kTile + 1) * A.Bd * Tq < ((int64_t)1 << 28);
+  if (flat) {
+    A.qtok = Tq;
+    A.qrecip = (65536u + (unsigned)Tq - 1) / (unsigned)Tq;
+    A.Bq = 1;
+    A.Tq = (int)ntok;
+    A.ntq = (int)ftiles;
+    A.nqg = (int)fgroups;
+  }
   // kBlocks blocks per CU (CUs a multiple of 8, so slot x stays on XCD x % 8).
   const int cus = std::max(kSpXcds, device_cus() / kSpXcds * kSpXcds);
   const int per_cu = dtype == 0 ? SplitShape<4>::kBlocks : SplitShape<2>::kBlocks;
@@ -747,7 +833,7 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   const size_t plan_bytes = al((size_t)nwords * sizeof(uint32_t));
   const size_t list_bytes = al((size_t)A.Bd * std::max(nch, 1) * sizeof(uint4));
   const size_t rs_bytes = al((size_t)(A.R + 1 + kSpXcds) * sizeof(int32_t));  // (slots past R look there)
-  const size_t st_bytes = A.ntq > 1 ? (size_t)A.Bq * A.ntq * A.Bd * sizeof(float) : 0;
+  const size_t st_bytes = A.ntq > 1 ? (size_t)A.Bq * A.ntq * A.Bd * sizeof(float) * (flat ? kTile : 1) : 0;
   void* ws = nullptr;
   hipError_t e = workspace_alloc(&ws, plan_bytes + list_bytes + rs_bytes + st_bytes, stream);
   if (e != hipSuccess) return e;
@@ -766,13 +852,18 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   e = hipGetLastError();
   const dim3 grid((unsigned)std::min(A.nslots, cus * per_cu)), block(64 * kSpWaves);
   if (e == hipSuccess) {
-    auto go = [&](auto op, auto whole, auto tape) {
-      hipLaunchKernelGGL((inbatch_split<decltype(op), decltype(whole)::value, decltype(tape)::value>), grid,
-                         block, 0, stream, A);
+    auto go = [&](auto op, auto whole, auto tape, auto fl) {
+      hipLaunchKernelGGL((inbatch_split<decltype(op), decltype(whole)::value, decltype(tape)::value,
+                                        decltype(fl)::value>),
+                         grid, block, 0, stream, A);
+    };
+    auto by_flat = [&](auto op, auto whole, auto tape) {
+      if (flat) go(op, whole, tape, std::true_type());
+      else go(op, whole, tape, std::false_type());
     };
     auto by_tape = [&](auto op, auto whole) {
-      if (A.args) go(op, whole, std::true_type());
-      else go(op, whole, std::false_type());
+      if (A.args) by_flat(op, whole, std::true_type());
+      else by_flat(op, whole, std::false_type());
     };
     auto by_whole = [&](auto op) {
       if (A.rowbytes % kSliceBytes == 0) by_tape(op, std::true_type());
@@ -783,7 +874,12 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
     else by_whole(OpF32());
     e = hipGetLastError();
   }
-  if (e == hipSuccess && A.ntq > 1) {
+  if (e == hipSuccess && flat) {
+    hipLaunchKernelGGL(split_token_sum_kernel,
+                       dim3((unsigned)std::min<int64_t>(((int64_t)Bq * A.Bd + 255) / 256, 8192)), dim3(256), 0,
+                       stream, A.St, ftiles * kTile, Bq, A.Bd, A.qm, Tq, A.norm, A.S);
+    e = hipGetLastError();
+  } else if (e == hipSuccess && A.ntq > 1) {
     hipLaunchKernelGGL(split_tile_sum_kernel,
                        dim3((unsigned)std::min((A.Bd + 255) / 256, 64),
                             (unsigned)std::min(A.Bq, 65535)),

@@ -23,6 +23,10 @@ struct InBatchSplitArgs {
   // groups of 8 query rows
   int ntq = 1, nqg = 1;
   float* St = nullptr;
+  // filled by the launcher when tiles are cut from all queries' tokens as one run:
+  // tokens of a query (Bq is then 1, Tq all tokens, St token maxima (Bd, 32 * ntq))
+  int qtok = 0;
+  uint32_t qrecip = 0;  // ceil(2^16 / qtok)
   // filled by the launcher: valid tokens of every query row, the list of
   // document chunks (see split_list_kernel), the first entry of each of its R
   // ranges, and the number of block-order slots (see split_slot)

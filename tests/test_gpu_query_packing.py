@@ -1,5 +1,5 @@
 """Queries packed row after row into a wave's tiles (16-bit in-batch and multi-query
-packed scans) against the same queries padded with masked tokens to whole tiles, which
+packed scans), or all queries' tokens cut into tiles (split-K in-batch), against the same queries padded with masked tokens to whole tiles, which
 takes the kernel with a query per tile: the sums run in the same order, so scores and
 tapes are equal bit for bit.  Lengths at both ends of each count of queries per wave,
 query counts that leave a wave or a block part filled, documents without a valid token,
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 def _padded(Q, qm):
     B, Tq, dim = Q.shape
-    T = 32 if Tq <= 32 else 64
+    T = (Tq + 31) // 32 * 32
     Qp = torch.zeros(B, T, dim, dtype=Q.dtype, device=Q.device)
     mp = torch.zeros(B, T, dtype=torch.bool, device=Q.device)
     Qp[:, :Tq] = Q
@@ -58,13 +58,30 @@ def test_packed_queries_match_a_query_per_tile(device, dtype, dim, Tq):
             _check(fm.packed_multi_forward, Q, P, qm)
 
 
+@pytest.mark.parametrize("dtype,dim", [(torch.float16, 256), (torch.bfloat16, 768), (torch.bfloat16, 200),
+                                       (torch.float32, 128), (torch.float32, 36)])
+@pytest.mark.parametrize("Bq,Tq", [(300, 1), (40, 9), (130, 21), (140, 25), (50, 40), (40, 100)])
+def test_split_k_tokens_in_one_run(device, dtype, dim, Bq, Tq):
+    g = torch.Generator(device=device).manual_seed(Tq * 1000 + dim)
+    for Bd, Td in ((1, 1), (37, 70), (200, 200)):
+        Q = torch.randn(Bq, Tq, dim, generator=g, device=device).to(dtype)
+        D = torch.randn(Bd, Td, dim, generator=g, device=device).to(dtype)
+        qm = torch.rand(Bq, Tq, generator=g, device=device) < 0.8
+        dm = torch.rand(Bd, Td, generator=g, device=device) < 0.6
+        if Bd > 2:
+            dm[0] = dm[Bd - 1] = False
+        _check(fm.inbatch_forward, Q, D, qm, dm)
+        _check(fm.inbatch_forward, Q, D, None, None)
+
+
+@pytest.mark.parametrize("dim", [64, 256])
 @pytest.mark.parametrize("Tq", [11, 20, 40])
-def test_non_finite_tokens(device, Tq):
+def test_non_finite_tokens(device, Tq, dim):
     g = torch.Generator(device=device).manual_seed(Tq)
-    Q = torch.randn(21, Tq, 64, generator=g, device=device).half()
-    D = torch.randn(50, 70, 64, generator=g, device=device).half()
+    Q = torch.randn(21, Tq, dim, generator=g, device=device).half()
+    D = torch.randn(50, 70, dim, generator=g, device=device).half()
     Q[3, Tq - 1, 5], Q[4, 0, 0], Q[20, Tq // 2, 1] = float("nan"), float("inf"), float("-inf")
     D[7, 0, 2], D[8, 30, 2], D[49, 0] = float("nan"), float("inf"), float("-inf")
     _check(fm.inbatch_forward, Q, D, None, None)
     cu = torch.arange(51, dtype=torch.int32, device=device) * 70 + 1
-    _check(fm.packed_multi_forward, Q, fm.PackedSeq(D.reshape(-1, 64), cu, 70), None)
+    _check(fm.packed_multi_forward, Q, fm.PackedSeq(D.reshape(-1, dim), cu, 70), None)
