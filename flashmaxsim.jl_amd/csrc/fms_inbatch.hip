@@ -10,7 +10,8 @@
 // valid row and its first valid token.  The in-batch kernel then runs two
 // workgroups per CU (at C3 a single round of the grid):
 //
-// Workgroup = 4 waves (one per SIMD), 16 queries x a range of documents.
+// Workgroup = 4 waves (one per SIMD), 16 queries (more of short ones, whose
+// tokens share tiles: kFlat) x a range of documents.
 //   * document ranges split the documents by work (chunk steps plus one per
 //     document, from the plan), so the workgroups finish together; every
 //     workgroup checks the split against the per-block document limit and

@@ -19,7 +19,7 @@ struct InBatchArgs {
   int Bq, Bd, Tq, Td;
   int dim = 128;       // 32, 64, 96 or 128
   int norm = 0;
-  // filled by the launcher for Tq > 32: query rows of the kernel are tiles of
+  // filled by the launcher for Tq > 32 (where qpw is 0): query rows of the kernel are tiles of
   // 32 tokens, ntq per query, scored into St (Bq * ntq, Bd) and summed into S
   int ntq = 1;
   float* St = nullptr;        // S *= 1 / max(valid tokens of query i, 1)

@@ -12,7 +12,8 @@
 // order (a document without one keeps one chunk, all masked, so that it
 // closes), and cuts the list into R ranges of equal length at document
 // boundaries.  Work item = one range x kRows query rows (a query row is a
-// 32-token tile of a query: query v / ntq, tokens 32 (v % ntq) ..).  Blocks of 4
+// 32-token tile of a query: query v / ntq, tokens 32 (v % ntq) ..; of all queries'
+// tokens as one run where that leaves fewer tiles, kFlat).  Blocks of 4
 // waves, one per CU for 16-bit features and two for fp32, each walk their
 // items in turn (a persistent grid).  An item's chunks are taken kCg at a time
 // whatever documents they belong to (a chunk group: 6 chunks for 16-bit
@@ -795,13 +796,14 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   // Tokens in one run (kFlat) where that saves a fifth of the query groups, up to 8
   // of them counted as the power of two that the XCDs are dealt: less is used up
   // by the token maxima's way through memory and the sum's launch (fp32, d = 64, 60 x
-  // 60: 8 groups 50 us, as 5 groups of one run 53, as 4 37).  The maxima's array is
+  // 60: 8 groups 50 us, as 5 groups of one run 53, as 4 37), and where there is work to
+  // save (bf16, d = 256, 30 x 30: 4 groups 18.8 us, as 2 22.5).  The maxima's array is
   // bounded, and a tile's tape entries lie within 2^30 bytes.
   const int Bq = A.Bq, Tq = A.Tq;
   const int64_t ntok = (int64_t)Bq * Tq, ftiles = (ntok + kTile - 1) / kTile;
   const int64_t fgroups = (ftiles + kRows - 1) / kRows;
   auto dealt = [](int64_t n) { return n <= 2 ? n : n <= 4 ? 4 : n <= kSpXcds ? kSpXcds : n; };
-  const bool flat = dealt(fgroups) * 5 <= dealt(A.nqg) * 4 && ntok <= ((int64_t)1 << 30) && (Tq + kTile) * Tq < 65536 &&
+  const bool flat = dealt(fgroups) * 5 <= dealt(A.nqg) * 4 && (int64_t)A.nqg * A.Bd >= 256 && ntok <= ((int64_t)1 << 30) && (Tq + kTile) * Tq < 65536 &&
                     ftiles * kTile * A.Bd <= ((int64_t)1 << 26) &&
                     (int64_t)(kTile + 1) * A.Bd * Tq < ((int64_t)1 << 28);
   if (flat) {
