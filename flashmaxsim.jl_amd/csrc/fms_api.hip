@@ -756,6 +756,16 @@ int32_t fms_debug_inbatch_kernel(int32_t dtype, int64_t dim, int64_t Tq, int64_t
   return inbatch_path(dtype, dim, Tq, Td, Bq, Bd, Q, D);
 }
 
+fms_status fms_debug_split_rows(int64_t Tq, int64_t Bq, int64_t Bd, int64_t* out) {
+  if (Tq < 1 || Bq < 1 || Bd < 1 || !out) return FMS_EINVAL;
+  const SplitRows r = split_rows(Bq, Tq, Bd);
+  out[0] = r.flat ? 1 : 0;
+  out[1] = r.ntq;
+  out[2] = r.nqg;
+  out[3] = r.stored;
+  return FMS_OK;
+}
+
 fms_status fms_int8_dots(int32_t* out, const int8_t* qc, const int8_t* dc, int64_t dim,
                          int64_t Tq, int64_t Td, void* stream) {
   if (dim < 0 || Tq < 0 || Td < 0) return FMS_EINVAL;

@@ -788,31 +788,44 @@ SplitCut split_cut(int nqg, int Bd, int nch, int xcd_blocks, int cg, bool f32) {
 
 }  // namespace
 
+// Tokens in one run (kFlat) where that saves a fifth of the query groups, up to 8
+// of them counted as the power of two that the XCDs are dealt: less is used up
+// by the token maxima's way through memory and the sum's launch (fp32, d = 64, 60 x
+// 60: 8 groups 50 us, as 5 groups of one run 53, as 4 37), and where there is work to
+// save (bf16, d = 256, 30 x 30: 4 groups 18.8 us, as 2 22.5).  The maxima's array is
+// bounded, and a tile's tape entries lie within 2^30 bytes.
+SplitRows split_rows(int64_t Bq, int64_t Tq, int64_t Bd) {
+  SplitRows r;
+  r.ntq = Tq > kTile ? (Tq + kTile - 1) / kTile : 1;
+  r.nqg = (Bq * r.ntq + kRows - 1) / kRows;
+  const int64_t ntok = Bq * Tq, ftiles = (ntok + kTile - 1) / kTile;
+  const int64_t fgroups = (ftiles + kRows - 1) / kRows;
+  auto dealt = [](int64_t n) { return n <= 2 ? n : n <= 4 ? 4 : n <= kSpXcds ? kSpXcds : n; };
+  r.flat = dealt(fgroups) * 5 <= dealt(r.nqg) * 4 && r.nqg * Bd >= 256 && ntok <= ((int64_t)1 << 30) &&
+           (Tq + kTile) * Tq < 65536 && ftiles * kTile * Bd <= ((int64_t)1 << 26) &&
+           (kTile + 1) * Bd * Tq < ((int64_t)1 << 28);
+  if (r.flat) {
+    r.ntq = ftiles;
+    r.nqg = fgroups;
+  }
+  // One run stores token maxima whatever its tiles (32 tokens in all are one).
+  r.stored = r.flat ? ftiles * kTile * Bd : r.ntq > 1 ? Bq * r.ntq * Bd : 0;
+  return r;
+}
+
 hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
                                 hipStream_t stream) {
   InBatchSplitArgs A = args_in;
-  A.ntq = A.Tq > kTile ? (A.Tq + kTile - 1) / kTile : 1;
-  A.nqg = (int)(((int64_t)A.Bq * A.ntq + kRows - 1) / kRows);
-  // Tokens in one run (kFlat) where that saves a fifth of the query groups, up to 8
-  // of them counted as the power of two that the XCDs are dealt: less is used up
-  // by the token maxima's way through memory and the sum's launch (fp32, d = 64, 60 x
-  // 60: 8 groups 50 us, as 5 groups of one run 53, as 4 37), and where there is work to
-  // save (bf16, d = 256, 30 x 30: 4 groups 18.8 us, as 2 22.5).  The maxima's array is
-  // bounded, and a tile's tape entries lie within 2^30 bytes.
   const int Bq = A.Bq, Tq = A.Tq;
-  const int64_t ntok = (int64_t)Bq * Tq, ftiles = (ntok + kTile - 1) / kTile;
-  const int64_t fgroups = (ftiles + kRows - 1) / kRows;
-  auto dealt = [](int64_t n) { return n <= 2 ? n : n <= 4 ? 4 : n <= kSpXcds ? kSpXcds : n; };
-  const bool flat = dealt(fgroups) * 5 <= dealt(A.nqg) * 4 && (int64_t)A.nqg * A.Bd >= 256 && ntok <= ((int64_t)1 << 30) && (Tq + kTile) * Tq < 65536 &&
-                    ftiles * kTile * A.Bd <= ((int64_t)1 << 26) &&
-                    (int64_t)(kTile + 1) * A.Bd * Tq < ((int64_t)1 << 28);
+  const SplitRows rows = split_rows(Bq, Tq, A.Bd);
+  const bool flat = rows.flat;
+  A.ntq = (int)rows.ntq;
+  A.nqg = (int)rows.nqg;
   if (flat) {
     A.qtok = Tq;
     A.qrecip = (65536u + (unsigned)Tq - 1) / (unsigned)Tq;
     A.Bq = 1;
-    A.Tq = (int)ntok;
-    A.ntq = (int)ftiles;
-    A.nqg = (int)fgroups;
+    A.Tq = Bq * Tq;
   }
   // kBlocks blocks per CU (CUs a multiple of 8, so slot x stays on XCD x % 8).
   const int cus = std::max(kSpXcds, device_cus() / kSpXcds * kSpXcds);
@@ -828,14 +841,13 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   // could hold two long documents and its neighbour none.
   const int by_docs = A.Bd < 4 * A.R ? 1 : 0;
   // One workspace: the plan words (documents' chunk words, then query rows'
-  // words), the chunk list, the ranges, then, with several tiles per query, the
-  // tile scores St.
+  // words), the chunk list, the ranges, then the tile scores or token maxima St.
   const int64_t ndw = (int64_t)A.Bd * nch, nwords = ndw + (int64_t)A.Bq * A.ntq;
   auto al = [](size_t v) { return (v + 255) / 256 * 256; };
   const size_t plan_bytes = al((size_t)nwords * sizeof(uint32_t));
   const size_t list_bytes = al((size_t)A.Bd * std::max(nch, 1) * sizeof(uint4));
   const size_t rs_bytes = al((size_t)(A.R + 1 + kSpXcds) * sizeof(int32_t));  // (slots past R look there)
-  const size_t st_bytes = A.ntq > 1 ? (size_t)A.Bq * A.ntq * A.Bd * sizeof(float) * (flat ? kTile : 1) : 0;
+  const size_t st_bytes = (size_t)rows.stored * sizeof(float);
   void* ws = nullptr;
   hipError_t e = workspace_alloc(&ws, plan_bytes + list_bytes + rs_bytes + st_bytes, stream);
   if (e != hipSuccess) return e;
@@ -845,7 +857,7 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   A.qwords = plan + ndw;
   A.list = list;
   A.rs = rs;
-  if (A.ntq > 1)
+  if (st_bytes > 0)
     A.St = reinterpret_cast<float*>(static_cast<char*>(ws) + plan_bytes + list_bytes + rs_bytes);
   hipLaunchKernelGGL(split_plan_kernel, dim3((unsigned)std::min<int64_t>((nwords + 7) / 8, 1024)),
                      dim3(256), 0, stream, A.dm, A.qm, A.Bd, A.Td, nch, A.Bq, A.Tq, A.ntq, plan);
@@ -879,7 +891,7 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   if (e == hipSuccess && flat) {
     hipLaunchKernelGGL(split_token_sum_kernel,
                        dim3((unsigned)std::min<int64_t>(((int64_t)Bq * A.Bd + 255) / 256, 8192)), dim3(256), 0,
-                       stream, A.St, ftiles * kTile, Bq, A.Bd, A.qm, Tq, A.norm, A.S);
+                       stream, A.St, (int64_t)A.ntq * kTile, Bq, A.Bd, A.qm, Tq, A.norm, A.S);
     e = hipGetLastError();
   } else if (e == hipSuccess && A.ntq > 1) {
     hipLaunchKernelGGL(split_tile_sum_kernel,

@@ -40,6 +40,14 @@ struct InBatchSplitArgs {
 // Element bytes 2 or 4; rows a multiple of 16 bytes; 16-byte aligned bases.
 bool inbatch_split_supported(int esz, int64_t dim, int64_t Tq, int64_t Td, int64_t Bq,
                              int64_t Bd, const void* Q, const void* D);
+// The query rows of a call: one run of all tokens (flat) or tiles per query, ntq
+// tiles (flat: in all) in nqg groups of 8, and the floats of St (0: scores go
+// straight to S).
+struct SplitRows {
+  bool flat = false;
+  int64_t ntq = 1, nqg = 1, stored = 0;
+};
+SplitRows split_rows(int64_t Bq, int64_t Tq, int64_t Bd);
 // dtype: 0 fp32, 1 fp16, 2 bf16 (the C ABI's codes).
 hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args, hipStream_t stream);
 

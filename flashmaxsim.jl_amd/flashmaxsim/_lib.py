@@ -60,6 +60,7 @@ SIGNATURES = {
     "fms_workspace_lend": [_p, _i64],
     "fms_workspace_return": [],
     "fms_debug_inbatch_kernel": [_i32, _i64, _i64, _i64, _i64, _i64, _p, _p],
+    "fms_debug_split_rows": [_i64, _i64, _i64, _p],
     "fms_debug_cross_lane": [_p, _p],
     "fms_topk": [_p, _i64, _i64, _i64, _p, _p, _p],
     "fms_launch_packed_multi_scan": [_i32, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64,

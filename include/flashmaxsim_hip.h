@@ -482,6 +482,15 @@ int32_t fms_debug_inbatch_kernel(int32_t dtype, int64_t dim, int64_t Tq, int64_t
                                  int64_t Bd, const void* Q, const void* D);
 
 /*
+ * Test-only: how the split-K kernel takes the query rows of a call (no reference
+ * counterpart; host arithmetic, no device needed): out[0] = 1 when all queries'
+ * tokens are cut into 32-token tiles as one run, out[1] tiles (of the run, else
+ * per query), out[2] groups of 8 tiles, out[3] floats of workspace for their
+ * token maxima (one run) or tile scores (0: scores are written directly).
+ */
+fms_status fms_debug_split_rows(int64_t Tq, int64_t Bq, int64_t Bd, int64_t* out);
+
+/*
  * Test-only: streaming read of `bytes` (multiple of 16, 16-byte aligned)
  * with `blocks` workgroups of 256 threads; out receives blocks*256 words.
  * No reference counterpart: it measures the HBM read ceiling reported

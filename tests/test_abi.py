@@ -2,6 +2,7 @@
 public header declares, and its host-side validation returns the documented
 status codes without touching a GPU (every call here returns before any HIP
 call is made)."""
+import ctypes
 import os
 import re
 
@@ -164,3 +165,25 @@ def test_noalloc_rejects_workspace_beyond_its_scratch():
     import flashmaxsim as fm
     with pytest.raises(fm.UnsupportedError):
         _lib.check(_lib.FMS_ESCRATCH, "x")
+
+
+def test_split_rows_have_room_for_what_they_store():
+    """The split-K kernel stores token maxima (all tokens as one run) or tile scores
+    (several tiles per query) into workspace: its size covers them for every small call,
+    those whose tokens fit one 32-token tile included."""
+    out = (ctypes.c_int64 * 4)()
+    flat_tiles = set()
+    for Bq in list(range(1, 50)) + [300]:
+        for Tq in list(range(1, 70)) + [240]:
+            for Bd in (1, 64, 86, 128, 600):
+                assert _lib.lib().fms_debug_split_rows(Tq, Bq, Bd, out) == OK
+                flat, ntq, nqg, stored = out
+                per_query = -(-Tq // 32)
+                if flat:  # a row of whole tiles per document
+                    assert ntq == -(-Bq * Tq // 32) and stored == ntq * 32 * Bd
+                    flat_tiles.add(ntq)
+                else:
+                    assert ntq == per_query and stored == (Bq * ntq * Bd if ntq > 1 else 0)
+                assert nqg == -(-(ntq if flat else Bq * ntq) // 8)
+    assert {1, 2} <= flat_tiles
+    assert _lib.lib().fms_debug_split_rows(0, 1, 1, out) == EINVAL

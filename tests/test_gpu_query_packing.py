@@ -4,10 +4,13 @@ takes the kernel with a query per tile: the sums run in the same order, so score
 tapes are equal bit for bit.  Lengths at both ends of each count of queries per wave,
 query counts that leave a wave or a block part filled, documents without a valid token,
 documents that share a chunk, and Inf / NaN tokens."""
+import ctypes
+
 import pytest
 import torch
 
 import flashmaxsim as fm
+from flashmaxsim import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -72,6 +75,23 @@ def test_split_k_tokens_in_one_run(device, dtype, dim, Bq, Tq):
             dm[0] = dm[Bd - 1] = False
         _check(fm.inbatch_forward, Q, D, qm, dm)
         _check(fm.inbatch_forward, Q, D, None, None)
+
+
+@pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 256), (torch.float32, 128)])
+@pytest.mark.parametrize("Bq,Tq,Bd", [(32, 1, 64), (24, 1, 86), (16, 2, 128), (10, 3, 128), (9, 3, 600),
+                                      (33, 1, 128), (17, 2, 128)])
+def test_split_k_tokens_in_one_or_two_tiles(device, dtype, dim, Bq, Tq, Bd):
+    out = (ctypes.c_int64 * 4)()
+    assert _lib.lib().fms_debug_split_rows(Tq, Bq, Bd, out) == 0
+    assert list(out) == [1, -(-Bq * Tq // 32), 1, -(-Bq * Tq // 32) * 32 * Bd]  # one run, with room
+    g = torch.Generator(device=device).manual_seed(Bq)
+    Q = torch.randn(Bq, Tq, dim, generator=g, device=device).to(dtype)
+    D = torch.randn(Bd, 70, dim, generator=g, device=device).to(dtype)
+    qm = torch.rand(Bq, Tq, generator=g, device=device) < 0.8
+    dm = torch.rand(Bd, 70, generator=g, device=device) < 0.6
+    dm[0] = dm[Bd - 1] = False
+    _check(fm.inbatch_forward, Q, D, qm, dm)
+    _check(fm.inbatch_forward, Q, D, None, None)
 
 
 @pytest.mark.parametrize("dim", [64, 256])
