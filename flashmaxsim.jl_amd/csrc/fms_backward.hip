@@ -172,8 +172,10 @@ struct RowGeo {
 // layouts those before the first and after the last document too (`off` rows
 // precede the document's first).  The documents' rows and these ends together
 // cover every row, whatever cu holds.  npairs / first / slot0 / rows take a
-// wave-uniform document; pair / qok / qrow0 take per-lane arguments.
+// wave-uniform document; pair / qok / qrow0 take per-lane arguments.  kRagged:
+// documents differ in length; at(row) is the one whose rows hold `row`.
 struct DocsInBatch {  // document j: pairs p = j + Bd * i, i < Bq
+  static constexpr bool kRagged = false;
   int64_t ndocs;
   uint32_t Bd, Bq;
   int trows, Tq, Td;
@@ -187,6 +189,7 @@ struct DocsInBatch {  // document j: pairs p = j + Bd * i, i < Bq
   __device__ int64_t qrow0(uint32_t p) const { return (int64_t)(p / Bd) * Tq; }
 };
 struct DocsPaired {  // document b: pair b
+  static constexpr bool kRagged = false;
   int64_t ndocs;
   int trows, Tq, Td;
   const uint8_t* qm;
@@ -199,6 +202,7 @@ struct DocsPaired {  // document b: pair b
   __device__ int64_t qrow0(uint32_t p) const { return (int64_t)p * Tq; }
 };
 struct DocsCand {  // gallery document j: the pairs the document order lists for it
+  static constexpr bool kRagged = false;
   int64_t ndocs;
   const uint32_t* end;
   const PairRef* order;
@@ -223,13 +227,27 @@ __device__ __forceinline__ void ragged_rows(const int32_t* cu, int64_t nseg, int
   off = a - r0;
   cnt = z - r0;
 }
+// A segment whose rows (ends included) hold `row`: the last that starts at or
+// before it (row wave-uniform: scalar loads).
+__device__ __forceinline__ int64_t ragged_at(const int32_t* cu, int64_t nseg, int64_t row) {
+  int64_t lo = 0, hi = nseg;
+  while (hi - lo > 1) {
+    const int64_t mid = (lo + hi) >> 1;
+    const bool before = (int64_t)sload(cu, mid) - 1 <= row;
+    lo = before ? mid : lo;
+    hi = before ? hi : mid;
+  }
+  return lo;
+}
 struct DocsPacked {  // document b: pair b; one shared query
+  static constexpr bool kRagged = true;
   int64_t ndocs;
   int trows;
   const uint8_t* qm;
   const int32_t* cu;
   int64_t ntok;
   __device__ void rows(int64_t d, int64_t& r0, int64_t& n, int64_t& off) const { ragged_rows(cu, ndocs, ntok, d, r0, n, off); }
+  __device__ int64_t at(int64_t row) const { return ragged_at(cu, ndocs, row); }
   __device__ int64_t npairs(int64_t) const { return 1; }
   __device__ int64_t first(int64_t d) const { return d; }
   __device__ int64_t pair(int64_t d, uint32_t) const { return d; }
@@ -238,12 +256,14 @@ struct DocsPacked {  // document b: pair b; one shared query
   __device__ int64_t qrow0(uint32_t) const { return 0; }
 };
 struct DocsVarlen {  // document segment n: pair n
+  static constexpr bool kRagged = true;
   int64_t ndocs;
   int trows;
   const int32_t* cu_q;
   const int32_t* cu_d;
   int64_t nq, nd;
   __device__ void rows(int64_t d, int64_t& r0, int64_t& n, int64_t& off) const { ragged_rows(cu_d, ndocs, nd, d, r0, n, off); }
+  __device__ int64_t at(int64_t row) const { return ragged_at(cu_d, ndocs, row); }
   __device__ int64_t npairs(int64_t) const { return 1; }
   __device__ int64_t first(int64_t d) const { return d; }
   __device__ int64_t pair(int64_t d, uint32_t) const { return d; }
@@ -716,10 +736,21 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 // took 2 + 45 + 25 us, the sort idle for want of sources (about 40 a
 // document).  Bound by the chain of dependent loads (pair, tape, delta, list,
 // query row) and by the write of dD.
+//
+// Shares are cut for documents of average length.  In ragged stores the host
+// does not know a document's length, so a document's own workgroups stop `cap`
+// rows in, and workgroups past them take windows of `win` <= cap rows of the
+// store each: the rows of a window that lie cap or more into their document (one
+// document's, since any other that starts in the window has its first cap rows
+// beyond it) and none in a store of even lengths.(us per
+// varlen pullback, d = 128, bf16, with a long document's rows left to its own
+// workgroups / with windows: 1100 documents of 40 rows and one of 100000 3085 / 34;
+// 2000 of 100 and one of 8192 288 / 46.)
 template <class L, class Docs, class E, int kCPL>
 __global__ void __launch_bounds__(kDocThreads) bwd_doc_dd_kernel(
     const L lay, const Docs docs, const DeltaOf<E> delta, const int32_t* args, int rows, RowGeo geo,
-    int64_t rb, const char* Qbase, char* dD, int shares, uint32_t* heavy) {
+    int64_t rb, const char* Qbase, char* dD, int shares, int64_t cap, int64_t win, int64_t nwin,
+    uint32_t* heavy) {
   constexpr int kV = E::kV;
   __shared__ uint32_t cnt[kDocTile], cur[kDocTile];
   __shared__ uint2 list[kDocList];
@@ -727,14 +758,32 @@ __global__ void __launch_bounds__(kDocThreads) bwd_doc_dd_kernel(
   const int tid = threadIdx.x, lane = tid & 63, w = uniform(tid >> 6);
   const int lg = geo.lg_lr, lr = 1 << lg, rpi = 64 >> lg;
   const int gid = lane >> lg, c0 = lane & (lr - 1);
-  for (int64_t blk = blockIdx.x; blk < docs.ndocs * shares; blk += gridDim.x) {
-    const int64_t d = blk / shares;
-    const int share = (int)(blk - d * shares);
+  const int64_t own = docs.ndocs * shares;
+  for (int64_t blk = blockIdx.x; blk < own + nwin; blk += gridDim.x) {
+    int64_t d = blk / shares;
+    int share = (int)(blk - d * shares);
+    const int64_t w0 = (blk - own) * win;  // (below 0: the document's own share)
+    if constexpr (Docs::kRagged) {
+      if (w0 >= 0) d = uni64(docs.at(w0));
+    }
     int64_t r0, nrow, off;
     docs.rows(d, r0, nrow, off);
     r0 = uni64(r0);
     nrow = uni64(nrow);
     off = uni64(off);
+    // rows [ubeg, uend) of the document are this workgroup's
+    int64_t ubeg, uend;
+    if (Docs::kRagged && w0 >= 0) {
+      share = 0;
+      ubeg = std::max(w0 - r0, cap);
+      uend = std::min(w0 + win - r0, nrow);
+      if (ubeg >= uend) continue;
+    } else {
+      const int64_t mine = Docs::kRagged ? std::min(nrow, cap) : nrow;
+      const int64_t per = (mine + shares - 1) / shares;
+      ubeg = share * per;
+      uend = std::min(mine, ubeg + per);
+    }
     const int64_t np = uni64(docs.npairs(d));
     int td = 0, tq = 0;
     if (np > 0) {
@@ -747,8 +796,6 @@ __global__ void __launch_bounds__(kDocThreads) bwd_doc_dd_kernel(
       if (share == 0 && tid == 0) heavy[1 + atomicAdd(&heavy[0], 1u)] = (uint32_t)d;
       continue;
     }
-    const int64_t per = (nrow + shares - 1) / shares;
-    const int64_t rend = std::min(nrow, (int64_t)(share + 1) * per);
     // Sources f = k * tq + t of the document (pair k, query token t): its row
     // among the rows this document writes (-1: none) and its list entry.
     int64_t key[kDocKeep];
@@ -767,8 +814,8 @@ __global__ void __launch_bounds__(kDocThreads) bwd_doc_dd_kernel(
         if (u >= 1 && u <= td && dl != 0.0f && docs.qok((uint32_t)p, t)) key[q] = off + u - 1;
       }
     }
-    for (int64_t u0 = share * per; u0 < rend; u0 += kDocTile) {
-      const int ut = (int)std::min<int64_t>(kDocTile, rend - u0);
+    for (int64_t u0 = ubeg; u0 < uend; u0 += kDocTile) {
+      const int ut = (int)std::min<int64_t>(kDocTile, uend - u0);
       if (nsrc > 0) {
         for (int i = tid; i < ut; i += kDocThreads) cnt[i] = 0u;
         __syncthreads();
@@ -1913,13 +1960,20 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hi
         // at least 32 rows (ragged stores: on average).
         const int64_t avg = a.nd_rows / ndocs;
         const int shares = (int)std::max<int64_t>(1, std::min<int64_t>(bcdiv(1024, ndocs), avg / 32));
-        const unsigned blocks = (unsigned)std::min<int64_t>(ndocs * shares, 65536);
+        // (windows: enough to spread a long document, few enough to find their rows)
+        constexpr bool kRagged = decltype(docs)::kRagged;
+        const int64_t win = std::max<int64_t>(256, bcdiv(a.nd_rows, 32768));
+        const int64_t cap = std::max(win, 2 * avg);
+        const int64_t nwin = kRagged && a.nd_rows > cap ? bcdiv(a.nd_rows, win) : 0;
+        const unsigned blocks = (unsigned)std::min<int64_t>(ndocs * shares + nwin, 65536);
         if (geo.cpl == 1)
           hipLaunchKernelGGL((bwd_doc_dd_kernel<L, decltype(docs), E, 1>), dim3(blocks), dim3(kDocThreads),
-                             0, st, lay, docs, delta, a.args, a.rows, geo, rb, a.Qbase, a.dD, shares, heavy);
+                             0, st, lay, docs, delta, a.args, a.rows, geo, rb, a.Qbase, a.dD, shares, cap, win, nwin,
+                             heavy);
         else
           hipLaunchKernelGGL((bwd_doc_dd_kernel<L, decltype(docs), E, 2>), dim3(blocks), dim3(kDocThreads),
-                             0, st, lay, docs, delta, a.args, a.rows, geo, rb, a.Qbase, a.dD, shares, heavy);
+                             0, st, lay, docs, delta, a.args, a.rows, geo, rb, a.Qbase, a.dD, shares, cap, win, nwin,
+                             heavy);
       }
       if (many) {
         // (heavy documents: at most nsrc / kDocList of them, usually none)

@@ -102,3 +102,84 @@ def test_ragged_tokens_outside_every_segment(device, dtype):
     g = dP.float().cpu().numpy()
     assert np.isfinite(g).all() and (g[:5] == 0).all() and (g[69:] == 0).all()
     assert (g[5:7] != 0).any()
+
+
+def _ragged_want(Qt, Dt, cu_q, cu_d, args, Dl):
+    """(dQ, dD, |dQ| terms, |dD| terms) of ragged pairs; cu_q None: one query for all."""
+    q, d = Qt.double().numpy(), Dt.double().numpy()
+    out = [np.zeros_like(q), np.zeros_like(d), np.zeros_like(q), np.zeros_like(d)]
+    n, rows = args.shape
+    for i in range(n):
+        a, tq = (0, len(q)) if cu_q is None else (cu_q[i] - 1, min(cu_q[i + 1] - cu_q[i], rows))
+        u = args[i, :tq].astype(np.int64)
+        t = np.flatnonzero((u >= 1) & (u <= cu_d[i + 1] - cu_d[i]))
+        r, c = a + t, cu_d[i] - 1 + u[t] - 1
+        for k, (dst, src, x) in enumerate(((r, c, d), (c, r, q))):
+            np.add.at(out[k], dst, Dl[i] * x[src])
+            np.add.at(out[k + 2], dst, np.abs(Dl[i] * x[src]))
+    return out
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: DT_ID[d])
+@pytest.mark.parametrize("dim", [64, 768])
+@pytest.mark.parametrize("lens,before,after", [
+    # far from the average length: past what a document's own workgroups take (256 rows
+    # here), to the row, in several windows, and next to one another
+    ([255, 256, 257, 1, 0, 511, 512, 513, 1300] + [3] * 40, 0, 0),
+    ([3] * 30 + [2900] + [3] * 30 + [0, 700], 600, 1025),  # rows of no document on both ends
+    ([2000, 2000, 9], 0, 0),  # three documents: shares of long ones, none in a window
+])
+def test_ragged_long_documents(device, dtype, dim, lens, before, after):
+    rng = np.random.default_rng([len(lens), before])
+    N, Tq = len(lens), 12
+    cu_d = (before + 1 + np.concatenate([[0], np.cumsum(lens)])).astype(np.int32)
+    qlens = rng.integers(0, Tq + 1, N)
+    qlens[0] = Tq
+    cu_q = (1 + np.concatenate([[0], np.cumsum(qlens)])).astype(np.int32)
+    nd = before + sum(lens) + after
+    Dt, _, _ = as_feature(tokens(rng, (nd, dim)), dtype)
+    Qt, _, _ = as_feature(tokens(rng, (int(qlens.sum()), dim)), dtype)
+    args = np.stack([rng.integers(0, n + 2, Tq) for n in lens]).astype(np.int32)
+    Dl_t, Dl = _vals(rng, (N,), dtype, device)
+    P = fm.PackedSeq(Dt.to(device), _dev(cu_d, device), max(lens))
+    R = fm.PackedSeq(Qt.to(device), _dev(cu_q, device), Tq)
+    dQ, dD = bw.varlen_pullback(Dl_t, R, P, _dev(args, device))
+    want = _ragged_want(Qt, Dt, cu_q, cu_d, args, Dl)
+    assert_grad(dQ, want[0], want[2], dtype, "dQ")
+    assert_grad(dD, want[1], want[3], dtype, "dD")
+    q1 = Qt[:Tq].contiguous()
+    dq, dP = bw.packed_pullback(Dl_t, q1.to(device), P, None, _dev(args, device))
+    want = _ragged_want(q1, Dt, None, cu_d, args, Dl)
+    assert_grad(dq, want[0], want[2], dtype, "dq")
+    assert_grad(dP, want[1], want[3], dtype, "dP")
+
+
+def _best_us(fn):
+    fn()
+    best = float("inf")
+    for _ in range(8):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        fn()
+        e1.record()
+        e1.synchronize()
+        best = min(best, e0.elapsed_time(e1) * 1e3)
+    return best
+
+
+def test_one_long_document_costs_no_more_than_its_rows(device):
+    """1000 documents over 100000 rows, all of 100 rows or one of 90000: the same rows,
+    pairs and sources, so about the same time (left to one workgroup, the long one took
+    over 20 times as long)."""
+    g = torch.Generator(device=device).manual_seed(1)
+    tok = torch.randn(100000, 128, generator=g, device=device).bfloat16()
+    q = torch.randn(32, 128, generator=g, device=device).bfloat16()
+    us = []
+    for lens in ([100] * 1000, [10] * 500 + [90009] + [10] * 498 + [11]):
+        cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]) + 1, dtype=torch.int32, device=device)
+        assert int(cu[-1]) == 100001
+        P = fm.PackedSeq(tok, cu, max(lens))
+        S, a = fm.packed_forward(q, P)
+        us.append(_best_us(lambda: bw.packed_pullback(torch.ones_like(S), q, P, None, a)))
+    print("us", us)
+    assert us[1] < 6 * us[0]
