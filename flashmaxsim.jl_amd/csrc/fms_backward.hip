@@ -303,6 +303,14 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_zero16_kernel(uint16_t* w, in
 
 // ---- vector path: dQ --------------------------------------------------------------------
 
+constexpr int kZeroRows = 128;  // query rows of no pair that a wave writes (varlen)
+
+// Rows a .. b - 1 of nch 16-byte chunks = 0, by one wave.
+__device__ __forceinline__ void zero_rows(char* p, int64_t a, int64_t b, int nch, int lane) {
+  for (int64_t c = a * nch + lane; c < b * nch; c += 64)
+    *reinterpret_cast<uint4*>(p + c * 16) = make_uint4(0u, 0u, 0u, 0u);
+}
+
 // Work item = (query group g, token block tb).  kWaveSplit: a workgroup owns
 // one (item, split) and its four waves split the split's pairs (the pairs of
 // split s of group g are g*G + [s*ps, (s+1)*ps)); otherwise each wave owns
@@ -325,7 +333,20 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dq_vec_kernel(
   } else {
     split = 0;
     item = (int64_t)blockIdx.x * 4 + w;
-    if (item >= nitems) return;  // whole wave
+    if (item >= nitems) {  // whole wave
+      if constexpr (std::is_same<L, LayVarlen>::value) {
+        // window of query rows past the pairs' waves (see the end of the kernel)
+        const int64_t w0 = (item - nitems) * kZeroRows;
+        if (w0 >= nq_rows) return;
+        const int64_t n = nitems / ntb, d = uni64(ragged_at(lay.cu_q, n, w0));
+        int64_t r0, cnt, off;
+        ragged_rows(lay.cu_q, n, lay.nq, d, r0, cnt, off);
+        const int64_t lo = std::max(w0, r0 + kZeroRows), hi = std::min(w0 + kZeroRows, r0 + cnt);
+        zero_rows(dQ, lo, std::min(hi, r0 + off), geo.nch, lane);
+        zero_rows(dQ, std::max(lo, r0 + off + lay.get(d).tq), hi, geo.nch, lane);
+      }
+      return;
+    }
   }
   const int64_t g = item / ntb;
   const int tb = (int)(item - g * ntb);
@@ -454,16 +475,18 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dq_vec_kernel(
   if constexpr (std::is_same<L, LayVarlen>::value) {
     // Query rows of no pair: tokens past `rows` of this pair, and those before
     // the first and after the last pair (rows past the segment's own tokens
-    // and before it; see ragged_rows).
+    // and before it; see ragged_rows).  There can be any number of them, so this
+    // wave takes those within its segment's first kZeroRows rows, and waves past
+    // the pairs' take a window of kZeroRows rows each: what lies further into the
+    // segment that holds the window's first row (us per varlen pullback of 200 pairs,
+    // d = 128, bf16, 300000 rows of queries and of documents past the last pair, dQ's
+    // by one wave / by windows: 1919 / 49).
     if (tb == ntb - 1) {
       int64_t r0, n, off;
       ragged_rows(lay.cu_q, nitems / ntb, lay.nq, g, r0, n, off);
-      auto zero = [&](int64_t a, int64_t b) {
-        for (int64_t c = a * geo.nch + lane; c < b * geo.nch; c += 64)
-          *reinterpret_cast<uint4*>(dQ + c * 16) = make_uint4(0u, 0u, 0u, 0u);
-      };
-      zero(r0, r0 + off);
-      zero(r0 + off + v0.tq, r0 + n);
+      const int64_t end = r0 + std::min<int64_t>(n, kZeroRows);
+      zero_rows(dQ, r0, std::min(end, r0 + off), geo.nch, lane);
+      zero_rows(dQ, r0 + off + v0.tq, end, geo.nch, lane);
     }
   }
 }
@@ -742,7 +765,7 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 // rows in, and workgroups past them take windows of `win` <= cap rows of the
 // store each: the rows of a window that lie cap or more into their document (one
 // document's, since any other that starts in the window has its first cap rows
-// beyond it) and none in a store of even lengths.(us per
+// beyond it) and none in a store of even lengths.  (us per
 // varlen pullback, d = 128, bf16, with a long document's rows left to its own
 // workgroups / with windows: 1100 documents of 40 rows and one of 100000 3085 / 34;
 // 2000 of 100 and one of 8192 288 / 46.)
@@ -1939,7 +1962,8 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hi
                        lay, delta, a.args, a.G, a.rows, ntb, (int)nsplit, nitems, geo, rb, a.dim,
                        a.Qbase, a.dQ, part, a.nq_rows, heavy);
   } else {
-    hipLaunchKernelGGL((bwd_dq_vec_kernel<L, E, false>), dim3((unsigned)bcdiv(nitems, 4)),
+    const int64_t zero_waves = std::is_same<L, LayVarlen>::value ? bcdiv(a.nq_rows, kZeroRows) : 0;
+    hipLaunchKernelGGL((bwd_dq_vec_kernel<L, E, false>), dim3((unsigned)bcdiv(nitems + zero_waves, 4)),
                        dim3(kBwdThreads), 0, st, lay, delta, a.args, a.G, a.rows, ntb, 1, nitems,
                        geo, rb, a.dim, a.Qbase, a.dQ, part, a.nq_rows, heavy);
   }

@@ -154,6 +154,31 @@ def test_ragged_long_documents(device, dtype, dim, lens, before, after):
     assert_grad(dP, want[1], want[3], dtype, "dP")
 
 
+@pytest.mark.parametrize("dtype", DTYPES, ids=lambda d: DT_ID[d])
+@pytest.mark.parametrize("dim", [64, 768])
+@pytest.mark.parametrize("before,after", [(0, 127), (128, 0), (129, 130), (700, 1100)])
+def test_query_rows_of_no_pair_are_zero(device, dtype, dim, before, after):
+    """Any number of them: ahead of the first query and past the last (windows of 128 rows),
+    and a query segment far longer than max_q."""
+    rng = np.random.default_rng([before, after])
+    qlens, dlens, max_q = [3, 12, 0, 500, 1, 128, 129, 12], [20] * 8, 12
+    cu_q = (before + 1 + np.concatenate([[0], np.cumsum(qlens)])).astype(np.int32)
+    cu_d = (1 + np.concatenate([[0], np.cumsum(dlens)])).astype(np.int32)
+    Qt, _, _ = as_feature(tokens(rng, (before + sum(qlens) + after, dim)), dtype)
+    Dt, _, _ = as_feature(tokens(rng, (sum(dlens), dim)), dtype)
+    args = rng.integers(1, 21, size=(8, max_q)).astype(np.int32)
+    Dl_t, Dl = _vals(rng, (8,), dtype, device)
+    junk = torch.full_like(Qt, float("nan"), device=device)  # what the allocator hands out next
+    R = fm.PackedSeq(Qt.to(device), _dev(cu_q, device), max_q)
+    P = fm.PackedSeq(Dt.to(device), _dev(cu_d, device), 20)
+    tape = _dev(args, device)
+    del junk
+    dQ, dD = bw.varlen_pullback(Dl_t, R, P, tape)
+    want = _ragged_want(Qt, Dt, cu_q, cu_d, args, Dl)
+    assert_grad(dQ, want[0], want[2], dtype, "dQ")
+    assert_grad(dD, want[1], want[3], dtype, "dD")
+
+
 def _best_us(fn):
     fn()
     best = float("inf")
@@ -183,3 +208,19 @@ def test_one_long_document_costs_no_more_than_its_rows(device):
         us.append(_best_us(lambda: bw.packed_pullback(torch.ones_like(S), q, P, None, a)))
     print("us", us)
     assert us[1] < 6 * us[0]
+
+
+def test_rows_past_the_last_pair_cost_no_more_than_their_bytes(device):
+    """200 pairs in stores with 100000 rows past the last one, against the same rows as 200
+    longer pairs (left to one wave, dQ's spare rows took over 10 times as long)."""
+    g = torch.Generator(device=device).manual_seed(1)
+    q = torch.randn(104000, 128, generator=g, device=device).bfloat16()
+    cu_d = torch.arange(201, dtype=torch.int32, device=device) * 100 + 1
+    P = fm.PackedSeq(torch.randn(20000, 128, generator=g, device=device).bfloat16(), cu_d, 100)
+    us = []
+    for n in (520, 20):
+        R = fm.PackedSeq(q, torch.arange(201, dtype=torch.int32, device=device) * n + 1, 20)
+        S, a = fm.varlen_forward(R, P)
+        us.append(_best_us(lambda: bw.varlen_pullback(torch.ones_like(S), R, P, a)))
+    print("us", us)
+    assert us[1] < 5 * us[0]
