@@ -901,12 +901,16 @@ __global__ void __launch_bounds__(kDocThreads) bwd_doc_dd_kernel(
 // ---- dD of documents with many sources --------------------------------------------------------
 // Past kDocList sources a document, one 1024-thread sort per document into
 // global row lists and a row-sum kernel over all rows are the better split:
-// every row has its own waves however few documents there are (fp32, d = 128,
-// Td = 180, us per pullback with these / with a workgroup per document and
-// share: in-batch 128 x 128 66 / 97, 512 x 512 670 / 916; 64 x 100 candidates
-// on three documents 221 / 389; below kDocList sources, in-batch 64 x 64 73 /
-// 45).  In-batch and long queries the host knows; of candidates the device
-// lists such documents (heavy), and there may be none.
+// every row has its own waves however few documents there are.  us per pullback
+// with these / with a workgroup per document and share, both with lent workspace,
+// 32 query tokens, Td = 180: in-batch fp32, d = 64: 32 x 32 25 / 25, 48 x 48 32 / 29, 64 x 64
+// (2048 sources) 37 / 33, 80 x 80 41 / 40, 112 x 112 56 / 76, 128 x 128 64 / 86; d = 128: 64 x 64
+// 38 / 38, 80 x 80 44 / 48, 128 x 128 68 / 99; 64 x 100 candidates on three documents
+// 221 / 389.  In-batch and long queries the host knows; of candidates the device
+// lists such documents (heavy), and there may be none, unless their average is
+// at 3/4 of the line or more: then all take these, since with a few on each
+// side both passes are paid (bf16, d = 128, 200 documents of 1792 / 2048 / 2304 sources on
+// average: @C2).
 // Exclusive scan of cnt[0, n) (n <= kCsrTile) into out[]; returns the total.
 // Every thread of the (kCsrThreads) block calls it.
 __device__ uint32_t csr_scan_tile(const uint32_t* cnt, uint32_t* out, int n) {
@@ -1757,6 +1761,9 @@ template <class L> size_t docs_workspace(const L&, int64_t) { return 0; }
 int64_t doc_sources(const LayInBatch& l, const PullbackArgs& a) { return a.npairs / l.Bd * a.rows; }
 int64_t doc_sources(const LayCand&, const PullbackArgs& a) { return a.npairs * a.rows; }
 template <class L> int64_t doc_sources(const L&, const PullbackArgs& a) { return a.rows; }
+// Documents of a candidate call (host; of the other layouts it is not asked).
+int64_t doc_count(const LayCand& l) { return l.N; }
+template <class L> int64_t doc_count(const L&) { return 0; }
 template <> size_t docs_workspace<LayCand>(const LayCand& l, int64_t npairs) {
   return al256(group_workspace_bytes(npairs, l.N));
 }
@@ -1937,10 +1944,13 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hi
   const size_t b_part = nsplit > 1 ? al256((size_t)(nsplit * a.nq_rows * a.dim) * 4) : 0;
   constexpr bool kCand = std::is_same<L, LayCand>::value;
   const bool many = doc_sources(lay, a) > kDocList;  // (for candidates: possibly)
+  // Every document is sorted by bwd_doc_csr.  Candidates: where the average is near the
+  // line, since a mix of documents on both sides of it pays both passes (see kDocList).
+  const bool sorted = many && (!kCand || nsrc * 4 >= (int64_t)kDocList * 3 * doc_count(lay));
   const size_t b_list = many ? al256((size_t)nsrc * 8) : 0;
   const size_t b_rows = many ? al256((size_t)std::max<int64_t>(a.nd_rows, 1) * 4) : 0;
   const size_t b_docs = docs_workspace(lay, a.npairs);
-  const size_t b_heavy = kCand && many ? al256((size_t)(nsrc / kDocList + 1) * 4) : 0;
+  const size_t b_heavy = many && !sorted ? al256((size_t)(nsrc / kDocList + 1) * 4) : 0;
   const size_t b_all = b_part + b_list + 2 * b_rows + b_docs + b_heavy;
   void* ws = nullptr;
   hipError_t e = hipSuccess;
@@ -1979,7 +1989,7 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hi
     const auto docs = make_docs(lay, a, gws, st, &eg);
     if (eg == hipSuccess) {
       const int64_t ndocs = std::max<int64_t>(docs.ndocs, 1);
-      if (kCand || !many) {
+      if (!sorted) {
         // Shares of a document's rows: enough workgroups for four on each CU, of
         // at least 32 rows (ragged stores: on average).
         const int64_t avg = a.nd_rows / ndocs;
@@ -2001,13 +2011,13 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hi
       }
       if (many) {
         // (heavy documents: at most nsrc / kDocList of them, usually none)
-        const int td = kCand ? (int)(a.nd_rows / ndocs) : 0;
-        const int64_t cdocs = kCand ? std::min<int64_t>(256, nsrc / kDocList) : ndocs;
-        const int64_t crows = kCand ? std::min<int64_t>(nsrc / kDocList * td, 8192) : a.nd_rows;
+        const int td = sorted ? 0 : (int)(a.nd_rows / ndocs);
+        const int64_t cdocs = sorted ? ndocs : std::min<int64_t>(256, nsrc / kDocList);
+        const int64_t crows = sorted ? a.nd_rows : std::min<int64_t>(nsrc / kDocList * td, 8192);
         const int64_t per_block = 4 * (int64_t)(64 >> geo.lg_lr);
         const unsigned dblocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(cdocs, 65536));
         const unsigned rblocks = (unsigned)std::max<int64_t>(1, std::min<int64_t>(1048576, bcdiv(crows, per_block)));
-        if (!kCand)
+        if (sorted)
           hipLaunchKernelGGL(bwd_zero_kernel, dim3(grid_for(bcdiv(a.nd_rows, 64))), dim3(kBwdThreads), 0,
                              st, rcount, a.nd_rows);
         hipLaunchKernelGGL((bwd_doc_csr_kernel<L, decltype(docs), E>), dim3(dblocks), dim3(kCsrThreads), 0,

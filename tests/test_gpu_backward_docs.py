@@ -25,6 +25,8 @@ def _dev(a, device):
 @pytest.mark.parametrize("B,C,N,Tq,Td,dim,hot", [
     (5, 16, 4, 32, 40, 128, 2),      # 640 sources a document, and none on two
     (9, 60, 30, 32, 33, 64, 3),      # documents past the LDS list among documents without a pair
+    (9, 16, 3, 32, 40, 64, 2),       # 1536 sources on average: every document sorted
+    (9, 16, 3, 31, 40, 64, 2),       # just below: two documents past the list, one empty
     (2, 64, 2, 32, 1030, 128, 1),    # exactly 4096 sources, two row tiles
     (1, 64, 1, 32, 70, 768, 1),      # exactly 2048: the largest LDS list; two chunks a lane
 ])
