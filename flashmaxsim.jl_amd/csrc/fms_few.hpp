@@ -198,6 +198,27 @@ constexpr int64_t few_pairs() {
   return Op::kEsz == 4 ? (int64_t)1 << 22 : 512;
 }
 
+// Past one workgroup per CU, 16-bit rows that are not kept (every chunk loads the query
+// tile again) compete with scan_fast at d = 256 and scan_split, which keep or stream it:
+// bytes of a document, on average, up to which a workgroup per pair still pays.
+// us per call at 512 pairs, wave / workgroup per pair: packed documents (one query,
+// whose lines all workgroups read at once), d = 256, up to 180 / 400 / 2000 tokens 16 / 14,
+// 27 / 27, 105 / 158; d = 768, 90 / 900 / 2000 tokens 21 / 24, 153 / 255, 334 / 582; pairs
+// with a query each, d = 256, 900 / 2000 tokens 68 / 62, 163 / 180 (ragged, 666 .. 2000
+// tokens 106 / 153), d = 768 417 / 290, 902 / 638.  (At 256 pairs the workgroups win
+// throughout, 1.1 to 4 times.)
+constexpr int64_t kFewFull = 256;
+template <class L>
+constexpr int64_t few_doc_bytes(bool) { return 0; }
+template <>
+constexpr int64_t few_doc_bytes<LayPacked>(bool split) { return split ? 48 << 10 : 96 << 10; }
+template <>
+constexpr int64_t few_doc_bytes<LayPaired>(bool split) { return split ? INT64_MAX : 512 << 10; }
+template <>
+constexpr int64_t few_doc_bytes<LayCand>(bool split) { return few_doc_bytes<LayPaired>(split); }
+template <>
+constexpr int64_t few_doc_bytes<LayVarlen>(bool split) { return few_doc_bytes<LayPaired>(split); }
+
 // 16-byte fragment loads: every row is whole 16-byte units from an aligned base
 // (fp32 scans otherwise load dwords and ask for neither).
 inline bool few_aligned(const void* q, const void* d) {
@@ -210,9 +231,10 @@ inline bool few_aligned(const LayPacked& l) { return few_aligned(l.q, l.tok); }
 inline bool few_aligned(const LayVarlen& l) { return few_aligned(l.Qt, l.Dt); }
 
 // The launch, or false when the call stays with the wave-per-pair scans.
-// two: the scan that serves this dim with more pairs keeps two chains.
+// two: the scan that serves this dim with more pairs is scan_split, which keeps two
+// chains; fast: it is scan_fast.
 template <class Op, class L>
-bool launch_few(const ScanArgs<L>& A, bool vec, bool two, hipStream_t stream, hipError_t* err) {
+bool launch_few(const ScanArgs<L>& A, bool vec, bool two, bool fast, hipStream_t stream, hipError_t* err) {
   const int rowbytes = A.dim * Op::kEsz;
   if (!vec || A.dim <= 0 || rowbytes % 16 != 0 || A.npairs < 1 || A.npairs > few_pairs<Op>()) return false;
   if (!few_aligned(A.lay)) return false;
@@ -221,6 +243,9 @@ bool launch_few(const ScanArgs<L>& A, bool vec, bool two, hipStream_t stream, hi
   const unsigned W = (unsigned)(nch < kFewMaxWaves ? nch : kFewMaxWaves);
   const dim3 grid((unsigned)A.npairs), block(64 * W);
   const int nm = (rowbytes + 31) / 32;
+  if (Op::kEsz == 2 && A.npairs > kFewFull && nm > 8 && (two || fast) &&
+      nch * kTile * rowbytes > few_doc_bytes<L>(two))
+    return false;
   if constexpr (Op::kEsz == 4) {
     if (two && nm <= 8)
       hipLaunchKernelGGL((scan_few<Op, L, 8, true, true>), grid, block, 0, stream, A);

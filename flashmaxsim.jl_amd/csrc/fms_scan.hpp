@@ -434,7 +434,7 @@ __global__ void __launch_bounds__(64 * kWaves) scan_generic(const ScanArgs<L> A)
 
 // The scan of few pairs (fms_few.hpp): false when the call is not its.
 template <class Op, class L>
-bool launch_few(const ScanArgs<L>& A, bool vec, bool two, hipStream_t stream, hipError_t* err);
+bool launch_few(const ScanArgs<L>& A, bool vec, bool two, bool fast, hipStream_t stream, hipError_t* err);
 // The layouts it serves (document order holds many pairs: fp32 only).
 template <class Op, class L>
 struct few_layout { static constexpr bool value = true; };
@@ -484,7 +484,7 @@ hipError_t launch_scan(const L& lay, int dim, int rows, int64_t npairs, int32_t*
   const bool split = nkb_fast == 0 && vec && dim > 0 && dim % (kbat * Op::kKb) == 0;
   if constexpr (few_layout<Op, L>::value) {
     hipError_t e = hipSuccess;
-    if (launch_few<Op, L>(A, vec, split, stream, &e)) return e;
+    if (launch_few<Op, L>(A, vec, split, nkb_fast != 0, stream, &e)) return e;
   }
   if constexpr (Op::kEsz != 4) {
     constexpr int b = (Op::kKb == 16) ? 4 : 2;

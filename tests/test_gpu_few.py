@@ -152,3 +152,21 @@ def test_d96_matches_padded_rows(device, dtype, grouping):
     finally:
         boundary.candidates_grouping(prev)
     assert torch.equal(S, S_p) and torch.equal(a, a_p)
+
+
+@pytest.mark.parametrize("dim,Td", [(256, 160), (256, 240), (384, 60), (768, 100), (192, 300)])
+@pytest.mark.parametrize("layout", ["packed", "varlen"])
+def test_wide_rows_past_one_workgroup_per_cu(device, layout, dim, Td):
+    """256 and 257 16-bit pairs, documents on both sides of the size up to which the latter
+    still take a workgroup each: the same pairs score and choose alike."""
+    g = torch.Generator(device=device).manual_seed(dim + Td)
+    d = [torch.randn(Td - i % 3, dim, generator=g, device=device).half() for i in range(257)]
+    q = [torch.randn(1 + i % 35, dim, generator=g, device=device).half() for i in range(257)]
+    out = []
+    for n in (256, 257):
+        if layout == "packed":
+            out.append(fm.packed_forward(q[31], fm.pack_docs(d[:n])))
+        else:
+            out.append(fm.varlen_forward(*fm.pack_pairs(q[:n], d[:n])))
+    (S, a), (S1, a1) = out
+    assert _same(S, S1[:256]) and torch.equal(a, a1[:256])
