@@ -183,84 +183,108 @@ __global__ void __launch_bounds__(256) split_plan_kernel(const uint8_t* dm, cons
   }
 }
 
-// The chunk list, one block: entry {valid rows, document, chunk | last << 31, 0}
-// per listed chunk (see above), and rs[r], the first entry of range r (rs[R]: the
-// entries' number).  byDocs: range r starts at document r Bd / R; otherwise at the
-// first document whose first entry is at or past r / R of the list.
+// The chunk list: entry {valid rows, document, chunk | last << 31, 0} per listed
+// chunk (see above), and rs[r], the first entry of range r (rs[R]: the entries'
+// number).  byDocs: range r starts at document r Bd / R; otherwise at the first
+// document whose first entry is at or past r / R of the list.
+//
+// A block lists kListThreads documents, a thread per document.  With several
+// blocks split_count_kernel has left each one's number of entries in counts, and
+// every block adds up those before it and all of them; one block counts for itself.
+// (All documents by one block, kListThreads at a time, were a serial stretch ahead of
+// the scan.  us per call of 8 queries of 32 tokens, one block / a block per 1024: d = 40,
+// fp16, 5000 documents of 60 .. 180 tokens 121 / 99, with the tape 155 / 137; d = 256, bf16,
+// 50000 of them 1622 / 1318; d = 8, 200000 documents of one chunk 1523 / 1004; 2100 63 / 56.)
 constexpr int kListThreads = 1024;
-__global__ void __launch_bounds__(kListThreads) split_list_kernel(const uint32_t* plan, int Bd, int nch,
-                                                                  int R, int byDocs, uint4* list,
-                                                                  int32_t* rs) {
-  __shared__ int wsum[kListThreads / 64];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+
+// f(chunk, valid rows) for the chunks of document j with a valid row.
+template <class F>
+__device__ __forceinline__ void each_chunk(const uint32_t* plan, int nch, int64_t j, F f) {
   constexpr int kWords = 8;  // plan words in flight per thread
-  // f(chunk, valid rows) for the chunks of document j with a valid row
-  auto each_chunk = [&](int j, auto f) {
-    const uint32_t* const words = plan + (int64_t)j * nch;
-    for (int c0 = 0; c0 < nch; c0 += kWords) {
-      uint32_t m[kWords];
+  const uint32_t* const words = plan + j * nch;
+  for (int c0 = 0; c0 < nch; c0 += kWords) {
+    uint32_t m[kWords];
 #pragma unroll
-      for (int i = 0; i < kWords; ++i) m[i] = c0 + i < nch ? words[c0 + i] : 0u;
+    for (int i = 0; i < kWords; ++i) m[i] = c0 + i < nch ? words[c0 + i] : 0u;
 #pragma unroll
-      for (int i = 0; i < kWords; ++i)
-        if (m[i] != 0u) f(c0 + i, m[i]);
-    }
-  };
-  auto chunks_of = [&](int j) {
-    int n = 0;
-    each_chunk(j, [&](int, uint32_t) { ++n; });
-    return n > 0 ? n : 1;
-  };
-  // exclusive prefix of v over the block and its total (two barriers)
-  auto scan = [&](int v, int& total) {
-    int x = v;
+    for (int i = 0; i < kWords; ++i)
+      if (m[i] != 0u) f(c0 + i, m[i]);
+  }
+}
+
+// Entries of document j (0 past the last document).
+__device__ __forceinline__ int doc_entries(const uint32_t* plan, int nch, int64_t j, int Bd) {
+  if (j >= Bd) return 0;
+  int n = 0;
+  each_chunk(plan, nch, j, [&](int, uint32_t) { ++n; });
+  return n > 0 ? n : 1;
+}
+
+// Exclusive prefix of v over the block and its total (two barriers).
+__device__ __forceinline__ int list_scan(int v, int& total) {
+  __shared__ int wsum[kListThreads / 64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int x = v;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(x, o);
-      if (lane >= o) x += y;
-    }
-    if (lane == 63) wsum[w] = x;
-    __syncthreads();
-    int before = x - v;
-    total = 0;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) wsum[w] = x;
+  __syncthreads();
+  int before = x - v;
+  total = 0;
 #pragma unroll
-    for (int i = 0; i < kListThreads / 64; ++i) {
-      if (i < w) before += wsum[i];
-      total += wsum[i];
+  for (int i = 0; i < kListThreads / 64; ++i) {
+    if (i < w) before += wsum[i];
+    total += wsum[i];
+  }
+  __syncthreads();
+  return before;
+}
+
+__global__ void __launch_bounds__(kListThreads) split_count_kernel(const uint32_t* plan, int Bd, int nch,
+                                                                   int32_t* counts) {
+  int total;
+  list_scan(doc_entries(plan, nch, (int64_t)blockIdx.x * kListThreads + threadIdx.x, Bd), total);
+  if (threadIdx.x == 0) counts[blockIdx.x] = total;
+}
+
+__global__ void __launch_bounds__(kListThreads) split_list_kernel(const uint32_t* plan, int Bd, int nch,
+                                                                  int R, int byDocs, const int32_t* counts,
+                                                                  uint4* list, int32_t* rs) {
+  int base = 0, all = 0;
+  if (gridDim.x > 1) {
+    int mine = 0, every = 0;
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += kListThreads) {
+      const int c = counts[b];
+      every += c;
+      mine += b < (int)blockIdx.x ? c : 0;
     }
-    __syncthreads();
-    return before;
-  };
-  int all = 0;
-  if (!byDocs)
-    for (int j0 = 0; j0 < Bd; j0 += kListThreads) {
-      int t;
-      scan(j0 + tid < Bd ? chunks_of(j0 + tid) : 0, t);
-      all += t;
-    }
+    list_scan(mine, base);
+    list_scan(every, all);
+  }
+  const int64_t jt = (int64_t)blockIdx.x * kListThreads + threadIdx.x;
+  const int n = doc_entries(plan, nch, jt, Bd);
+  int total;
+  const int e0 = base + list_scan(n, total);
+  if (gridDim.x == 1) all = total;
+  if (n == 0) return;
+  const int j = (int)jt;
   // the range that document j, first entry e, belongs to
   auto range_of = [&](int j, int e) {
     return byDocs ? (int)(((int64_t)j * R + R - 1) / Bd) : (int)(((int64_t)e * R) / all);
   };
-  int base = 0;
-  for (int j0 = 0; j0 < Bd; j0 += kListThreads) {
-    const int j = j0 + tid;
-    const int n = j < Bd ? chunks_of(j) : 0;
-    int t;
-    const int e0 = base + scan(n, t);
-    base += t;
-    if (n == 0) continue;
-    int e = e0;
-    each_chunk(j, [&](int c, uint32_t m) {
-      list[e] = make_uint4(m, (uint32_t)j, (uint32_t)c | ((e + 1 == e0 + n) ? 0x80000000u : 0u), 0u);
-      ++e;
-    });
-    if (e == e0) list[e] = make_uint4(0u, (uint32_t)j, 0x80000000u, 0u);
-    // the ranges that start at the next document (or, past the last one, at the end)
-    const int en = e0 + n, lo = range_of(j, e0), hi = j + 1 == Bd ? R : range_of(j + 1, en);
-    if (j == 0) rs[0] = 0;
-    for (int r = lo + 1; r <= hi; ++r) rs[r] = en;
-  }
+  int e = e0;
+  each_chunk(plan, nch, j, [&](int c, uint32_t m) {
+    list[e] = make_uint4(m, (uint32_t)j, (uint32_t)c | ((e + 1 == e0 + n) ? 0x80000000u : 0u), 0u);
+    ++e;
+  });
+  if (e == e0) list[e] = make_uint4(0u, (uint32_t)j, 0x80000000u, 0u);
+  // the ranges that start at the next document (or, past the last one, at the end)
+  const int en = e0 + n, lo = range_of(j, e0), hi = j + 1 == Bd ? R : range_of(j + 1, en);
+  if (j == 0) rs[0] = 0;
+  for (int r = lo + 1; r <= hi; ++r) rs[r] = en;
 }
 
 // Slot x of the block order -> (range, query group); qg = nqg marks a slot with
@@ -841,28 +865,35 @@ hipError_t launch_inbatch_split(int32_t dtype, const InBatchSplitArgs& args_in,
   // could hold two long documents and its neighbour none.
   const int by_docs = A.Bd < 4 * A.R ? 1 : 0;
   // One workspace: the plan words (documents' chunk words, then query rows'
-  // words), the chunk list, the ranges, then the tile scores or token maxima St.
+  // words), the chunk list, the ranges, the list blocks' counts, then the tile
+  // scores or token maxima St.
   const int64_t ndw = (int64_t)A.Bd * nch, nwords = ndw + (int64_t)A.Bq * A.ntq;
   auto al = [](size_t v) { return (v + 255) / 256 * 256; };
   const size_t plan_bytes = al((size_t)nwords * sizeof(uint32_t));
   const size_t list_bytes = al((size_t)A.Bd * std::max(nch, 1) * sizeof(uint4));
   const size_t rs_bytes = al((size_t)(A.R + 1 + kSpXcds) * sizeof(int32_t));  // (slots past R look there)
+  const int list_blocks = (A.Bd + kListThreads - 1) / kListThreads;
+  const size_t counts_bytes = list_blocks > 1 ? al((size_t)list_blocks * sizeof(int32_t)) : 0;
   const size_t st_bytes = (size_t)rows.stored * sizeof(float);
   void* ws = nullptr;
-  hipError_t e = workspace_alloc(&ws, plan_bytes + list_bytes + rs_bytes + st_bytes, stream);
+  hipError_t e = workspace_alloc(&ws, plan_bytes + list_bytes + rs_bytes + counts_bytes + st_bytes, stream);
   if (e != hipSuccess) return e;
   uint32_t* const plan = static_cast<uint32_t*>(ws);
   uint4* const list = reinterpret_cast<uint4*>(static_cast<char*>(ws) + plan_bytes);
   int32_t* const rs = reinterpret_cast<int32_t*>(static_cast<char*>(ws) + plan_bytes + list_bytes);
+  int32_t* const counts = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(rs) + rs_bytes);
   A.qwords = plan + ndw;
   A.list = list;
   A.rs = rs;
   if (st_bytes > 0)
-    A.St = reinterpret_cast<float*>(static_cast<char*>(ws) + plan_bytes + list_bytes + rs_bytes);
+    A.St = reinterpret_cast<float*>(reinterpret_cast<char*>(counts) + counts_bytes);
   hipLaunchKernelGGL(split_plan_kernel, dim3((unsigned)std::min<int64_t>((nwords + 7) / 8, 1024)),
                      dim3(256), 0, stream, A.dm, A.qm, A.Bd, A.Td, nch, A.Bq, A.Tq, A.ntq, plan);
-  hipLaunchKernelGGL(split_list_kernel, dim3(1), dim3(kListThreads), 0, stream, plan, A.Bd, nch, A.R,
-                     by_docs, list, rs);
+  if (list_blocks > 1)
+    hipLaunchKernelGGL(split_count_kernel, dim3((unsigned)list_blocks), dim3(kListThreads), 0, stream, plan,
+                       A.Bd, nch, counts);
+  hipLaunchKernelGGL(split_list_kernel, dim3((unsigned)list_blocks), dim3(kListThreads), 0, stream, plan,
+                     A.Bd, nch, A.R, by_docs, counts, list, rs);
   e = hipGetLastError();
   const dim3 grid((unsigned)std::min(A.nslots, cus * per_cu)), block(64 * kSpWaves);
   if (e == hipSuccess) {

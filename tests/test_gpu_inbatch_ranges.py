@@ -1,6 +1,6 @@
 """The split-K in-batch kernel's chunk list and ranges at their edges, against the
 paired scan of the same pairs (16-bit, d = 256: the same k order, so bit for bit):
-more documents than one tile of the list kernel, fewer query groups than XCDs and
+more documents than one and than several blocks of the list kernel, fewer query groups than XCDs and
 many, documents without a valid token at both ends of the list, single valid rows
 in late chunks, documents longer than a chunk group, and one K slice per group."""
 import pytest
@@ -20,7 +20,7 @@ def _masks(g, B, T, device, p):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("Bq,Bd,Tq,Td", [
     (1, 1, 1, 1), (3, 2500, 5, 40), (300, 7, 32, 33), (9, 1025, 33, 31), (70, 60, 32, 225),
-    (2, 1024, 8, 64), (17, 300, 40, 400)])
+    (2, 1024, 8, 64), (17, 300, 40, 400), (2, 5003, 3, 70), (1, 2048, 9, 33)])
 def test_ranges_match_the_paired_scan(device, dtype, Bq, Bd, Tq, Td):
     dim = 256
     g = torch.Generator(device=device).manual_seed(Bq * 1000 + Bd)
@@ -71,3 +71,4 @@ def test_fp32_ranges(device, dim, Bq, Bd, Tq, Td):
     took = torch.gather(sims, 3, (a.long() - 1).clamp(min=0)[..., None])[..., 0]
     assert bool(((took - best)[a > 0].abs() <= tol).all())
     assert bool(((S.double() - want.sum(-1)).abs() <= tol * Tq).all())
+
