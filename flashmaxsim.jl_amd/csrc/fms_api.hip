@@ -745,9 +745,7 @@ int32_t fms_candidates_grouping(int32_t mode) {
   return prev;
 }
 
-void fms_workspace_lend(void* ptr, int64_t bytes) { workspace_lend(ptr, bytes > 0 ? (size_t)bytes : 0); }
-
-int64_t fms_workspace_return(void) { return (int64_t)workspace_return(); }
+void fms_set_workspace_lender(fms_workspace_lender lender) { workspace_lender(lender); }
 
 uint64_t fms_debug_workspace_allocs(void) { return workspace_alloc_count(); }
 

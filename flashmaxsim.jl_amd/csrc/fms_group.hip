@@ -412,38 +412,31 @@ hipError_t stream_device(hipStream_t stream, int* dev) {
 namespace {
 std::atomic<uint64_t> g_workspace_allocs{0};
 
-struct Loan {
-  char* p = nullptr;
-  size_t bytes = 0, used = 0, wanted = 0;
-};
-thread_local Loan t_loan;
+thread_local WorkspaceLender t_lender = nullptr;
+// Lent pieces in use by this thread's call (an entry point holds two at most).
+constexpr int kMaxLent = 8;
+thread_local void* t_lent[kMaxLent];
+thread_local int t_nlent = 0;
 }  // namespace
 
-void workspace_lend(void* ptr, size_t bytes) {
-  t_loan = Loan();
-  if (ptr != nullptr && (reinterpret_cast<uintptr_t>(ptr) & 255u) == 0) {
-    t_loan.p = static_cast<char*>(ptr);
-    t_loan.bytes = bytes;
-  }
-}
-
-size_t workspace_return() {
-  const size_t wanted = t_loan.wanted;
-  t_loan = Loan();
-  return wanted;
-}
+void workspace_lender(WorkspaceLender lender) { t_lender = lender; }
 
 uint64_t workspace_alloc_count() { return g_workspace_allocs.load(std::memory_order_relaxed); }
 
 hipError_t workspace_alloc(void** ptr, size_t bytes, hipStream_t stream) {
   g_workspace_allocs.fetch_add(1, std::memory_order_relaxed);
-  Loan& loan = t_loan;
-  const size_t need = align256(bytes);
-  loan.wanted += need;
-  if (loan.p != nullptr && need <= loan.bytes - loan.used) {
-    *ptr = loan.p + loan.used;
-    loan.used += need;
-    return hipSuccess;
+  if (t_lender != nullptr && t_nlent < kMaxLent) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+      (void)hipGetLastError();
+      cap = hipStreamCaptureStatusActive;
+    }
+    void* const p = cap == hipStreamCaptureStatusNone ? t_lender((int64_t)bytes, stream) : nullptr;
+    if (p != nullptr && (reinterpret_cast<uintptr_t>(p) & 255u) == 0) {
+      t_lent[t_nlent++] = p;
+      *ptr = p;
+      return hipSuccess;
+    }
   }
   int dev = 0;
   hipError_t e = stream_device(stream, &dev);
@@ -455,8 +448,11 @@ hipError_t workspace_alloc(void** ptr, size_t bytes, hipStream_t stream) {
 }
 
 hipError_t workspace_free(void* ptr, hipStream_t stream) {
-  const uintptr_t off = reinterpret_cast<uintptr_t>(ptr) - reinterpret_cast<uintptr_t>(t_loan.p);
-  if (t_loan.p != nullptr && off < t_loan.bytes) return hipSuccess;
+  for (int i = t_nlent - 1; i >= 0; --i)
+    if (t_lent[i] == ptr) {
+      t_lent[i] = t_lent[--t_nlent];
+      return hipSuccess;
+    }
   return hipFreeAsync(ptr, stream);
 }
 

@@ -49,11 +49,10 @@ hipError_t stream_device(hipStream_t stream, int* dev);
 // device (created on first use, kept for the life of the process so repeated
 // calls do not return memory to the driver between synchronisations).
 hipError_t workspace_alloc(void** ptr, size_t bytes, hipStream_t stream);
-// Memory lent to this host thread: workspace_alloc serves from it what fits
-// (bump allocation; workspace_free of such a piece does nothing) until
-// workspace_return, which returns the bytes asked for since.
-void workspace_lend(void* ptr, size_t bytes);
-size_t workspace_return();
+// This host thread's lender (null: none), asked first for every workspace outside graph
+// capture; workspace_free of what it gave does nothing.
+typedef void* (*WorkspaceLender)(int64_t bytes, void* stream);
+void workspace_lender(WorkspaceLender lender);
 // Number of workspace_alloc calls so far in this process (a test probe).
 uint64_t workspace_alloc_count();
 hipError_t workspace_free(void* ptr, hipStream_t stream);

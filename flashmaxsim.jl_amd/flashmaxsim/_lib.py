@@ -26,6 +26,7 @@ _p = ctypes.c_void_p
 _i64 = ctypes.c_int64
 _i32 = ctypes.c_int32
 _f = ctypes.c_float
+LENDER = ctypes.CFUNCTYPE(_p, _i64, _p)  # fms_workspace_lender: (bytes, stream) -> memory
 
 # name -> argtypes (restype fms_status = int32 unless listed in _RESTYPES)
 SIGNATURES = {
@@ -57,8 +58,7 @@ SIGNATURES = {
     "fms_debug_gather_bandwidth": [_p, _i64, _i64, _p, _i64, _p, _p],
     "fms_candidates_grouping": [_i32],
     "fms_debug_workspace_allocs": [],
-    "fms_workspace_lend": [_p, _i64],
-    "fms_workspace_return": [],
+    "fms_set_workspace_lender": [LENDER],
     "fms_debug_inbatch_kernel": [_i32, _i64, _i64, _i64, _i64, _i64, _p, _p],
     "fms_debug_split_rows": [_i64, _i64, _i64, _p],
     "fms_debug_cross_lane": [_p, _p],
@@ -80,8 +80,7 @@ _RESTYPES = {
     "fms_arch_supported": ctypes.c_int,
     "fms_version": ctypes.c_char_p,
     "fms_debug_workspace_allocs": ctypes.c_uint64,
-    "fms_workspace_lend": None,
-    "fms_workspace_return": ctypes.c_int64,
+    "fms_set_workspace_lender": None,
 }
 
 _lib = None

@@ -111,32 +111,48 @@ def _norm(normalize) -> int:
 # ---- workspace -------------------------------------------------------------------------
 # The library takes its workspace from a stream-ordered pool of its own, whose
 # allocation holds the host until earlier work on the stream is done (a 64 x 64
-# in-batch call returned after its 64 us on the GPU).  A call that is lent memory
-# uses it instead: a torch allocation on the same stream, as large as the entry
-# point last asked for on this thread, given back when the call returns (the
-# caching allocator reuses it in stream order).  What does not fit, and every
+# in-batch call returned after its 64 us on the GPU).  Calls made here lend it torch
+# memory instead: the library asks for what the call needs (_lend), the pieces come
+# from the caching allocator on the call's stream and go back to it, to be reused
+# in stream order, when the call returns.  Whatever _lend declines, and every
 # allocation under graph capture, comes from the library's pool.
 
-_wanted = threading.local()  # entry point -> bytes its last call on this thread asked for
+class _Call(threading.local):
+    """The call this thread is in: its device and the pieces lent to it."""
+    device = None
+    pieces = None
+    known = False  # the library has this thread's lender
+
+
+_call = _Call()
+
+
+@_lib.LENDER
+def _lend(nbytes, stream):
+    if _call.pieces is None:  # not one of the calls below
+        return None
+    try:
+        # (a torch allocation belongs to torch's current stream)
+        if (stream or 0) != stream_handle(_call.device):
+            return None
+        t = torch.empty(nbytes, dtype=torch.uint8, device=_call.device)
+    except Exception:  # out of memory, say: the pool decides
+        return None
+    _call.pieces.append(t)
+    return t.data_ptr()
 
 
 def _call_with_workspace(fn, device, *args):
-    """fn(*args) with lent workspace on `device` (torch's current stream); its status."""
-    L = _lib.lib()
-    wanted = _wanted.__dict__
-    name = fn.__name__
-    n = wanted.get(name, 0)
-    ws = None
-    if n and not torch._C._cuda_isCurrentStreamCapturing():
-        try:
-            ws = torch.empty(n, dtype=torch.uint8, device=device)
-        except torch.OutOfMemoryError:
-            pass  # the library's pool decides
-    L.fms_workspace_lend(ptr(ws), 0 if ws is None else n)
+    """fn(*args) on `device`, its workspace lent by torch; its status."""
+    if not _call.known:
+        _lib.lib().fms_set_workspace_lender(_lend)
+        _call.known = True
+    outer = _call.device, _call.pieces
+    _call.device, _call.pieces = device, []
     try:
         return fn(*args)
     finally:
-        wanted[name] = L.fms_workspace_return()
+        _call.device, _call.pieces = outer
 
 
 # ---- argument checks ---------------------------------------------------------------
@@ -277,7 +293,7 @@ def inbatch_device_scan(S, args, Q, D, qmask, dmask, normalize=False):
     _buf(args, "args", torch.int32, Bq * Bd * Tq)
     dev = require_device(S, args, Q, D, qmask, dmask)
     st = _call_with_workspace(
-        _lib.lib().fms_inbatch_device_scan, dev, 
+        _lib.lib().fms_inbatch_device_scan, dev,
         dtype_code(Q), ptr(S), ptr(args), ptr(Q), ptr(D), ptr(_maskn(qmask, "qmask", Bq * Tq)),
         ptr(_maskn(dmask, "dmask", Bd * Td)), dim, Tq, Bq, Td, Bd, _norm(normalize),
         stream_handle(dev))
@@ -318,7 +334,7 @@ def launch_packed_multi_scan(args, scores, Q, tokens, cu, qmask, max_len, normal
     _buf(args, "args", torch.int32, nq * B * Tq)
     dev = require_device(args, scores, Q, tokens, cu, qmask)
     st = _call_with_workspace(
-        _lib.lib().fms_launch_packed_multi_scan, dev, 
+        _lib.lib().fms_launch_packed_multi_scan, dev,
         dtype_code(Q), ptr(args), ptr(scores), ptr(Q), ptr(tokens), ptr(cu),
         ptr(_maskn(qmask, "qmask", nq * Tq)), dim, Tq, nq, B, tokens.shape[0], int(max_len),
         _norm(normalize), stream_handle(dev))
@@ -457,7 +473,7 @@ def launch_int8_candidates_scan(args, partial, Qc, Qs, Gc, Gs, idx, qmask, dmask
     _buf(scores, "scores", torch.float32, B * C)
     dev = require_device(args, partial, Qc, Qs, Gc, Gs, idx, qmask, dmask, scores)
     st = _call_with_workspace(
-        _lib.lib().fms_launch_int8_candidates_scan, dev, 
+        _lib.lib().fms_launch_int8_candidates_scan, dev,
         ptr(args), ptr(partial), ptr(Qc), ptr(Qs), qsc, ptr(Gc), ptr(Gs), dsc, ptr(idx),
         _idx_bytes(idx), ptr(_maskn(qmask, "qmask", B * Tq)), ptr(_maskn(dmask, "dmask", N * Td)),
         dim, Tq, B, Td, N, C, ptr(scores), float(neg), _norm(normalize), stream_handle(dev))
@@ -539,7 +555,7 @@ def pair_apply_pullback(dq, dd, q, d, qmask, argmax_u, delta):
     for t, w in ((dq, "dq"), (dd, "dd"), (d, "d"), (delta, "delta")):
         _like(t, q, w)
     st = _call_with_workspace(
-        _lib.lib().fms_pair_pullback, dev, 
+        _lib.lib().fms_pair_pullback, dev,
         dtype_code(q), ptr(dq), ptr(dd), ptr(q), ptr(d), ptr(_mask(qmask)), ptr(_tape(argmax_u)),
         ptr(delta), dim, Tq, Td, stream_handle(dev))
     _lib.check(st, "pair_apply_pullback")
@@ -552,7 +568,7 @@ def paired_apply_pullback(dQ, dD, Q, D, qmask, args, Delta, inv_n):
     for t, w in ((dQ, "dQ"), (dD, "dD"), (D, "D"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, Q, w)
     st = _call_with_workspace(
-        _lib.lib().fms_paired_pullback, dev, 
+        _lib.lib().fms_paired_pullback, dev,
         dtype_code(Q), ptr(dQ), ptr(dD), ptr(Q), ptr(D), ptr(_mask(qmask)), ptr(_tape(args)),
         ptr(Delta), ptr(inv_n), dim, Tq, Td, B, stream_handle(dev))
     _lib.check(st, "paired_apply_pullback")
@@ -566,7 +582,7 @@ def inbatch_apply_pullback(dQ, dD, Q, D, qmask, args, Delta, inv_n):
     for t, w in ((dQ, "dQ"), (dD, "dD"), (D, "D"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, Q, w)
     st = _call_with_workspace(
-        _lib.lib().fms_inbatch_pullback, dev, 
+        _lib.lib().fms_inbatch_pullback, dev,
         dtype_code(Q), ptr(dQ), ptr(dD), ptr(Q), ptr(D), ptr(_mask(qmask)), ptr(_tape(args)),
         ptr(Delta), ptr(inv_n), dim, Tq, Td, Bq, Bd, stream_handle(dev))
     _lib.check(st, "inbatch_apply_pullback")
@@ -581,7 +597,7 @@ def candidates_apply_pullback(dQ, dG, Q, gallery, idx, qmask, args, Delta, inv_n
     for t, w in ((dQ, "dQ"), (dG, "dG"), (gallery, "gallery"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, Q, w)
     st = _call_with_workspace(
-        _lib.lib().fms_candidates_pullback, dev, 
+        _lib.lib().fms_candidates_pullback, dev,
         dtype_code(Q), ptr(dQ), ptr(dG), ptr(Q), ptr(gallery), ptr(idx), _idx_bytes(idx),
         ptr(_mask(qmask)), ptr(_tape(args)), ptr(Delta), ptr(inv_n), dim, Tq, B, Td, N, C,
         stream_handle(dev))
@@ -597,7 +613,7 @@ def packed_apply_pullback(dq, dP, q, tokens, cu, qmask, args, Delta, inv_n):
     for t, w in ((dq, "dq"), (dP, "dP"), (tokens, "tokens"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, q, w)
     st = _call_with_workspace(
-        _lib.lib().fms_packed_pullback, dev, 
+        _lib.lib().fms_packed_pullback, dev,
         dtype_code(q), ptr(dq), ptr(dP), ptr(q), ptr(tokens), ptr(cu), ptr(_mask(qmask)),
         ptr(_tape(args)), ptr(Delta), ptr(inv_n), dim, Tq, B, tokens.shape[0],
         stream_handle(dev))
@@ -614,7 +630,7 @@ def varlen_apply_pullback(dQ, dD, Qp, Dp, cu_q, cu_d, args, Delta, inv_n):
     for t, w in ((dQ, "dQ"), (dD, "dD"), (Dp, "D tokens"), (Delta, "Delta"), (inv_n, "inv_n")):
         _like(t, Qp, w)
     st = _call_with_workspace(
-        _lib.lib().fms_varlen_pullback, dev, 
+        _lib.lib().fms_varlen_pullback, dev,
         dtype_code(Qp), ptr(dQ), ptr(dD), ptr(Qp), ptr(Dp), ptr(cu_q), ptr(cu_d),
         ptr(_tape(args)), ptr(Delta), ptr(inv_n), dim, max_q, N, Qp.shape[0], Dp.shape[0],
         stream_handle(dev))

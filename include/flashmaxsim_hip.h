@@ -451,19 +451,19 @@ fms_status fms_debug_mfma_layout(float* out, int32_t dtype_or_int8, void* stream
 fms_status fms_debug_cross_lane(float* out, void* stream);
 
 /*
- * Workspace lent to the calling host thread's next calls (no reference
- * counterpart).  An entry point that needs workspace takes it from the library's
- * stream-ordered pool; allocating there holds the host until earlier work on the
- * stream is done.  Between fms_workspace_lend(ptr, bytes) and
- * fms_workspace_return() it uses the lent device memory first (256-byte aligned,
- * on the device of the calls' stream; NULL or 0 bytes lends none) and the pool
- * for what does not fit.  Work that uses the memory is enqueued on the calls'
- * streams: the owner may reuse it in stream order, or once that work is done.
- * fms_workspace_return ends the loan and returns the bytes asked for since it
- * began, i.e. what would have fitted everything.
+ * Workspace lent by the caller (no reference counterpart).  An entry point that
+ * needs workspace takes it from the library's stream-ordered pool; allocating
+ * there holds the host until earlier work on the stream is done.  A host thread
+ * that has set a lender is asked first: lender(bytes, stream) returns device
+ * memory of at least `bytes` (256-byte aligned, on the stream's device) or NULL,
+ * and the pool serves the latter.  Work that uses the memory is enqueued on
+ * `stream` before the call returns, and none of it is used by a later call: the
+ * owner may reuse it in stream order from then on.  The lender belongs to the
+ * calling host thread (NULL: none, the default), may be asked several times by a
+ * call, and is not asked while the stream is being captured.
  */
-void fms_workspace_lend(void* ptr, int64_t bytes);
-int64_t fms_workspace_return(void);
+typedef void* (*fms_workspace_lender)(int64_t bytes, void* stream);
+void fms_set_workspace_lender(fms_workspace_lender lender);
 
 /*
  * Test-only: the number of workspace allocations the library's calls have made

@@ -1,7 +1,9 @@
-"""Workspace lent to a call (fms_workspace_lend): results do not depend on it,
-whether it holds everything, part or nothing of what the call asks for; loans
-are per host thread and end with the call; calls of changing sizes on several
-threads and streams use memory that the allocator has given back in between."""
+"""Workspace lent to a call (fms_set_workspace_lender): results do not depend on it,
+whether all, some or none of the pieces a call asks for are lent, and nothing is
+written beside a piece; torch lends each call exactly what it asks for, whatever sizes
+came before, on every thread; calls of changing sizes on several threads and streams
+use memory that the allocator has given back in between."""
+import gc
 import threading
 
 import pytest
@@ -14,36 +16,122 @@ pytestmark = pytest.mark.gpu
 
 
 def _inputs(device, seed, B=40, Tq=70, Td=90, dim=128, dtype=torch.float16):
+    """Small integers: sums of their products are exact in any order."""
     g = torch.Generator(device=device).manual_seed(seed)
-    Q = torch.randn(B, Tq, dim, generator=g, device=device).to(dtype)
-    D = torch.randn(B + 3, Td, dim, generator=g, device=device).to(dtype)
+    Q = torch.randint(-3, 4, (B, Tq, dim), generator=g, device=device).to(dtype)
+    D = torch.randint(-3, 4, (B + 3, Td, dim), generator=g, device=device).to(dtype)
     return Q, D
 
 
-@pytest.mark.parametrize("share", [0.0, 0.3, 1.0])
-@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
-def test_any_loan_gives_the_same_results(device, share, dtype):
-    Q, D = _inputs(device, 1, dtype=dtype)
+class _Lender:
+    """Lends the first `pieces` requests of a call from one guarded buffer."""
+
+    GAP, FILL = 4096, 77
+
+    def __init__(self, device, pieces):
+        self.buf = torch.full((64 << 20,), self.FILL, dtype=torch.uint8, device=device)
+        self.base = -self.buf.data_ptr() % 256 + self.GAP
+        self.pieces, self.asked, self.lent = pieces, [], []
+        self.fn = _lib.LENDER(self._lend)
+
+    def _lend(self, nbytes, stream):
+        self.asked.append(nbytes)
+        if len(self.asked) > self.pieces:
+            return None
+        at = self.lent[-1][1] + self.GAP if self.lent else self.base
+        at += -(self.buf.data_ptr() + at) % 256
+        assert at + nbytes + self.GAP <= self.buf.numel()
+        self.lent.append((at, at + nbytes))
+        return self.buf.data_ptr() + at
+
+    def __enter__(self):
+        _lib.lib().fms_set_workspace_lender(self.fn)
+        return self
+
+    def __exit__(self, *exc):
+        _lib.lib().fms_set_workspace_lender(_lib.LENDER(0))
+        boundary._call.known = False  # the drivers set theirs again
+        torch.cuda.synchronize()
+        at = 0
+        for a, z in self.lent + [(self.buf.numel(), 0)]:
+            assert bool((self.buf[at:a] == self.FILL).all()), (self.lent, at)
+            at = z
+
+
+# In-batch scans ask once; the pullback of rows that are not whole 16-byte units asks
+# twice, holding the first piece (its cotangents) while it uses the second (its sources).
+@pytest.mark.parametrize("pieces", [0, 1, 2])
+@pytest.mark.parametrize("dtype,dim", [(torch.float16, 128), (torch.float16, 256), (torch.float32, 64),
+                                       (torch.float16, 100), (torch.float32, 101)])
+def test_any_loan_gives_the_same_results(device, pieces, dtype, dim):
+    Q, D = _inputs(device, 1, dim=dim, dtype=dtype)
     L = _lib.lib()
-    B, Bd = Q.shape[0], D.shape[0]
-    boundary._wanted.__dict__.clear()
-    S0, a0 = fm.inbatch_forward(Q, D)  # nothing lent on a thread's first call
-    want = boundary._wanted.__dict__["fms_inbatch_device_scan"]
-    assert want > 0
-    n = int(want * share)
-    ws = torch.empty(max(n, 1), dtype=torch.uint8, device=device)
-    guard = ws.new_full((4096,), 77)
-    S, a = torch.empty_like(S0), torch.empty_like(a0)
-    L.fms_workspace_lend(ws.data_ptr(), n)
-    st = L.fms_inbatch_device_scan(boundary.dtype_code(Q), S.data_ptr(), a.data_ptr(), Q.data_ptr(),
-                                   D.data_ptr(), None, None, Q.shape[2], Q.shape[1], B, D.shape[1],
-                                   Bd, 0, boundary.stream_handle(Q.device))
-    assert st == 0 and L.fms_workspace_return() == want
-    assert L.fms_workspace_return() == 0  # the loan ended
-    torch.cuda.synchronize()
-    assert torch.equal(S, S0) and torch.equal(a, a0) and bool((guard == 77).all())
-    S1, a1 = fm.inbatch_forward(Q, D)  # the driver's own loan
+    B, Tq, Bd, Td = Q.shape[0], Q.shape[1], D.shape[0], D.shape[1]
+    S0, a0 = fm.inbatch_forward(Q, D)
+    G = (torch.arange(B * Bd, device=device).reshape(B, Bd) % 3 - 1).to(dtype)
+    dQ0, dD0 = fm.inbatch_pullback(G, Q, D, None, a0)
+    S, a, dQ, dD = (torch.empty_like(x) for x in (S0, a0, dQ0, dD0))
+    code, stream = boundary.dtype_code(Q), boundary.stream_handle(Q.device)
+    one_ask = dim * Q.element_size() % 16 == 0
+    with _Lender(device, pieces) as lender:
+        assert L.fms_inbatch_device_scan(code, S.data_ptr(), a.data_ptr(), Q.data_ptr(), D.data_ptr(),
+                                         None, None, dim, Tq, B, Td, Bd, 0, stream) == 0
+        assert len(lender.asked) == (1 if one_ask else 0)
+    with _Lender(device, pieces) as lender:
+        assert L.fms_inbatch_pullback(code, dQ.data_ptr(), dD.data_ptr(), Q.data_ptr(), D.data_ptr(), None,
+                                      a.data_ptr(), G.data_ptr(), None, dim, Tq, Td, B, Bd, stream) == 0
+        assert len(lender.asked) == (1 if one_ask else 2) and len(lender.lent) == min(pieces, len(lender.asked))
+    for x, y in ((S, S0), (a, a0), (dQ, dQ0), (dD, dD0)):
+        assert torch.equal(x, y)
+    S1, a1 = fm.inbatch_forward(Q, D)  # the driver's own lender again
     assert torch.equal(S1, S0) and torch.equal(a1, a0)
+
+
+def _lent_by(call):
+    """(torch allocations, most bytes held) of a call, results dropped."""
+    gc.collect()
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    n0 = torch.cuda.memory_stats()["allocation.all.allocated"]
+    out = call()
+    n = torch.cuda.memory_stats()["allocation.all.allocated"] - n0
+    peak = torch.cuda.max_memory_allocated() - base
+    del out
+    return n, peak
+
+
+def test_torch_lends_what_each_call_needs(device):
+    """The scores, the tape and one workspace per call: the first call of a size and of a
+    thread as well, and no more for a small call after a large one."""
+    sizes = [(4, 20), (90, 70), (4, 20), (40, 33), (90, 70)]
+    cases = [_inputs(device, k, B=b, Tq=t, dim=256) for k, (b, t) in enumerate(sizes)]
+    seen = {}
+
+    def work(tag):
+        seen[tag] = [_lent_by(lambda: fm.inbatch_forward(*c)) for c in cases]
+
+    work("here")
+    th = threading.Thread(target=work, args=("there",))
+    th.start()
+    th.join()
+    assert seen["here"] == seen["there"]
+    assert [n for n, _ in seen["here"]] == [3] * len(sizes)
+    assert seen["here"][0] == seen["here"][2] and seen["here"][1] == seen["here"][4]
+    assert seen["here"][2][1] * 20 < seen["here"][1][1]
+
+
+def test_a_call_outside_the_drivers_is_not_lent_to(device):
+    """The library keeps a thread's lender; it declines calls that the drivers do not make."""
+    Q, D = _inputs(device, 2)
+    S0, a0 = fm.inbatch_forward(Q, D)
+    S, a = torch.empty_like(S0), torch.empty_like(a0)
+    n0 = torch.cuda.memory_stats()["allocation.all.allocated"]
+    assert _lib.lib().fms_inbatch_device_scan(
+        boundary.dtype_code(Q), S.data_ptr(), a.data_ptr(), Q.data_ptr(), D.data_ptr(), None, None, Q.shape[2],
+        Q.shape[1], Q.shape[0], D.shape[1], D.shape[0], 0, boundary.stream_handle(Q.device)) == 0
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] == n0
+    assert torch.equal(S, S0) and torch.equal(a, a0)
 
 
 def test_loans_on_threads_and_streams(device):
@@ -79,7 +167,7 @@ def test_topk_and_grouped_candidates_with_loans(device):
     G = torch.randn(500, 40, 128, generator=g, device=device).half()
     idx = torch.randint(0, 501, (40, 500), generator=g, device=device)
     runs = []
-    for _ in range(3):  # the first call on the pool, later ones on lent memory
+    for _ in range(3):
         S, a = fm.candidates_forward(Q, G, idx)
         v, i = fm.topk(torch.cat([S] * 40, 1), 100)
         runs.append((S, a, v, i))
