@@ -48,22 +48,30 @@ def _varlen_inv(Q: PackedSeq) -> torch.Tensor:
     return inv
 
 
-def _cotangent(delta, y: torch.Tensor) -> torch.Tensor:
-    """as_array_cotangent (rrule.jl:8-27): fp32 device array of y's shape."""
+def _like(y: torch.Tensor):
+    """What a pullback keeps of the scores: their shape and device.  The scores themselves
+    hold the autograd node, which holds the pullback; a pullback that held them too would
+    keep its tape alive until the cyclic collector runs."""
+    return y.shape, y.device
+
+
+def _cotangent(delta, like) -> torch.Tensor:
+    """as_array_cotangent (rrule.jl:8-27): fp32 device array of the scores' shape."""
+    shape, device = like
     if delta is None:
-        return torch.zeros_like(y, dtype=torch.float32)
+        return torch.zeros(shape, dtype=torch.float32, device=device)
     if isinstance(delta, torch.Tensor):
-        if tuple(delta.shape) != tuple(y.shape):
-            if delta.numel() == 1 and y.numel() == 1:
-                return delta.reshape(y.shape).to(device=y.device, dtype=torch.float32)
+        if tuple(delta.shape) != tuple(shape):
+            if delta.numel() == 1 and shape.numel() == 1:
+                return delta.reshape(shape).to(device=device, dtype=torch.float32)
             raise DimensionMismatch(
                 f"MaxSim cotangent axes {tuple(delta.shape)} do not match score axes "
-                f"{tuple(y.shape)}")
-        return delta.to(device=y.device, dtype=torch.float32)
+                f"{tuple(shape)}")
+        return delta.to(device=device, dtype=torch.float32)
     if isinstance(delta, (int, float)):
-        if y.numel() != 1:
-            raise ArgumentError(f"scalar MaxSim cotangent for a {y.numel()}-element score array")
-        return torch.full(y.shape, float(delta), dtype=torch.float32, device=y.device)
+        if shape.numel() != 1:
+            raise ArgumentError(f"scalar MaxSim cotangent for a {shape.numel()}-element score array")
+        return torch.full(shape, float(delta), dtype=torch.float32, device=device)
     raise ArgumentError(f"unsupported MaxSim cotangent type {type(delta).__name__}")
 
 
@@ -94,9 +102,10 @@ def rrule(cfg, *args):
         y, tape = F.varlen_forward(a, b, cfg.neg, norm)
         inv = _varlen_inv(a) if norm else None
         T = a.tokens.dtype
+        like = _like(y)
 
         def pullback(delta):
-            dh = _cotangent(delta, y).to(T)
+            dh = _cotangent(delta, like).to(T)
             dQ, dD = BW.varlen_pullback(dh, a, b, tape, inv, mode)
             return _pad((dQ, dD), nargs)
         return y, pullback
@@ -108,9 +117,10 @@ def rrule(cfg, *args):
         nq, Tq = a.shape[0], a.shape[1]
         inv = _inv_counts(qmask, nq, Tq, a) if norm else None
         T = a.dtype
+        like = _like(y)
 
         def pullback(delta):
-            dh = _cotangent(delta, y).to(T)
+            dh = _cotangent(delta, like).to(T)
             dQ = torch.empty_like(a)
             dP = None
             for i in range(nq):
@@ -129,9 +139,10 @@ def rrule(cfg, *args):
         y, tape = F.packed_forward(a, b, qmask, cfg.neg, norm)
         inv = _inv_counts(qmask, 1, a.shape[0], a) if norm else None
         T = a.dtype
+        like = _like(y)
 
         def pullback(delta):
-            dh = _cotangent(delta, y).to(T)
+            dh = _cotangent(delta, like).to(T)
             dq, dP = BW.packed_pullback(dh, a, b, qmask, tape, inv, mode)
             return _pad((dq, dP), nargs)
         return y, pullback
@@ -155,9 +166,10 @@ def rrule(cfg, *args):
         qmask, dmask = (masks + [None, None])[:2]
         y, tape = F.candidates_forward(a, b, idxs, qmask, dmask, cfg.neg, norm)
         inv = _inv_counts(qmask, a.shape[0], a.shape[1], a) if norm else None
+        like = _like(y)
 
         def pullback(delta):
-            dh = _cotangent(delta, y).to(T)
+            dh = _cotangent(delta, like).to(T)
             dQ, dG = BW.candidates_pullback(dh, a, b, idxs, qmask, tape, inv, mode)
             return _pad((dQ, dG), nargs)
         return y, pullback
@@ -167,9 +179,10 @@ def rrule(cfg, *args):
     if inbatch:
         y, tape = F.inbatch_forward(a, b, qmask, dmask, cfg.neg, norm)
         inv = _inv_counts(qmask, a.shape[0], a.shape[1], a) if norm else None
+        like = _like(y)
 
         def pullback(delta):
-            dh = _cotangent(delta, y).to(T)
+            dh = _cotangent(delta, like).to(T)
             dQ, dD = BW.inbatch_pullback(dh, a, b, qmask, tape, inv, mode)
             return _pad((dQ, dD), nargs)
         return y, pullback
@@ -178,9 +191,10 @@ def rrule(cfg, *args):
     if a.dim() == 2:
         y, tape = F.pair_forward(a, b, qmask, dmask, cfg.neg, norm)
         inv = _inv_counts(qmask, 1, a.shape[0], a, torch.float32) if norm else None
+        like = _like(y)
 
         def pullback(delta):
-            d32 = _cotangent(delta, y)
+            d32 = _cotangent(delta, like)
             dl = (d32 * inv if norm else d32).to(T)  # δ = convert_scores(T, Δ * inv_n)
             dq, dd = BW.pair_pullback(dl, a, b, qmask, tape, mode)
             return _pad((dq, dd), nargs)
@@ -189,9 +203,10 @@ def rrule(cfg, *args):
     # ---- paired (rrule.jl:68-82) ----
     y, tape = F.paired_forward(a, b, qmask, dmask, cfg.neg, norm)
     inv = _inv_counts(qmask, a.shape[0], a.shape[1], a) if norm else None
+    like = _like(y)
 
     def pullback(delta):
-        dh = _cotangent(delta, y).to(T)
+        dh = _cotangent(delta, like).to(T)
         dQ, dD = BW.paired_pullback(dh, a, b, qmask, tape, inv, mode)
         return _pad((dQ, dD), nargs)
     return y, pullback

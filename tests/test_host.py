@@ -1,6 +1,9 @@
 """CPU checks of the host mirror: PackedSeq / pack_docs CSR logic, MaxSim
 config semantics, argument validation, and that no CPU scoring path exists
 (host tensors are refused, as the MI355X library is the only scorer)."""
+import gc
+import weakref
+
 import numpy as np
 import pytest
 import torch
@@ -158,3 +161,41 @@ def test_int8_index_at_rest_round_trip(tmp_path):
     save_file({"codes": codes, "scales": scales}, str(tmp_path / "plain.safetensors"))
     with pytest.raises(fm.ArgumentError):
         fm.load_int8_index(str(tmp_path / "plain.safetensors"))
+
+
+def _packed(*lens):
+    return fm.pack_docs([torch.randn(n, 8) for n in lens])
+
+
+@pytest.mark.parametrize("layout", ["pair", "paired", "inbatch", "candidates", "packed", "packed_multi",
+                                    "varlen"])
+def test_a_steps_tape_is_freed_with_its_scores(monkeypatch, layout):
+    """The autograd node of a call holds its pullback and the scores hold the node: without
+    the cyclic collector the tape goes when the scores do, so the pullback holds no scores."""
+    q = torch.randn(3, 4, 8, requires_grad=True)
+    calls = {"pair": (q[0].detach().requires_grad_(), torch.randn(5, 8)),
+             "paired": (q, torch.randn(3, 5, 8)),
+             "inbatch": (q, torch.randn(2, 5, 8), fm.InBatch()),
+             "candidates": (q, torch.randn(6, 5, 8), torch.ones(3, 2, dtype=torch.int64)),
+             "packed": (q[0].detach().requires_grad_(), _packed(2, 3)),
+             "packed_multi": (q, _packed(2, 3)),
+             "varlen": (_packed(2, 3), _packed(4, 1))}
+    args = calls[layout]
+    if layout == "varlen":
+        args[0].tokens.requires_grad_()
+    tapes = []
+
+    def forward(*a, **k):  # the device scan's outputs, on the host
+        tapes.append(weakref.ref(tape := torch.ones(2, 4, dtype=torch.int32)))
+        return torch.ones(1 if layout == "pair" else 2), tape
+
+    monkeypatch.setattr(F, layout + "_forward", forward)
+    gc.collect()
+    gc.disable()
+    try:
+        y = fm.maxsim(*args)
+        assert y.requires_grad and tapes[0]() is not None
+        del y
+        assert tapes[0]() is None
+    finally:
+        gc.enable()
