@@ -62,12 +62,16 @@ def score_eltype(dtype):
 dot_accum = score_eltype
 
 
-@functools.lru_cache(maxsize=64)
 def _cast_neg(neg: float, dtype) -> float:
     """MaxSim{T} stores T(neg) (types.jl:35-38); scores report it as Float32."""
-    if dtype in (torch.float16, torch.bfloat16, torch.float32, torch.float64):
-        return float(torch.tensor(neg, dtype=dtype).to(torch.float32))
-    return float(torch.tensor(neg, dtype=torch.float32))
+    return _rounded(neg.hex(), dtype if dtype in (torch.float16, torch.bfloat16, torch.float64)
+                    else torch.float32)
+
+
+@functools.lru_cache(maxsize=64)
+def _rounded(neg: str, dtype) -> float:
+    """By its text, since 0.0 == -0.0 would share an entry."""
+    return float(torch.tensor(float.fromhex(neg), dtype=dtype).to(torch.float32))
 
 
 class MaxSim:

@@ -199,3 +199,10 @@ def test_a_steps_tape_is_freed_with_its_scores(monkeypatch, layout):
         assert tapes[0]() is None
     finally:
         gc.enable()
+
+
+def test_config_neg_keeps_the_sign_of_zero():
+    """0.0 == -0.0, but each is its own fill value, whichever came first."""
+    for neg in (0.0, -0.0, 0.0):
+        for dtype in (torch.float32, torch.float16):
+            assert np.signbit(fm.MaxSim(dtype, neg=neg).neg) == np.signbit(neg)
