@@ -11,12 +11,13 @@
 // query).  dQ and dD are written in full (rows no source reaches are 0),
 // in the feature type; all sums run in fp32.
 //
-// dQ is a gather: one wave per (query group, token) sums its pairs in pair
-// order (deterministic).  dD is destination-owned: the sources are counted
-// per destination row, prefix-summed into a CSR and filled (atomic slot per
-// source), then one wave per destination row sums its sources.  The order
-// of sources within a row is the fill order, so dD may differ between runs
-// in the last bits, as the reference's device CSR does (src/invgrid.jl:10-14).
+// dQ is a gather: waves own tokens of a query group and sum its pairs in a
+// fixed order (deterministic).  dD is destination-owned: a document's sources
+// are counted per destination row, prefix-summed and filled (atomic slot per
+// source) in LDS or global lists, then every row's sources are summed in
+// registers.  The order of sources within a row is the fill order, so dD may
+// differ between runs in the last bits, as the reference's device CSR does
+// (src/invgrid.jl:10-14).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -39,7 +40,8 @@ struct PullbackArgs {
   int64_t nq_rows, nd_rows;  // rows of dQ / dD
   int rows;                  // tape rows per pair (Tq, or max_q for varlen)
   int dim;
-  bool zero_dq;              // dQ rows may belong to no group (varlen): clear dQ first
+  bool zero_dq;              // dQ rows may belong to no group (varlen): they are written 0
+                             // (generic rows: dQ is cleared first)
 };
 
 // Runs the pullback on `stream` (workspace from the library pool).

@@ -1444,10 +1444,10 @@ __global__ void __launch_bounds__(256) inbatch_tile_sum_kernel(const float* St, 
 // effect at Tq = 24, which has its own packing), 2 up to 64.  So Tq <= 25 but 24,
 // and 33 .. 42.  Also for so few queries that they make as many blocks either way: no
 // MFMA is saved there, but fewer waves are at work or the sum over two tiles' launch
-// goes, and the two are within a tenth of one another (bf16, d = 128, us per call,
-// a query per tile / packed: 16 x 16 on 5000 packed documents of 100 .. 300 tokens 132 / 115,
-// in-batch on 5000 of 60 .. 180 98 / 88, 2 x 40 on 32 21.9 / 20.0, 16 x 9 on 300 within 2%,
-// 32 x 20 on 32 20.5 / 22.2, 24 x 25 on 300 27.8 / 29.4, 8 x 16 on 300 23.7 / 24.9).
+// goes, and it is worth more than it costs (bf16, d = 128, us per call, a query per
+// tile / packed: 16 x 16 on 5000 packed documents of 100 .. 300 tokens 132 / 115, in-batch on
+// 5000 of 60 .. 180 98 / 88, 2 x 40 on 32 21.9 / 20.0, 16 x 9 on 300 23.0 / 24.0, 32 x 20 on 32 20.5 /
+// 22.2, 24 x 25 on 300 27.8 / 29.4, 8 x 16 on 300 23.7 / 24.9).
 static int flat_queries(int Tq) {
   if (Tq < 1 || Tq > 64 || Tq == 24) return 0;
   const int flat = std::min(kIbFlatQueries, kIbQpw * kTile / Tq);

@@ -13,8 +13,13 @@
 // MFMA per k-block and one running max/argmax update per accumulator
 // register.  Nothing of size Tq x Td ever reaches HBM.
 //
-// Three kernel shapes, tried in this order:
-//   scan_fast<Op, L, NKB>: dim == NKB * KB exactly, 16-byte aligned rows.
+// Four kernel shapes, tried in this order:
+//   scan_few<Op, L, KB, ...> (fms_few.hpp): rows of whole 16-byte units from
+//     aligned bases and documents of two chunks or more on average, up to 512
+//     pairs (16-bit and INT8; wide rows of long documents up to 256) or, in
+//     fp32, any number: a workgroup per pair, whose waves share its chunks.
+//     Not in-batch, and in document order fp32 only.
+//   scan_fast<Op, L, NKB>: 16-bit or INT8, dim == NKB * KB exactly, 16-byte aligned rows.
 //     The loads and MFMAs of a step are unconditional, so the compiler's
 //     in-order vmcnt accounting waits for exactly the chunk it multiplies
 //     and never drains the prefetch.  The query tile is register resident
@@ -23,7 +28,8 @@
 //     buffer while the current one is multiplied.
 //   scan_split<Op, L, KBAT> (fms_split.hpp): dims that are whole batches of
 //     KBAT k-blocks but whose query tile does not fit in registers (and
-//     fp32); document and query fragments stream one batch ahead.
+//     the fp32 calls that scan_few leaves: one-chunk documents, bases off a
+//     16-byte boundary); document and query fragments stream one batch ahead.
 //   scan_generic<Op, L, VEC>: any dim (split-d: the query fragment is
 //     re-read per k-block from L1/L2) and, with VEC = false, rows that are
 //     not 16-byte multiples (element-wise guarded loads).
@@ -445,7 +451,8 @@ struct few_layout<Op, LayInBatch> { static constexpr bool value = false; };
 
 // Fast-kernel instantiation for a given nkb (k-blocks per token); 0 = none,
 // use the generic kernel.  16-bit features: dim 64 / 96 / 128 / 256; int8: dim
-// 64 / 128 / 256; fp32 always uses the generic kernel.  (d = 96 through the
+// 64 / 128 / 256; fp32 none (what scan_few leaves of it takes scan_split or the
+// generic kernel).  (d = 96 through the
 // generic kernel, which keeps no query tile and prefetches no chunk, against
 // scan_fast and scan_runs, us: 20000 packed documents of 900 tokens 886 -> 553, 16 x
 // 1000 candidates of 180 tokens 157 -> 81, 256 x 1000 on 50000 documents 1982 -> 657.)

@@ -82,7 +82,7 @@ def _pad(tangents, nargs):
 
 def rrule(cfg, *args):
     """(y, pullback) for ``maxsim(cfg, *args)``; same argument forms as ``maxsim``."""
-    from .api import InBatch, MaxSim, _is_index  # (api imports this module lazily)
+    from .api import InBatch, MaxSim, _is_index  # (api imports this module)
     if not isinstance(cfg, MaxSim):
         raise ArgumentError("rrule(maxsim, cfg, args...) needs a MaxSim config")
     if len(args) < 2:
