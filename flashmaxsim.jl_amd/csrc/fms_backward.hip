@@ -227,15 +227,17 @@ __device__ __forceinline__ void ragged_rows(const int32_t* cu, int64_t nseg, int
   off = a - r0;
   cnt = z - r0;
 }
-// A segment whose rows (ends included) hold `row`: the last that starts at or
-// before it (row wave-uniform: scalar loads).
+// A segment whose rows (ends included) hold `row` (wave-uniform): the last that
+// starts at or before it.  The whole wave searches, 64 starts a step.
 __device__ __forceinline__ int64_t ragged_at(const int32_t* cu, int64_t nseg, int64_t row) {
-  int64_t lo = 0, hi = nseg;
+  const int lane = threadIdx.x & 63;
+  int64_t lo = 0, hi = nseg;  // (segment 0 takes what precedes it)
   while (hi - lo > 1) {
-    const int64_t mid = (lo + hi) >> 1;
-    const bool before = (int64_t)sload(cu, mid) - 1 <= row;
-    lo = before ? mid : lo;
-    hi = before ? hi : mid;
+    const int64_t step = (hi - lo + 63) >> 6, at = lo + lane * step;
+    const bool before = lane == 0 || (at < hi && (int64_t)cu[at] - 1 <= row);
+    const int last = 63 - __builtin_clzll(__ballot(before));
+    lo = uni64(lo + last * step);
+    hi = uni64(std::min(hi, lo + step));
   }
   return lo;
 }
@@ -303,7 +305,12 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_zero16_kernel(uint16_t* w, in
 
 // ---- vector path: dQ --------------------------------------------------------------------
 
-constexpr int kZeroRows = 128;  // query rows of no pair that a wave writes (varlen)
+// Query rows of no pair that a wave writes (varlen): 128, more in stores past 4096
+// such windows.
+__host__ __device__ inline int64_t zero_window(int64_t nq_rows) {
+  const int64_t w = (nq_rows + 4095) / 4096;
+  return w > 128 ? w : 128;
+}
 
 // Rows a .. b - 1 of nch 16-byte chunks = 0, by one wave.
 __device__ __forceinline__ void zero_rows(char* p, int64_t a, int64_t b, int nch, int lane) {
@@ -336,12 +343,12 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dq_vec_kernel(
     if (item >= nitems) {  // whole wave
       if constexpr (std::is_same<L, LayVarlen>::value) {
         // window of query rows past the pairs' waves (see the end of the kernel)
-        const int64_t w0 = (item - nitems) * kZeroRows;
+        const int64_t win = zero_window(nq_rows), w0 = (item - nitems) * win;
         if (w0 >= nq_rows) return;
-        const int64_t n = nitems / ntb, d = uni64(ragged_at(lay.cu_q, n, w0));
+        const int64_t n = nitems / ntb, d = ragged_at(lay.cu_q, n, w0);
         int64_t r0, cnt, off;
         ragged_rows(lay.cu_q, n, lay.nq, d, r0, cnt, off);
-        const int64_t lo = std::max(w0, r0 + kZeroRows), hi = std::min(w0 + kZeroRows, r0 + cnt);
+        const int64_t lo = std::max(w0, r0 + win), hi = std::min(w0 + win, r0 + cnt);
         zero_rows(dQ, lo, std::min(hi, r0 + off), geo.nch, lane);
         zero_rows(dQ, std::max(lo, r0 + off + lay.get(d).tq), hi, geo.nch, lane);
       }
@@ -476,15 +483,15 @@ __global__ void __launch_bounds__(kBwdThreads) bwd_dq_vec_kernel(
     // Query rows of no pair: tokens past `rows` of this pair, and those before
     // the first and after the last pair (rows past the segment's own tokens
     // and before it; see ragged_rows).  There can be any number of them, so this
-    // wave takes those within its segment's first kZeroRows rows, and waves past
-    // the pairs' take a window of kZeroRows rows each: what lies further into the
+    // wave takes those within its segment's first zero_window rows, and waves past
+    // the pairs' take a window of as many each: what lies further into the
     // segment that holds the window's first row (us per varlen pullback of 200 pairs,
     // d = 128, bf16, 300000 rows of queries and of documents past the last pair, dQ's
     // by one wave / by windows: 1919 / 49).
     if (tb == ntb - 1) {
       int64_t r0, n, off;
       ragged_rows(lay.cu_q, nitems / ntb, lay.nq, g, r0, n, off);
-      const int64_t end = r0 + std::min<int64_t>(n, kZeroRows);
+      const int64_t end = r0 + std::min(n, zero_window(nq_rows));
       zero_rows(dQ, r0, std::min(end, r0 + off), geo.nch, lane);
       zero_rows(dQ, r0 + off + v0.tq, end, geo.nch, lane);
     }
@@ -787,7 +794,7 @@ __global__ void __launch_bounds__(kDocThreads) bwd_doc_dd_kernel(
     int share = (int)(blk - d * shares);
     const int64_t w0 = (blk - own) * win;  // (below 0: the document's own share)
     if constexpr (Docs::kRagged) {
-      if (w0 >= 0) d = uni64(docs.at(w0));
+      if (w0 >= 0) d = docs.at(w0);
     }
     int64_t r0, nrow, off;
     docs.rows(d, r0, nrow, off);
@@ -1972,7 +1979,7 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hi
                        lay, delta, a.args, a.G, a.rows, ntb, (int)nsplit, nitems, geo, rb, a.dim,
                        a.Qbase, a.dQ, part, a.nq_rows, heavy);
   } else {
-    const int64_t zero_waves = std::is_same<L, LayVarlen>::value ? bcdiv(a.nq_rows, kZeroRows) : 0;
+    const int64_t zero_waves = std::is_same<L, LayVarlen>::value ? bcdiv(a.nq_rows, zero_window(a.nq_rows)) : 0;
     hipLaunchKernelGGL((bwd_dq_vec_kernel<L, E, false>), dim3((unsigned)bcdiv(nitems + zero_waves, 4)),
                        dim3(kBwdThreads), 0, st, lay, delta, a.args, a.G, a.rows, ntb, 1, nitems,
                        geo, rb, a.dim, a.Qbase, a.dQ, part, a.nq_rows, heavy);
@@ -1994,10 +2001,11 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hi
         // at least 32 rows (ragged stores: on average).
         const int64_t avg = a.nd_rows / ndocs;
         const int shares = (int)std::max<int64_t>(1, std::min<int64_t>(bcdiv(1024, ndocs), avg / 32));
-        // (windows: enough to spread a long document, few enough to find their rows)
+        // (windows of about 64 KB of rows: enough to spread a long document, few enough
+        // to find their rows)
         constexpr bool kRagged = decltype(docs)::kRagged;
-        const int64_t win = std::max<int64_t>(256, bcdiv(a.nd_rows, 32768));
-        const int64_t cap = std::max(win, 2 * avg);
+        const int64_t win = std::max(std::clamp<int64_t>(65536 / rb, 64, 256), bcdiv(a.nd_rows, 4096));
+        const int64_t cap = std::max({(int64_t)256, win, 2 * avg});
         const int64_t nwin = kRagged && a.nd_rows > cap ? bcdiv(a.nd_rows, win) : 0;
         const unsigned blocks = (unsigned)std::min<int64_t>(ndocs * shares + nwin, 65536);
         if (geo.cpl == 1)
@@ -2040,17 +2048,28 @@ hipError_t launch_vec(const L& lay, const PullbackArgs& a, const RowGeo& geo, hi
 }
 
 template <class L>
-hipError_t launch_generic(const L& lay, const PullbackArgs& a, const float* delta, hipStream_t st) {
+hipError_t launch_generic(const L& lay, const PullbackArgs& a, hipStream_t st) {
   const int esz = a.dtype == 0 ? 4 : 2;
   const int64_t rb = (int64_t)a.dim * esz;
-  // workspace: end offsets (nd_rows + 1), sources (npairs * rows), scan sums
+  // workspace: cotangents (npairs), end offsets (nd_rows + 1), sources (npairs * rows), scan sums
   const int64_t nsrc = a.npairs * a.rows;
-  const size_t b_end = al256((size_t)(a.nd_rows + 1) * 4);
+  const size_t b_delta = al256((size_t)a.npairs * 4), b_end = al256((size_t)(a.nd_rows + 1) * 4);
   const size_t b_col = al256((size_t)(nsrc > 0 ? nsrc : 1) * 4), b_sums = scan_workspace_bytes(a.nd_rows);
   void* ws = nullptr;
-  hipError_t e = workspace_alloc(&ws, b_end + b_col + b_sums, st);
+  hipError_t e = workspace_alloc(&ws, b_delta + b_end + b_col + b_sums, st);
   if (e != hipSuccess) return e;
-  char* w = static_cast<char*>(ws);
+  float* delta = static_cast<float*>(ws);
+  char* w = static_cast<char*>(ws) + b_delta;
+  const unsigned flat =
+      (unsigned)std::min<int64_t>(65536, std::max<int64_t>(1, bcdiv(a.npairs, kBwdThreads)));
+  const char* Dl = static_cast<const char*>(a.Delta);
+  const char* Il = static_cast<const char*>(a.inv_n);
+  if (a.dtype == 0)
+    hipLaunchKernelGGL(bwd_delta_kernel<EF32>, dim3(flat), dim3(kBwdThreads), 0, st, Dl, Il, a.npairs, a.G, delta);
+  else if (a.dtype == 1)
+    hipLaunchKernelGGL(bwd_delta_kernel<EF16>, dim3(flat), dim3(kBwdThreads), 0, st, Dl, Il, a.npairs, a.G, delta);
+  else
+    hipLaunchKernelGGL(bwd_delta_kernel<EBF16>, dim3(flat), dim3(kBwdThreads), 0, st, Dl, Il, a.npairs, a.G, delta);
   uint32_t* cnt = reinterpret_cast<uint32_t*>(w);
   uint32_t* col = reinterpret_cast<uint32_t*>(w + b_end);
   uint32_t* sums = reinterpret_cast<uint32_t*>(w + b_end + b_col);
@@ -2104,24 +2123,8 @@ hipError_t launch_pullback(const L& lay, const PullbackArgs& a, hipStream_t st) 
            : a.dtype == 1 ? launch_vec<L, EF16>(lay, a, geo, st)
                           : launch_vec<L, EBF16>(lay, a, geo, st);
   }
-  void* ws = nullptr;
-  hipError_t e = workspace_alloc(&ws, al256((size_t)a.npairs * 4), st);
-  if (e != hipSuccess) return e;
-  float* delta = static_cast<float*>(ws);
-  const unsigned flat =
-      (unsigned)std::min<int64_t>(65536, std::max<int64_t>(1, bcdiv(a.npairs, kBwdThreads)));
-  const char* Dl = static_cast<const char*>(a.Delta);
-  const char* Il = static_cast<const char*>(a.inv_n);
-  if (a.dtype == 0)
-    hipLaunchKernelGGL(bwd_delta_kernel<EF32>, dim3(flat), dim3(kBwdThreads), 0, st, Dl, Il, a.npairs, a.G, delta);
-  else if (a.dtype == 1)
-    hipLaunchKernelGGL(bwd_delta_kernel<EF16>, dim3(flat), dim3(kBwdThreads), 0, st, Dl, Il, a.npairs, a.G, delta);
-  else
-    hipLaunchKernelGGL(bwd_delta_kernel<EBF16>, dim3(flat), dim3(kBwdThreads), 0, st, Dl, Il, a.npairs, a.G, delta);
   if (a.zero_dq) clear(a.dQ, a.nq_rows);
-  e = launch_generic(lay, a, delta, st);
-  const hipError_t ef = workspace_free(ws, st);
-  return e != hipSuccess ? e : ef;
+  return launch_generic(lay, a, st);
 }
 
 template hipError_t launch_pullback<LayPaired>(const LayPaired&, const PullbackArgs&, hipStream_t);

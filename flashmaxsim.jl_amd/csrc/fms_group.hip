@@ -413,7 +413,7 @@ namespace {
 std::atomic<uint64_t> g_workspace_allocs{0};
 
 thread_local WorkspaceLender t_lender = nullptr;
-// Lent pieces in use by this thread's call (an entry point holds two at most).
+// Lent pieces in use by this thread's call.
 constexpr int kMaxLent = 8;
 thread_local void* t_lent[kMaxLent];
 thread_local int t_nlent = 0;

@@ -117,42 +117,51 @@ def _norm(normalize) -> int:
 # in stream order, when the call returns.  Whatever _lend declines, and every
 # allocation under graph capture, comes from the library's pool.
 
-class _Call(threading.local):
-    """The call this thread is in: its device and the pieces lent to it."""
-    device = None
-    pieces = None
-    known = False  # the library has this thread's lender
+class _Call:
+    """The call a thread is in: its device and the pieces lent to it."""
+    __slots__ = ("device", "pieces")
 
 
-_call = _Call()
+_threads = threading.local()  # .call of each thread that has given the library its lender
 
 
 @_lib.LENDER
 def _lend(nbytes, stream):
-    if _call.pieces is None:  # not one of the calls below
+    call = _threads.call
+    device = call.device
+    if device is None:  # not one of the calls below
         return None
     try:
         # (a torch allocation belongs to torch's current stream)
-        if (stream or 0) != stream_handle(_call.device):
+        if (stream or 0) != torch._C._cuda_getCurrentRawStream(device.index):
             return None
-        t = torch.empty(nbytes, dtype=torch.uint8, device=_call.device)
+        t = torch.empty(nbytes, dtype=torch.uint8, device=device)
     except Exception:  # out of memory, say: the pool decides
         return None
-    _call.pieces.append(t)
+    call.pieces.append(t)
     return t.data_ptr()
+
+
+def _this_thread():
+    call = _Call()
+    call.device, call.pieces = None, []
+    _lib.lib().fms_set_workspace_lender(_lend)
+    _threads.call = call
+    return call
 
 
 def _call_with_workspace(fn, device, *args):
     """fn(*args) on `device`, its workspace lent by torch; its status."""
-    if not _call.known:
-        _lib.lib().fms_set_workspace_lender(_lend)
-        _call.known = True
-    outer = _call.device, _call.pieces
-    _call.device, _call.pieces = device, []
+    try:
+        call = _threads.call
+    except AttributeError:
+        call = _this_thread()
+    outer, held = call.device, call.pieces
+    call.device, call.pieces = device, []
     try:
         return fn(*args)
     finally:
-        _call.device, _call.pieces = outer
+        call.device, call.pieces = outer, held
 
 
 # ---- argument checks ---------------------------------------------------------------
