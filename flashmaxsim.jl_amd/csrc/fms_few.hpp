@@ -192,7 +192,10 @@ inline int64_t few_chunks(const LayVarlen& l, int64_t n) { return l.nd / (n * kT
 // of 900 tokens 11.6 against 28.1, 1000 of them 44 against 35).  fp32: at any
 // count, since the other scans load dwords (16 bytes per lane here): 64 pairs
 // 9.9 against 88.7 us, 2000 58 against 176; the bound there is the grid's
-// 32-bit work-item count.
+// 32-bit work-item count.  Documents of one chunk leave nothing to share and stay
+// with the other scans, in fp32 too, where the loads alone would be worth a
+// workgroup from d = 64 on (2000 pairs of 32 x 32 tokens, d = 128: 15 against 44 us;
+// d = 32 within a tenth).
 template <class Op>
 constexpr int64_t few_pairs() {
   return Op::kEsz == 4 ? (int64_t)1 << 22 : 512;
