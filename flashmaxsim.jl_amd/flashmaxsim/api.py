@@ -25,6 +25,7 @@ Scores are Float32 for every feature type (score_eltype).
 from __future__ import annotations
 
 import functools
+from math import copysign
 
 import torch
 
@@ -62,16 +63,13 @@ def score_eltype(dtype):
 dot_accum = score_eltype
 
 
-def _cast_neg(neg: float, dtype) -> float:
-    """MaxSim{T} stores T(neg) (types.jl:35-38); scores report it as Float32."""
-    return _rounded(neg.hex(), dtype if dtype in (torch.float16, torch.bfloat16, torch.float64)
-                    else torch.float32)
-
-
 @functools.lru_cache(maxsize=64)
-def _rounded(neg: str, dtype) -> float:
-    """By its text, since 0.0 == -0.0 would share an entry."""
-    return float(torch.tensor(float.fromhex(neg), dtype=dtype).to(torch.float32))
+def _cast_neg(neg: float, sign: float, dtype) -> float:
+    """MaxSim{T} stores T(neg) (types.jl:35-38); scores report it as Float32.  sign is neg's
+    (0.0 == -0.0 would share an entry)."""
+    if dtype not in (torch.float16, torch.bfloat16, torch.float32, torch.float64):
+        dtype = torch.float32
+    return float(torch.tensor(neg, dtype=dtype).to(torch.float32))
 
 
 class MaxSim:
@@ -80,7 +78,8 @@ class MaxSim:
     def __init__(self, dtype=torch.float32, *, neg=-1.0e4, normalize: bool = False,
                  backward=AtomicUnified):
         self.dtype = dtype
-        self.neg = _cast_neg(float(neg), dtype)
+        neg = float(neg)
+        self.neg = _cast_neg(neg, copysign(1.0, neg), dtype)
         self.normalize = bool(normalize)
         self.backward = backward() if isinstance(backward, type) else backward
 
